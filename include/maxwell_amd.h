@@ -41,7 +41,11 @@ typedef struct {
   int max_problems;   /* Bloch problems solved together per launch */
   int smoother_steps; /* nu of V(nu,nu) (reference: 2) */
   int prec_steps;     /* edge V-cycles per PINVIT step (exp_bloch2d.c:233: 2) */
-  int gradient_steps; /* node V-cycles per lifting (exp_bloch2d.c:234: 5) */
+  int gradient_steps; /* node V-cycles per lifting (exp_bloch2d.c:234: 5), >= 1.
+                         The batched solver solves the lifting's node system
+                         exactly (mxh_lift: an error below any number of
+                         cycles) and runs the cycles only with phase_kernels
+                         and on grids mxh_lift_supported refuses */
   int phase_kernels;  /* 0: tile-fused smoother kernels (default); 1: one
                          launch per colour phase (same arithmetic, for checks) */
   int lock;           /* 1: converged wanted pairs are locked -- kept in the
@@ -62,7 +66,7 @@ typedef struct {
                          0: one sweep per launch */
   int autotune;       /* 1: at the first solve, time the square tiles and
                          row-marching tiles of 32..256 rows on every level
-                         for both smoothers over the batch, and use the
+                         for the smoothers in use over the batch, and use the
                          fastest (overrides march_min / march_rows; the
                          arithmetic, hence the result, is the same) */
   int graphs;         /* 1: capture each block step's preconditioner (the
@@ -141,7 +145,7 @@ int mx_extrapolate(mx_solver *s, const mx_batch *b, int sources, int ieigs, cons
 typedef struct {
   long long block_steps;   /* PINVIT block steps, summed over problems */
   long long edge_vcycles;  /* V-cycles (each over all active vectors) */
-  long long node_vcycles;
+  long long node_vcycles;  /* 0 where the lifting solves directly */
   long long launches;      /* kernel launches issued */
   long long active_vectors; /* preconditioned vectors, summed over steps */
   double solve_seconds;    /* wall time of the last mx_solve */

@@ -278,6 +278,28 @@ int mxh_lift_apply(int prec, const mxh_level *lv, const mxh_bloch *bl, int nv,
                    mxh_vecs xg, mxh_vecs u, mxh_vecs x, mxh_vecs e, double alpha,
                    const double *coef, double *work);
 
+/* The whole gradient lifting with an exact node solve:
+   out_v = u_v - x_v + alpha G xg_v with A xg_v = G^H M (e_v - x_v), A the Q1
+   Laplacian.  A has constant coefficients on the uniform periodic grid, so
+   the solve is one discrete Fourier transform pair in precision prec (the
+   Bloch phase taken out, division by the eigenvalues; Gamma point: the
+   constant mode stays zero) instead of node V-cycles; the lowest Bloch wave's
+   coefficient is formed in FP64 as in mxh_lift_rhs.  bg, xg: scratch node
+   vectors (xg holds the solution without the lowest wave); x.p, u.p, the maps
+   and in-place use of u = out as in mxh_lift_rhs / mxh_lift_apply.  table:
+   filled by mxh_lift_table (mxh_lift_table_bytes).  coef: 2 doubles per
+   vector; work: >= 2 * 513 * nv doubles.  mxh_lift_supported: nx and ny are
+   2^a, 3 2^a or 5 2^a and a few columns fit in LDS (ny <= 2048 in FP64, 4096
+   in FP32). */
+int mxh_lift_supported(int prec, const mxh_level *lv);
+int mxh_lift_launches(int prec, const mxh_level *lv); /* kernel launches of one mxh_lift */
+size_t mxh_lift_table_bytes(int prec, const mxh_level *lv);
+int mxh_lift_table(int prec, const mxh_level *lv, void *table);
+int mxh_lift(int prec, const mxh_level *lv, const mxh_bloch *bl, int nv,
+             mxh_vecs e, mxh_vecs x, mxh_vecs bg, mxh_vecs xg, mxh_vecs u,
+             mxh_vecs out, double alpha, const void *table, double *coef,
+             double *work);
+
 /* generic gradient / adjoint gradient in one precision */
 int mxh_gradient(int prec, const mxh_level *lv, const mxh_bloch *bl, int nv,
                  mxh_vecs v, mxh_vecs e, double ar, double ai);

@@ -43,6 +43,7 @@ struct mx_solver {
   void *eb[MX_MAXL], *ex[MX_MAXL];   /* edge MG vectors */
   void *nb[MX_MAXL], *nxv[MX_MAXL];  /* node MG vectors */
   void *ex2[MX_MAXL], *nxv2[MX_MAXL]; /* second x buffers: tile kernels write here, then swap */
+  void *lift_table;     /* the direct lifting's table; null: node V-cycles */
   void *rdef;           /* defects of a block step (MG precision, defect slots) */
   double *dbloch, *dAe, *dAn, *dlam, *dnorm, *dgram, *dC, *dwork, *dcoef;
   void *gramwork;
@@ -111,6 +112,7 @@ void mx_solver_destroy(mx_solver *s)
     mxh_free(s->nxv2[l]);
     free(s->hEtaL[l]);
   }
+  mxh_free(s->lift_table);
   mxh_free(s->rdef);
   mxh_free(s->dE);
   mxh_free(s->dU);
@@ -235,6 +237,11 @@ int mx_solver_create(const mx_config *cfg, const double *eta, mx_solver **out)
   }
   s->rdef = dalloc(s, s->csz * (size_t)edim(s, s->L) * nv);
   if (!s->rdef) goto nomem;
+  if (!cfg->phase_kernels && mxh_lift_supported(s->prec, &s->lv[s->L])) {
+    s->lift_table = dalloc(s, mxh_lift_table_bytes(s->prec, &s->lv[s->L]));
+    if (!s->lift_table) goto nomem;
+    if (mxh_lift_table(s->prec, &s->lv[s->L], s->lift_table)) goto dev;
+  }
   s->dE = (double *)dalloc(s, 16 * (size_t)edim(s, s->L) * vpp * P);
   s->dU = (double *)dalloc(s, 16 * (size_t)edim(s, s->L) * vpp * P);
   s->dbloch = (double *)dalloc(s, sizeof(double) * 4 * P);
@@ -323,7 +330,7 @@ static int tune_bucket(const mx_solver *s, int nv)
 static int march_rows_of(const mx_solver *s, int node, int l, int nv)
 {
   if (s->lv[l].nx < 8 || s->lv[l].ny < 8) return 0; /* halo of one sweep: 6 */
-  if (s->tuned) return s->tune_rows[tune_bucket(s, nv)][node][l];
+  if (s->tuned && !(node && s->lift_table)) return s->tune_rows[tune_bucket(s, nv)][node][l];
   if (s->cfg.march_min <= 0) return 0;
   const int rows = s->cfg.march_rows > 0 ? s->cfg.march_rows : 128;
   if (s->lv[l].nx >= s->cfg.march_min) return rows;
@@ -364,7 +371,8 @@ static int node_sweep(mx_solver *s, int l, int nv, const mxh_bloch *bl, mxh_vecs
   return mxh_node_tile(s->prec, &s->lv[l], bl, nv, b, x, xo, ns, mode, xc_in, bc, xc);
 }
 
-/* Autotuner: for every level, both smoothers and three launch sizes (the
+/* Autotuner: for every level, both smoothers (the nodal one only where the
+   lifting runs node V-cycles) and three launch sizes (the
    batch's nv vectors, nv/4 and nv/16: locking shrinks the launches as
    problems converge), time nu smoothing sweeps with the square tiles and
    with row-marching tiles of 32..256 rows (pairs of sweeps fused when
@@ -391,7 +399,7 @@ static int autotune(mx_solver *s, int nv_full, const mxh_bloch *bl)
     const int nv = nv_full >> (2 * bk);
     if (nv < 1 || (bk > 0 && nv == s->tune_nv[bk - 1])) break;
     s->tune_nv[bk] = nv;
-    for (int node = 0; node < 2 && !err; node++)
+    for (int node = 0; node < (s->lift_table ? 1 : 2) && !err; node++)
       for (int l = 1; l <= s->L && !err; l++) {
         const long long n = node ? ndim(s, l) : edim(s, l);
         void **bb = node ? s->nb : s->eb, **xx = node ? s->nxv : s->ex;
@@ -572,6 +580,19 @@ static int lift_to(mx_solver *s, int nv, const mxh_bloch *bl, double *E, const v
      ~(k/n)^2 near Gamma, below FP32 resolution and near the FP64 floor of an
      iterative solve) is handled exactly in FP64 in both precisions */
   double *coef = s->dcoef;
+  mxh_vecs wv = V(W, n);
+  wv.map = wmap;
+  if (s->lift_table) {
+    /* the node system solved exactly by transforms: its error is below that
+       of any number of V-cycles, and over the liftings of the 512^2 64-k mixed
+       solve it takes 53 ms where five V(2,2) cycles and the plane-wave passes
+       they need took 363 (256^2, PINVIT: 22 against 272; 64^2 FP64, one launch
+       per solve: 3 against 75) */
+    CK(mxh_lift(s->prec, &s->lv[L], bl, nv, ev, xv, V(s->nb[L], ndim(s, L)), V(s->nxv[L], ndim(s, L)),
+                W ? V(NULL, n) : ev, W ? wv : ev, -1.0, s->lift_table, coef, s->dwork));
+    s->st.launches += mxh_lift_launches(s->prec, &s->lv[L]);
+    return MX_OK;
+  }
   /* the first node V-cycle (gradient_steps >= 1) starts from zero without
      reading xg (its smoothers' zero-start modes, or a clear of its own), so
      xg is not cleared here */
@@ -582,8 +603,6 @@ static int lift_to(mx_solver *s, int nv, const mxh_bloch *bl, double *E, const v
     int e = vcycle_node(s, nv, bl, k == 0);
     if (e) return e;
   }
-  mxh_vecs wv = V(W, n);
-  wv.map = wmap;
   CK(mxh_lift_apply(s->prec, &s->lv[L], bl, nv, V(s->nxv[L], ndim(s, L)), W ? V(NULL, n) : ev, xv, W ? wv : ev,
                     -1.0, coef, s->dwork));
   s->st.launches += coef ? 3 : 1;

@@ -1727,7 +1727,8 @@ __global__ __launch_bounds__(256) void k_phi_dot(mxh_level lv, mxh_bloch bl, con
 // (x of precision T, optional; u may be e itself: each thread reads and
 // writes only its own edges): the plane-wave component of the node correction is replaced by the exact one
 // (coef from k_lift_deflate; xg has none in exact arithmetic since its right
-// hand side was deflated, so what phi^H xg finds is rounding).
+// hand side was deflated, so what phi^H xg finds is rounding).  pdot null: xg
+// holds no plane wave (the direct solve leaves its mode out).
 template <typename T>
 __global__ __launch_bounds__(256) void k_lift_apply(mxh_level lv, mxh_bloch bl, const C<T>* XG, long long xgs,
                                                     const C<double>* U, long long us, const int* umap,
@@ -1747,7 +1748,8 @@ __global__ __launch_bounds__(256) void k_lift_apply(mxh_level lv, mxh_bloch bl, 
   PlaneWave pw(g);
   C<double> a = czero<double>(), ex1 = czero<double>(), ey1 = czero<double>();
   if (coef) {
-    a = cmk(coef[2 * v] - pdot[2 * v] / N, coef[2 * v + 1] - pdot[2 * v + 1] / N);
+    a = cmk(coef[2 * v], coef[2 * v + 1]);
+    if (pdot) a -= cmk(pdot[2 * v] / N, pdot[2 * v + 1] / N);
     double s, c;
     sincos(pw.tx, &s, &c);
     ex1 = cmk(c - 1.0, s);  // phi(i+1,j) / phi(i,j) - 1
@@ -1784,6 +1786,353 @@ __global__ __launch_bounds__(256) void k_lift_apply(mxh_level lv, mxh_bloch bl, 
       e[N + k] = u1 + alpha * gy;
     }
   }
+}
+
+// ----------------------------------------------------------------- direct node solve
+// The node operator of the lifting (the Q1 Laplacian on a uniform periodic
+// grid) has constant coefficients, so with the Bloch phase taken out
+// (g(i,j) = e^{-i(tx i + ty j)} b(i,j)) it is diagonal in the discrete Fourier
+// basis, with eigenvalue
+//   mu(p,q) = rx S(thx) T(thy) + ry T(thx) S(thy),  S = 2s, T = 1 - s / 3,
+//   s = 1 - cos th = 2 sin^2(th / 2),  thx = (2 pi p + kx) / nx.
+// One transform pair replaces the node V-cycles of the lifting: three read +
+// write passes over the node vectors (one where a vector fits in LDS) against
+// the forty-odd of five V(2,2) cycles.  Measured over the liftings of the
+// 512^2 64-k mixed solve: row passes 3.1 TB/s, column pass 1.7 TB/s (its 128
+// byte row segments and six LDS stages), 53 ms where the cycles took 363.
+//
+// The forward transform decimates in frequency in place, so mode p ends at
+// the digit-reversed place; the eigenvalue is looked up by place and the
+// inverse (decimation in time, the same stages backwards) restores the order:
+// nothing is ever permuted.  Lines (rows or columns) of a workgroup sit in
+// LDS; consecutive lanes take consecutive lines, which an odd row pitch keeps
+// on different banks at every stage.
+#define FFT_MAXS 12
+struct FftPlan {
+  int n, ns;          // length and number of stages
+  int r[FFT_MAXS];    // radix of each stage: 3 or 5 (if any) first, then 8, 4, 2
+  int lm[FFT_MAXS];   // log2 of the stage's span (a power of two)
+};
+
+// multiply by -i (DIR < 0) or i (DIR > 0)
+template <int DIR, typename T> MXH_DEV C<T> mul_i(C<T> a)
+{
+  return DIR < 0 ? cmk(a.i, -a.r) : cmk(-a.i, a.r);
+}
+
+template <int R, int DIR, typename T> struct Dft;
+template <int DIR, typename T> struct Dft<2, DIR, T> {
+  static MXH_DEV void run(C<T>* a)
+  {
+    const C<T> t = a[0] - a[1];
+    a[0] = a[0] + a[1];
+    a[1] = t;
+  }
+};
+template <int DIR, typename T> struct Dft<4, DIR, T> {
+  static MXH_DEV void run(C<T>* a)
+  {
+    const C<T> s0 = a[0] + a[2], d0 = a[0] - a[2], s1 = a[1] + a[3], d1 = mul_i<DIR>(a[1] - a[3]);
+    a[0] = s0 + s1;
+    a[1] = d0 + d1;
+    a[2] = s0 - s1;
+    a[3] = d0 - d1;
+  }
+};
+template <int DIR, typename T> struct Dft<8, DIR, T> {
+  static MXH_DEV void run(C<T>* a)
+  {
+    C<T> e[4] = {a[0], a[2], a[4], a[6]}, o[4] = {a[1], a[3], a[5], a[7]};
+    Dft<4, DIR, T>::run(e);
+    Dft<4, DIR, T>::run(o);
+    const T h = T(0.70710678118654752440);
+    const C<T> i1 = mul_i<DIR>(o[1]), i3 = mul_i<DIR>(o[3]);
+    o[1] = h * (o[1] + i1);  // e^{DIR i pi / 4}
+    o[2] = mul_i<DIR>(o[2]);
+    o[3] = h * (i3 - o[3]);  // e^{DIR 3 i pi / 4}
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      a[k] = e[k] + o[k];
+      a[k + 4] = e[k] - o[k];
+    }
+  }
+};
+template <int DIR, typename T> struct Dft<3, DIR, T> {
+  static MXH_DEV void run(C<T>* a)
+  {
+    const C<T> s = a[1] + a[2], d = mul_i<DIR>(a[1] - a[2]);
+    const C<T> m = a[0] - T(0.5) * s, w = T(0.86602540378443864676) * d;
+    a[0] = a[0] + s;
+    a[1] = m + w;
+    a[2] = m - w;
+  }
+};
+template <int DIR, typename T> struct Dft<5, DIR, T> {
+  static MXH_DEV void run(C<T>* a)
+  {
+    // cos and sin of 2 pi / 5 and 4 pi / 5
+    const T c1 = T(0.30901699437494742410), c2 = T(-0.80901699437494742410);
+    const T s1 = T(0.95105651629515357212), s2 = T(0.58778525229247312917);
+    const C<T> p1 = a[1] + a[4], m1 = mul_i<DIR>(a[1] - a[4]), p2 = a[2] + a[3], m2 = mul_i<DIR>(a[2] - a[3]);
+    const C<T> u1 = a[0] + c1 * p1 + c2 * p2, u2 = a[0] + c2 * p1 + c1 * p2;
+    const C<T> v1 = s1 * m1 + s2 * m2, v2 = s2 * m1 - s1 * m2;
+    a[0] = a[0] + p1 + p2;
+    a[1] = u1 + v1;
+    a[2] = u2 + v2;
+    a[3] = u2 - v2;
+    a[4] = u1 - v1;
+  }
+};
+
+// frequency of the value at place pos after the forward stages
+MXH_DEV int fft_freq(const FftPlan& pl, int pos)
+{
+  int f = 0, mul = 1;
+  for (int s = 0; s < pl.ns; s++) {
+    f += (pos >> pl.lm[s]) * mul;
+    pos &= (1 << pl.lm[s]) - 1;
+    mul *= pl.r[s];
+  }
+  return f;
+}
+
+// One stage over nl lines in LDS (value k of line l at d[l ls + k ps]): a
+// thread takes line l0 + multiples of lstep and butterflies q0 + multiples of
+// qstep.  Forward (DIR < 0): transform, then the twiddles; inverse: the
+// conjugate twiddles, then the transform.  LAST (span 1, no twiddles): with
+// SCALE, forward and inverse butterfly in one go with the factor fac(line,
+// place) between them.
+template <int R, int DIR, bool SCALE, typename T, typename F>
+MXH_DEV void fft_stage(C<T>* d, int nl, int ls, int ps, int n, int lm, const C<T>* tw, int l0, int lstep,
+                       int q0, int qstep, F fac)
+{
+  const int m = 1 << lm, nq = n / R, tstep = nq >> lm;  // tstep = n / (R m)
+  for (int l = l0; l < nl; l += lstep)
+    for (int q = q0; q < nq; q += qstep) {
+      const int pos = q & (m - 1), base = ((q >> lm) << lm) * R + pos;
+      C<T>* p = d + l * ls + base * ps;
+      C<T> a[R];
+#pragma unroll
+      for (int k = 0; k < R; k++) a[k] = p[(k << lm) * ps];
+      if (SCALE) {
+        Dft<R, -1, T>::run(a);
+#pragma unroll
+        for (int k = 0; k < R; k++) a[k] = fac(l, base + k) * a[k];  // span 1: place base + k
+        Dft<R, 1, T>::run(a);
+      } else {
+        if (DIR > 0 && lm > 0) {
+#pragma unroll
+          for (int k = 1; k < R; k++) a[k] = cconj(tw[k * pos * tstep]) * a[k];
+        }
+        Dft<R, DIR, T>::run(a);
+        if (DIR < 0 && lm > 0) {
+#pragma unroll
+          for (int k = 1; k < R; k++) a[k] = tw[k * pos * tstep] * a[k];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < R; k++) p[(k << lm) * ps] = a[k];
+    }
+}
+
+template <int DIR, bool SCALE, typename T, typename F>
+MXH_DEV void fft_any_stage(const FftPlan& pl, int s, C<T>* d, int nl, int ls, int ps, const C<T>* tw, int l0,
+                           int lstep, int q0, int qstep, F fac)
+{
+  switch (pl.r[s]) {  // uniform
+  case 8: fft_stage<8, DIR, SCALE>(d, nl, ls, ps, pl.n, pl.lm[s], tw, l0, lstep, q0, qstep, fac); break;
+  case 4: fft_stage<4, DIR, SCALE>(d, nl, ls, ps, pl.n, pl.lm[s], tw, l0, lstep, q0, qstep, fac); break;
+  case 2: fft_stage<2, DIR, SCALE>(d, nl, ls, ps, pl.n, pl.lm[s], tw, l0, lstep, q0, qstep, fac); break;
+  case 3: fft_stage<3, DIR, SCALE>(d, nl, ls, ps, pl.n, pl.lm[s], tw, l0, lstep, q0, qstep, fac); break;
+  case 5: fft_stage<5, DIR, SCALE>(d, nl, ls, ps, pl.n, pl.lm[s], tw, l0, lstep, q0, qstep, fac); break;
+  }
+  __syncthreads();
+}
+
+// all stages of one direction over the lines of a workgroup
+template <int DIR, typename T>
+MXH_DEV void fft_lines(const FftPlan& pl, C<T>* d, int nl, int ls, int ps, const C<T>* tw, int l0, int lstep, int q0,
+                       int qstep)
+{
+  auto one = [](int, int) { return T(1); };
+  for (int t = 0; t < pl.ns; t++)
+    fft_any_stage<DIR, false>(pl, DIR < 0 ? t : pl.ns - 1 - t, d, nl, ls, ps, tw, l0, lstep, q0, qstep, one);
+}
+
+// the column transforms with the division by nx ny mu between them: the last
+// forward and the first inverse stage are one
+template <typename T, typename F>
+MXH_DEV void fft_solve_lines(const FftPlan& pl, C<T>* d, int nl, int ls, int ps, const C<T>* tw, int l0, int lstep,
+                             int q0, int qstep, F fac)
+{
+  auto one = [](int, int) { return T(1); };
+  for (int t = 0; t + 1 < pl.ns; t++)
+    fft_any_stage<-1, false>(pl, t, d, nl, ls, ps, tw, l0, lstep, q0, qstep, one);
+  fft_any_stage<-1, true>(pl, pl.ns - 1, d, nl, ls, ps, tw, l0, lstep, q0, qstep, fac);
+  for (int t = pl.ns - 2; t >= 0; t--)
+    fft_any_stage<1, false>(pl, t, d, nl, ls, ps, tw, l0, lstep, q0, qstep, one);
+}
+
+// s = 1 - cos th of the mode at place pos of a line of length n with Bloch
+// angle k: th in [-pi, pi], so small angles keep their relative accuracy
+MXH_DEV double mode_s(const FftPlan& pl, int pos, double k)
+{
+  int f = fft_freq(pl, pos);
+  if (2 * f > pl.n) f -= pl.n;
+  const double h = sin(0.5 * (6.283185307179586476925 * f + k) / pl.n);
+  return 2.0 * h * h;
+}
+
+// 1 / (nx ny mu); the lowest wave (place 0, 0) is left out: its coefficient
+// is formed in FP64 by the lifting (k_lift_coef)
+template <typename T>
+MXH_DEV T mode_factor(T sx, T sy, T rx, T ry, T cnt, bool lowest)
+{
+  const T mu = rx * (T(2) * sx) * (T(1) - sy / T(3)) + ry * (T(2) * sy) * (T(1) - sx / T(3));
+  return lowest ? T(0) : T(1) / (cnt * mu);
+}
+
+// Row transforms of RB rows per workgroup.  Forward: the Bloch phase is taken
+// out at load; inverse: put back at the store.
+template <typename T, int DIR>
+__global__ __launch_bounds__(256) void k_fft_rows(mxh_level lv, mxh_bloch bl, FftPlan pl, const C<T>* tw,
+                                                  const C<T>* IN, long long is, C<T>* OUT, long long os, int RB)
+{
+  extern __shared__ double smem[];
+  const int nx = lv.nx, ny = lv.ny, pitch = nx | 1, tid = threadIdx.x, bd = blockDim.x;
+  C<T>* d = (C<T>*)smem;                   // [RB][pitch]
+  C<T>* colf = d + (size_t)RB * pitch;     // [nx]: e^{-DIR' i tx i}
+  C<T>* rowf = colf + nx;                  // [RB]
+  const int v = blockIdx.y, j0 = blockIdx.x * RB, nr = min(RB, ny - j0);
+  const Geo<double> g = make_geo<double>(lv, bl, v);
+  const double tx = atan2(g.xf.i, g.xf.r) / nx, ty = atan2(g.yf.i, g.yf.r) / ny;
+  for (int w = tid; w < nx + nr; w += bd) {
+    double s, c;
+    sincos(DIR * (w < nx ? tx * w : ty * (j0 + w - nx)), &s, &c);
+    colf[w] = cmk(T(c), T(s));  // rowf follows colf
+  }
+  __syncthreads();
+  const C<T>* in = IN + (size_t)v * is + (size_t)j0 * nx;
+  C<T>* out = OUT + (size_t)v * os + (size_t)j0 * nx;
+  const int tot = nr * nx, dr = bd / nx, di = bd - dr * nx;
+  for (int w = tid, r = tid / nx, i = tid - r * nx; w < tot; w += bd) {
+    d[r * pitch + i] = DIR < 0 ? (colf[i] * rowf[r]) * in[w] : in[w];
+    r += dr;
+    i += di;
+    if (i >= nx) { i -= nx; r++; }
+  }
+  __syncthreads();
+  fft_lines<DIR>(pl, d, nr, pitch, 1, tw, tid & (RB - 1), RB, tid / RB, bd / RB);
+  for (int w = tid, r = tid / nx, i = tid - r * nx; w < tot; w += bd) {
+    out[w] = DIR > 0 ? (colf[i] * rowf[r]) * d[r * pitch + i] : d[r * pitch + i];
+    r += dr;
+    i += di;
+    if (i >= nx) { i -= nx; r++; }
+  }
+}
+
+// Column transforms, division by the eigenvalues and back, in place: CB
+// columns (128-byte row segments) of one vector per workgroup.
+template <typename T>
+__global__ __launch_bounds__(1024) void k_fft_cols(mxh_level lv, mxh_bloch bl, FftPlan px, FftPlan py, const C<T>* tw,
+                                                   C<T>* X, long long xs, int CB)
+{
+  extern __shared__ double smem[];
+  const int nx = lv.nx, ny = lv.ny, tid = threadIdx.x, bd = blockDim.x;
+  C<T>* d = (C<T>*)smem;            // [ny][CB]
+  T* sy = (T*)(d + (size_t)ny * CB);
+  T* sx = sy + ny;
+  const int v = blockIdx.y, c0 = blockIdx.x * CB, nc = min(CB, nx - c0);
+  const Geo<double> g = make_geo<double>(lv, bl, v);
+  const double kx = atan2(g.xf.i, g.xf.r), ky = atan2(g.yf.i, g.yf.r);
+  C<T>* x = X + (size_t)v * xs + c0;
+  const int l = tid & (CB - 1), q0 = tid / CB, qstep = bd / CB;
+  if (l < nc)
+    for (int j = q0; j < ny; j += qstep) d[j * CB + l] = x[l + (size_t)j * nx];
+  for (int w = tid; w < ny + nc; w += bd) {
+    if (w < ny) sy[w] = T(mode_s(py, w, ky));
+    else sx[w - ny] = T(mode_s(px, c0 + w - ny, kx));
+  }
+  __syncthreads();
+  const T rx = T(lv.hy / lv.hx), ry = T(lv.hx / lv.hy), cnt = T((double)nx * ny);
+  auto fac = [&](int li, int pos) { return mode_factor(sx[li], sy[pos], rx, ry, cnt, c0 + li == 0 && pos == 0); };
+  fft_solve_lines(py, d, nc, 1, CB, tw, l, CB, q0, qstep, fac);
+  if (l < nc)
+    for (int j = q0; j < ny; j += qstep) x[l + (size_t)j * nx] = d[j * CB + l];
+}
+
+// The whole solve of one vector in LDS (small grids): one launch, one read
+// and one write.
+template <typename T>
+__global__ __launch_bounds__(1024) void k_fft_solve(mxh_level lv, mxh_bloch bl, FftPlan px, FftPlan py,
+                                                    const C<T>* twx, const C<T>* twy, const C<T>* IN, long long is,
+                                                    C<T>* OUT, long long os)
+{
+  extern __shared__ double smem[];
+  const int nx = lv.nx, ny = lv.ny, pitch = nx | 1, tid = threadIdx.x, bd = blockDim.x, v = blockIdx.x;
+  C<T>* d = (C<T>*)smem;                  // [ny][pitch]
+  C<T>* colf = d + (size_t)ny * pitch;    // [nx]
+  C<T>* rowf = colf + nx;                 // [ny]
+  T* sx = (T*)(rowf + ny);                // [nx]
+  T* sy = sx + nx;                        // [ny]
+  const Geo<double> g = make_geo<double>(lv, bl, v);
+  const double kx = atan2(g.xf.i, g.xf.r), ky = atan2(g.yf.i, g.yf.r);
+  for (int w = tid; w < nx + ny; w += bd) {
+    const bool isx = w < nx;
+    const int k = isx ? w : w - nx;
+    double s, c;
+    sincos((isx ? kx / nx : ky / ny) * k, &s, &c);
+    colf[w] = cmk(T(c), T(s));
+    sx[w] = T(isx ? mode_s(px, k, kx) : mode_s(py, k, ky));
+  }
+  __syncthreads();
+  const C<T>* in = IN + (size_t)v * is;
+  C<T>* out = OUT + (size_t)v * os;
+  const int tot = nx * ny, dr = bd / nx, di = bd - dr * nx;
+  for (int w = tid, r = tid / nx, i = tid - r * nx; w < tot; w += bd) {
+    d[r * pitch + i] = cconj(colf[i] * rowf[r]) * in[w];
+    r += dr;
+    i += di;
+    if (i >= nx) { i -= nx; r++; }
+  }
+  __syncthreads();
+  const int l = tid & 31, q0 = tid >> 5, qstep = bd >> 5;
+  const T rx = T(lv.hy / lv.hx), ry = T(lv.hx / lv.hy), cnt = T((double)nx * ny);
+  auto fac = [&](int li, int pos) { return mode_factor(sx[li], sy[pos], rx, ry, cnt, li == 0 && pos == 0); };
+  fft_lines<-1>(px, d, ny, pitch, 1, twx, l, 32, q0, qstep);
+  fft_solve_lines(py, d, nx, 1, pitch, twy, l, 32, q0, qstep, fac);
+  fft_lines<1>(px, d, ny, pitch, 1, twx, l, 32, q0, qstep);
+  for (int w = tid, r = tid / nx, i = tid - r * nx; w < tot; w += bd) {
+    out[w] = (colf[i] * rowf[r]) * d[r * pitch + i];
+    r += dr;
+    i += di;
+    if (i >= nx) { i -= nx; r++; }
+  }
+}
+
+// e^{-2 pi i k / n}, k < n
+template <typename T>
+__global__ void k_fft_table(int n, C<T>* tw)
+{
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  double s, c;
+  sincospi(-2.0 * k / n, &s, &c);
+  tw[k] = cmk(T(c), T(s));
+}
+
+// coef[v] = (phi^H d / N) / mu of the lowest Bloch wave (zero at the Gamma
+// point) from the sums of k_lift_rhs
+__global__ void k_lift_coef(mxh_level lv, mxh_bloch bl, int nv, const double* csum, double* coef)
+{
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= nv) return;
+  const Geo<double> g = make_geo<double>(lv, bl, v);
+  const double N = (double)lv.nx * lv.ny;
+  const bool gamma = g.xf.r == 1.0 && g.xf.i == 0.0 && g.yf.r == 1.0 && g.yf.i == 0.0;
+  const double mu = plane_wave_mu(lv, atan2(g.xf.i, g.xf.r) / lv.nx, atan2(g.yf.i, g.yf.r) / lv.ny);
+  coef[2 * v] = gamma ? 0.0 : csum[2 * v] / N / mu;
+  coef[2 * v + 1] = gamma ? 0.0 : csum[2 * v + 1] / N / mu;
 }
 
 template <typename T>
@@ -3176,6 +3525,15 @@ int mxh_init(void)
     if (e != hipSuccess) return (int)e;
     g_scratch_ptr[dev] = p;
   }
+  // kernels that may use more dynamic LDS than the default limit of a launch
+  const void* big[] = {(const void*)k_fft_solve<double>, (const void*)k_fft_solve<float>,
+                       (const void*)k_fft_cols<double>, (const void*)k_fft_cols<float>,
+                       (const void*)k_fft_rows<double, -1>, (const void*)k_fft_rows<double, 1>,
+                       (const void*)k_fft_rows<float, -1>, (const void*)k_fft_rows<float, 1>};
+  for (const void* f : big) {
+    e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e != hipSuccess) return (int)e;
+  }
   e = hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     g_stream = nullptr;
@@ -3900,11 +4258,11 @@ int mxh_node_restrict(int prec, const mxh_level* fine, const mxh_bloch* bl, int 
   return 0;
 }
 
-int mxh_lift_rhs(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs e, mxh_vecs x,
-                 mxh_vecs u, mxh_vecs bg, mxh_vecs xg, double* coef, double* work)
+// k_lift_rhs over the interior and the frame; with coef the plane-wave sums
+// phi^H d per vector go to the returned place in work
+static int lift_rhs_launch(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs e, mxh_vecs x,
+                           mxh_vecs u, mxh_vecs bg, mxh_vecs xg, const double* coef, double* work, double** csum)
 {
-  if (x.p && u.p && u.p == e.p) return (int)hipErrorInvalidValue;
-  if (coef && !work) return (int)hipErrorInvalidValue;
   const unsigned nb = lift_blocks(lv->ny), nf = frame_blocks(lv);
   const dim3 grid(nb, nv), gridf(nf, nv);
   double* ph = coef ? work : nullptr;
@@ -3925,10 +4283,23 @@ int mxh_lift_rhs(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh
   }
   LAUNCH_CHECK();
   if (coef) {
-    double* csum = work + (size_t)(nb + nf) * 2 * nv;
+    *csum = work + (size_t)(nb + nf) * 2 * nv;
     hipLaunchKernelGGL(k_reduce_partials, dim3(reduce_blocks(2 * nv)), dim3(TPB), 0, g_stream, work, (int)(nb + nf),
-                       2 * nv, csum, 0);
+                       2 * nv, *csum, 0);
     LAUNCH_CHECK();
+  }
+  return 0;
+}
+
+int mxh_lift_rhs(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs e, mxh_vecs x,
+                 mxh_vecs u, mxh_vecs bg, mxh_vecs xg, double* coef, double* work)
+{
+  if (x.p && u.p && u.p == e.p) return (int)hipErrorInvalidValue;
+  if (coef && !work) return (int)hipErrorInvalidValue;
+  double* csum = nullptr;
+  const int err = lift_rhs_launch(prec, lv, bl, nv, e, x, u, bg, xg, coef, work, &csum);
+  if (err) return err;
+  if (coef) {
     dim3 g2(row_blocks(lv->ny), nv);
     if (prec == MXH_F64)
       hipLaunchKernelGGL(k_lift_deflate<double>, g2, dim3(TPB), 0, g_stream, *lv, *bl, (C<double>*)bg.p, bg.stride,
@@ -3938,6 +4309,22 @@ int mxh_lift_rhs(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh
                          csum, coef);
     LAUNCH_CHECK();
   }
+  return 0;
+}
+
+static int lift_apply_launch(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs xg, mxh_vecs u,
+                             mxh_vecs x, mxh_vecs e, double alpha, const double* coef, const double* pdot)
+{
+  dim3 grid(row_blocks(lv->ny), nv);
+  if (prec == MXH_F64)
+    hipLaunchKernelGGL(k_lift_apply<double>, grid, dim3(TPB), 0, g_stream, *lv, *bl, (const C<double>*)xg.p,
+                       xg.stride, (const C<double>*)u.p, u.stride, u.map, (const C<double>*)x.p, x.stride,
+                       (C<double>*)e.p, e.stride, e.map, alpha, coef, pdot);
+  else
+    hipLaunchKernelGGL(k_lift_apply<float>, grid, dim3(TPB), 0, g_stream, *lv, *bl, (const C<float>*)xg.p,
+                       xg.stride, (const C<double>*)u.p, u.stride, u.map, (const C<float>*)x.p, x.stride,
+                       (C<double>*)e.p, e.stride, e.map, alpha, coef, pdot);
+  LAUNCH_CHECK();
   return 0;
 }
 
@@ -3960,17 +4347,130 @@ int mxh_lift_apply(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, m
                        pdot, 0);
     LAUNCH_CHECK();
   }
-  dim3 grid(nb, nv);
-  if (prec == MXH_F64)
-    hipLaunchKernelGGL(k_lift_apply<double>, grid, dim3(TPB), 0, g_stream, *lv, *bl, (const C<double>*)xg.p,
-                       xg.stride, (const C<double>*)u.p, u.stride, u.map, (const C<double>*)x.p, x.stride,
-                       (C<double>*)e.p, e.stride, e.map, alpha, coef, pdot);
-  else
-    hipLaunchKernelGGL(k_lift_apply<float>, grid, dim3(TPB), 0, g_stream, *lv, *bl, (const C<float>*)xg.p,
-                       xg.stride, (const C<double>*)u.p, u.stride, u.map, (const C<float>*)x.p, x.stride,
-                       (C<double>*)e.p, e.stride, e.map, alpha, coef, pdot);
+  return lift_apply_launch(prec, lv, bl, nv, xg, u, x, e, alpha, coef, pdot);
+}
+
+// Factor n = 2^a, 3 2^a or 5 2^a into stages, the odd radix first (every span
+// is then a power of two).
+static bool fft_plan(int n, FftPlan* p)
+{
+  if (n < 2) return false;
+  p->n = n;
+  p->ns = 0;
+  int rest = n;
+  auto push = [&](int r) {
+    rest /= r;
+    int lm = 0;
+    while ((1 << lm) < rest) lm++;
+    p->r[p->ns] = r;
+    p->lm[p->ns++] = lm;
+  };
+  if (rest % 5 == 0) push(5);
+  else if (rest % 3 == 0) push(3);
+  if (rest & (rest - 1)) return false;
+  while (rest > 1) push(rest % 8 == 0 && rest != 16 ? 8 : (rest % 4 == 0 ? 4 : 2));
+  return p->ns <= FFT_MAXS;
+}
+
+#define FFT_LDS_MAX (160 * 1024)
+static size_t fft_csz(int prec) { return prec == MXH_F64 ? 16 : 8; }
+// LDS of the one-launch solve: the vector, the phases and the mode terms
+static size_t fft_solve_lds(int prec, const mxh_level* lv)
+{
+  const size_t c = fft_csz(prec), s = (size_t)lv->nx + lv->ny;
+  return c * ((size_t)lv->ny * (lv->nx | 1) + s) + c / 2 * s;
+}
+// columns per workgroup: 128-byte row segments, fewer where the columns are
+// long (at least 32 bytes of a row; 0: columns too long for LDS)
+static int fft_cols(int prec, const mxh_level* lv)
+{
+  const size_t c = fft_csz(prec);
+  int cb = (int)(128 / c);
+  while (cb * c >= 32 && c * cb * lv->ny + c / 2 * (lv->ny + cb) > FFT_LDS_MAX) cb >>= 1;
+  return cb * c >= 32 ? cb : 0;
+}
+// rows per workgroup: about 36 KB, so that four workgroups share a CU
+static int fft_rows(int prec, const mxh_level* lv)
+{
+  int rb = 64;
+  while (rb > 1 && (rb >= 2 * lv->ny || fft_csz(prec) * rb * (size_t)(lv->nx | 1) > 36 * 1024)) rb >>= 1;
+  return rb;
+}
+
+int mxh_lift_supported(int prec, const mxh_level* lv)
+{
+  FftPlan p;
+  return fft_plan(lv->nx, &p) && fft_plan(lv->ny, &p) && fft_cols(prec, lv) > 0 &&
+         fft_csz(prec) * (2 * (size_t)lv->nx + 2) <= 64 * 1024;
+}
+
+int mxh_lift_launches(int prec, const mxh_level* lv) { return fft_solve_lds(prec, lv) <= FFT_LDS_MAX ? 6 : 8; }
+
+size_t mxh_lift_table_bytes(int prec, const mxh_level* lv) { return fft_csz(prec) * ((size_t)lv->nx + lv->ny); }
+
+int mxh_lift_table(int prec, const mxh_level* lv, void* table)
+{
+  for (int k = 0; k < 2; k++) {
+    const int n = k ? lv->ny : lv->nx;
+    if (prec == MXH_F64)
+      hipLaunchKernelGGL(k_fft_table<double>, dim3(nblocks(n)), dim3(TPB), 0, g_stream, n,
+                         (C<double>*)table + (k ? lv->nx : 0));
+    else
+      hipLaunchKernelGGL(k_fft_table<float>, dim3(nblocks(n)), dim3(TPB), 0, g_stream, n,
+                         (C<float>*)table + (k ? lv->nx : 0));
+    LAUNCH_CHECK();
+  }
+  return 0;
+}
+
+extern "C++" {
+template <typename T>
+static int node_direct(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs b, mxh_vecs x,
+                       const C<T>* tw)
+{
+  FftPlan px, py;
+  if (!fft_plan(lv->nx, &px) || !fft_plan(lv->ny, &py)) return (int)hipErrorInvalidValue;
+  const C<T>*twx = tw, *twy = tw + lv->nx;
+  const C<T>* B = (const C<T>*)b.p;
+  C<T>* X = (C<T>*)x.p;
+  const size_t one = fft_solve_lds(prec, lv);
+  if (one <= FFT_LDS_MAX) {
+    const long long N = (long long)lv->nx * lv->ny;
+    hipLaunchKernelGGL(k_fft_solve<T>, dim3(nv), dim3(N >= 8192 ? 1024 : N >= 2048 ? 512 : 256), one, g_stream, *lv,
+                       *bl, px, py, twx, twy, B, b.stride, X, x.stride);
+    LAUNCH_CHECK();
+    return 0;
+  }
+  const int RB = fft_rows(prec, lv), CB = fft_cols(prec, lv);
+  const dim3 gr((lv->ny + RB - 1) / RB, nv), gc((lv->nx + CB - 1) / CB, nv);
+  const size_t shr = sizeof(C<T>) * ((size_t)RB * (lv->nx | 1) + lv->nx + RB);
+  const size_t shc = sizeof(C<T>) * (size_t)CB * lv->ny + sizeof(T) * (lv->ny + CB);
+  const int tc = CB * lv->ny / 8, bc = tc >= 1024 ? 1024 : tc >= 512 ? 512 : 256;
+  hipLaunchKernelGGL((k_fft_rows<T, -1>), gr, dim3(TPB), shr, g_stream, *lv, *bl, px, twx, B, b.stride, X, x.stride, RB);
+  LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_fft_cols<T>, gc, dim3(bc), shc, g_stream, *lv, *bl, px, py, twy, X, x.stride, CB);
+  LAUNCH_CHECK();
+  hipLaunchKernelGGL((k_fft_rows<T, 1>), gr, dim3(TPB), shr, g_stream, *lv, *bl, px, twx, (const C<T>*)X, x.stride, X,
+                     x.stride, RB);
   LAUNCH_CHECK();
   return 0;
+}
+}  // extern "C++"
+
+int mxh_lift(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs e, mxh_vecs x, mxh_vecs bg,
+             mxh_vecs xg, mxh_vecs u, mxh_vecs out, double alpha, const void* table, double* coef, double* work)
+{
+  if (!table || !coef || !work || !bg.p || !xg.p || !mxh_lift_supported(prec, lv)) return (int)hipErrorInvalidValue;
+  double* csum = nullptr;
+  const mxh_vecs none = {nullptr, 0, nullptr};
+  int err = lift_rhs_launch(prec, lv, bl, nv, e, x, none, bg, none, coef, work, &csum);
+  if (err) return err;
+  hipLaunchKernelGGL(k_lift_coef, dim3(nblocks(nv, 64)), dim3(64), 0, g_stream, *lv, *bl, nv, csum, coef);
+  LAUNCH_CHECK();
+  err = prec == MXH_F64 ? node_direct<double>(prec, lv, bl, nv, bg, xg, (const C<double>*)table)
+                        : node_direct<float>(prec, lv, bl, nv, bg, xg, (const C<float>*)table);
+  if (err) return err;
+  return lift_apply_launch(prec, lv, bl, nv, xg, u, x, out, alpha, coef, nullptr);
 }
 
 int mxh_gradient(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs v, mxh_vecs e, double ar,
