@@ -821,16 +821,32 @@ __global__ __launch_bounds__(256) void k_coarse_solve(int n, const double* Lm, c
 //   4 + S + S^H = 6 (a + b S)^H (a + b S),  a, b = (1 +- 1/sqrt 3) / 2
 // (a^2 + b^2 = 2/3, ab = 1/6), so x^H M y = ux^H uy + (y-edge analogue) with
 // ux = sqrt(6 mx) (a x(i,j) + b x(i,j+1)): every cell contributes three
-// features of its own edges and their upper and right neighbours.  A tile of
-// cells is staged in LDS for all m vectors; the m (m+1)/2 pairs times cell
-// slices are spread over the 256 threads, slices are summed in LDS at the end.
-#define GRAM_TILE_MAX 64
+// features (c, ux, uy) of its own edges and their upper and right neighbours.
+//
+// The contraction runs on the FP64 matrix cores without LDS: eight vectors
+// are the 16 real columns of a tile (real parts, then imaginary parts), and
+// v_mfma_f64_16x16x4 wants both operands of P^T P in the same lane layout
+// (column lane & 15, cell lane >> 4), so one register holds a feature of a
+// tile as left and as right operand.  A lane loads (16 bytes) the complex
+// values of vector lane & 7 at cell 2 (lane >> 4) + ((lane >> 3) & 1) of a
+// strip of eight cells (128 bytes per vector) and trades one half with lane ^ 8
+// to have the operands of the even and of the odd cells.  A wave walks a strip
+// down its rows, carrying x(j + 1) over as the next row's x(j); the next row's
+// loads are issued as soon as a tile's features are formed and land behind
+// its products.  The waves share nothing until the end, where their sums meet
+// in LDS.
+//
+// What bounds it: the FP64 pipe.  36 columns (5 tiles, one wave per SIMD: the
+// sums of 15 tile pairs take 240 registers) spend 90 MFMAs of 64 cycles per
+// strip row and wave and about a sixth of that on features, which the matrix
+// core does not overlap.  512^2, against a register-blocked vector kernel fed
+// from LDS (bound by its LDS reads and their latency): 36 columns of 16
+// problems 2.66 -> 1.69 ms (37 -> 58 TFLOP/s counting the padded tiles'
+// products once), 32 columns 2.62 -> 1.27, 12 columns of 64 problems 2.2 -> 1.70
+// (3.8 TB/s).  The tile loop's MFMA and vector instructions interleaved by
+// hand, and two waves per SIMD at 3 tiles, measured no better.
 #define GRAM_MMAX 48
-#define GRAM_ITEMS 4 /* staged (cell, vector) items per thread and segment */
-
-// 16-byte slots per staged cell of mp vectors: three features each, then one
-// or two spare so that the count is odd
-__host__ __device__ inline int gram_cell_slots(int mp) { return 3 * mp + ((3 * mp) & 1 ? 2 : 1); }
+#define GRAM_STRIP 8
 
 MXH_DEV void pair_ab(int p, int& a, int& b)
 {
@@ -841,200 +857,226 @@ MXH_DEV void pair_ab(int p, int& a, int& b)
   b = p - r * (r + 1) / 2;
 }
 
-// Gram products of each problem's block, register-blocked: thread (group g,
-// block pair (A, B)) accumulates the GB x GB pairs a = A GB + ka, b = B GB + kb
-// (A >= B) over the cells t = g, g + ngrp, ... of each staged row segment.
-// Per cell and vector three features are staged in LDS, the curl c and the
-// mass factors ux, uy above (from x(i,j), x(i,j+1), y(i,j), y(i+1,j) only),
-// so a pair costs three complex multiply-adds per cell:
-//   K_ab += conj(c_a) eta c_b,   M_ab += conj(ux_a) ux_b + conj(uy_a) uy_b.
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+// the value of lane ^ 8 (a rotation by 8 in each row of 16 lanes) where the
+// bank mask selects (banks of four lanes: 0xf all, 0x3 lanes 0-7 of a row,
+// 0xc lanes 8-15), elsewhere old
+template <int BANKS>
+MXH_DEV double lane_xor8(double old, double v)
+{
+  union { double d; int i[2]; } u, o;
+  u.d = v;
+  o.d = old;
+  o.i[0] = __builtin_amdgcn_update_dpp(o.i[0], u.i[0], 0x128, 0xf, BANKS, false);
+  o.i[1] = __builtin_amdgcn_update_dpp(o.i[1], u.i[1], 0x128, 0xf, BANKS, false);
+  return o.d;
+}
+
+struct gram_false { static constexpr bool value = false; };
+struct gram_true { static constexpr bool value = true; };
+
+struct GramArgs {
+  const C<double>* U;  // the problem's first vector
+  long long us;
+  const int* cl;       // its column list (after the count), or null
+  const double* eta;
+  double* out;         // the workgroup's partial sums
+  C<double> xf, yf;
+  double xa, xb, ya, yb;
+  int nx, ny, mq, j0, j1;
+};
+
+// The sums of one workgroup's rows over Q tiles (8 vectors each): K (MATS & 1)
+// and M (MATS & 2).
+template <int Q, int MATS = 3>
+MXH_DEV void gram_rows(const GramArgs& g, double* lds)
+{
+  constexpr int NP = Q * (Q + 1) / 2;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = (lane >> 3) & 1, k2 = 2 * (lane >> 4);
+  const int nx = g.nx, ny = g.ny;
+  const size_t N = (size_t)nx * ny;
+  const C<double>* u[Q];
+#pragma unroll
+  for (int t = 0; t < Q; t++) {
+    // columns past the list repeat the last one; their sums are not written
+    const int a = min(8 * t + (lane & 7), g.mq - 1);
+    u[t] = g.U + (size_t)(g.cl ? g.cl[a] : a) * g.us;
+  }
+  v4d K[NP], M[NP];
+#pragma unroll
+  for (int p = 0; p < NP; p++) K[p] = M[p] = v4d{0.0, 0.0, 0.0, 0.0};
+  // the waves share the strips of a row, or the rows where there are few strips
+  const int ns = (nx + GRAM_STRIP - 1) / GRAM_STRIP;
+  int ja = g.j0, jb = g.j1, s0 = wave, sstep = 4;
+  if (ns < 4) {
+    const int sub = (g.j1 - g.j0 + 3) >> 2;
+    ja = min(g.j1, g.j0 + wave * sub);
+    jb = min(g.j1, ja + sub);
+    s0 = 0;
+    sstep = 1;
+  }
+  for (int s = s0; s < ns; s += sstep) {
+    if (ja >= jb) break;
+    const int cell = GRAM_STRIP * s + k2 + h, i = min(cell, nx - 1);
+    const bool last = GRAM_STRIP * s + GRAM_STRIP >= nx;  // wraps in x (and may hold cells past the grid)
+    const int ir = i + 1 < nx ? i + 1 : 0;
+    const int ie = min(GRAM_STRIP * s + k2, nx - 1), io = min(GRAM_STRIP * s + k2 + 1, nx - 1);
+    C<double> x0[Q], x1[Q], y0[Q], yr[Q];
+    size_t row = (size_t)ja * nx, up = (size_t)(ja + 1 < ny ? ja + 1 : 0) * nx;
+    double ee = g.eta[row + ie], eo = g.eta[row + io];
+#pragma unroll
+    for (int t = 0; t < Q; t++) {
+      x0[t] = u[t][row + i];
+      x1[t] = u[t][up + i];
+      y0[t] = u[t][N + row + i];
+      yr[t] = u[t][N + row + ir];
+    }
+    // Row j of the strip.  edge: the strip wraps in x, or the row in y; the
+    // other rows run without the test, as a loop of one block, so that the
+    // next row's loads stay where they are issued
+    auto row_step = [&](int j, auto edge) {
+      const double e0 = ee, e1 = eo;
+      // the next row (the last one loads itself again)
+      const int jn = j + 1 < jb ? j + 1 : j;
+      row = (size_t)jn * nx;
+      up = (size_t)(jn + 1 < ny ? jn + 1 : 0) * nx;
+      ee = g.eta[row + ie];
+      eo = g.eta[row + io];
+      double F[Q][3][2];
+#pragma unroll
+      for (int t = 0; t < Q; t++) {
+        if constexpr (decltype(edge)::value) {
+          if (j + 1 == ny) x1[t] = g.yf * x1[t];
+          if (i + 1 == nx) yr[t] = g.xf * yr[t];
+          if (cell >= nx) x0[t] = x1[t] = y0[t] = yr[t] = czero<double>();
+        }
+        C<double> f[3];
+        f[0] = x0[t] - x1[t] - y0[t] + yr[t];
+        f[1] = g.xa * x0[t] + g.xb * x1[t];
+        f[2] = g.ya * y0[t] + g.yb * yr[t];
+        x0[t] = x1[t];
+        x1[t] = u[t][up + i];
+        y0[t] = u[t][N + row + i];
+        yr[t] = u[t][N + row + ir];
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+          // lanes 0-7 hold the even cell, lanes 8-15 the odd one: the even
+          // cell's operand takes its imaginary parts to lanes 8-15, the odd
+          // cell's its real parts to lanes 0-7
+          F[t][q][0] = lane_xor8<0xc>(f[q].r, f[q].i);
+          F[t][q][1] = lane_xor8<0x3>(f[q].i, f[q].r);
+        }
+        const double a0 = e0 * F[t][0][0], a1 = e1 * F[t][0][1];
+        const int p0 = t * (t + 1) / 2;
+        auto mac = [&](v4d* acc, double l, int q, int cell2) {
+#pragma unroll
+          for (int c = 0; c <= t; c++)
+            acc[p0 + c] = __builtin_amdgcn_mfma_f64_16x16x4f64(l, F[c][q][cell2], acc[p0 + c], 0, 0, 0);
+        };
+        if (MATS & 1) mac(K, a0, 0, 0);
+        if (MATS & 2) mac(M, F[t][1][0], 1, 0);
+        if (MATS & 1) mac(K, a1, 0, 1);
+        if (MATS & 2) {
+          mac(M, F[t][1][1], 1, 1);
+          mac(M, F[t][2][0], 2, 0);
+          mac(M, F[t][2][1], 2, 1);
+        }
+      }
+    };
+    int j = ja;
+    if (!last)
+      for (const int je = min(jb, ny - 1); j < je; j++) row_step(j, gram_false());
+    for (; j < jb; j++) row_step(j, gram_true());
+  }
+  // Element e of a tile in lane (j = lane & 15, im = lane >> 4) is row 4 e +
+  // im, column j.  With a = row & 7, b = column & 7 the complex sum is
+  // rr + ii + i (ri - ir): lanes j < 8 form the real part of rows 4 e + im,
+  // e < 2, lanes j >= 8 the imaginary part.  Summed over the waves in order.
+  for (int w = 0; w < 4; w++) {
+    if (wave == w) {
+#pragma unroll
+      for (int p = 0; p < NP; p++)
+#pragma unroll
+        for (int mat = 0; mat < 2; mat++) {
+          if (!(MATS >> mat & 1)) continue;
+          const v4d d = mat ? M[p] : K[p];
+#pragma unroll
+          for (int e = 0; e < 2; e++) {
+            const double o = lane_xor8<0xf>(0.0, d[e + 2]);
+            const double v = h ? d[e] - o : d[e] + o;
+            double* q = lds + ((p * 2 + mat) * 2 + e) * 64 + lane;
+            *q = w ? *q + v : v;
+          }
+        }
+    }
+    __syncthreads();
+  }
+  for (int w = tid; w < NP * 256; w += 256) {
+    const int l = w & 63, e = (w >> 6) & 1, mat = (w >> 7) & 1;
+    int T, S;
+    pair_ab(w >> 8, T, S);
+    const int a = 8 * T + 4 * e + (l >> 4), b = 8 * S + (l & 7);
+    if ((MATS >> mat & 1) && a < g.mq && b <= a) g.out[4 * (a * (a + 1) / 2 + b) + 2 * mat + ((l >> 3) & 1)] = lds[w];
+  }
+}
+
 // A workgroup covers a band of rows of one problem; bands are summed by
-// k_reduce_partials in a fixed order.  The segment width T and the item
-// count per thread are chosen by mxh_gram; the next segment's loads stay in
-// flight in registers while the current one is summed (two waves per SIMD).
-// With a column list (cmap: per problem q, cmap[q (m+1)] = mq columns, then
-// their indices in the block, increasing) a problem's sums run over those mq
+// k_reduce_partials in a fixed order.  NT: tiles of the widest block.  With a
+// column list (cmap: per problem q, cmap[q (m+1)] = mq columns, then their
+// indices in the block, increasing) a problem's sums run over those mq
 // columns only and land at the pair indices of the list (pair a (a+1)/2 + b
 // of list positions a >= b); the rest of its output is left unwritten.
-#define GB 3
-
-__global__ __launch_bounds__(256) void k_gram(mxh_level lv, mxh_bloch bl, int m, const int* pmap, const int* cmap,
-                                              const C<double>* U0, long long us, const double* eta, double* part,
-                                              int T, int rpb)
+template <int NT>
+__global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gram(mxh_level lv, mxh_bloch bl, int m, const int* pmap,
+                                                               const int* cmap, const C<double>* U0, long long us,
+                                                               const double* eta, double* part, int rpb)
 {
   extern __shared__ double smem[];
   const int jb = blockIdx.y;
   const int prob = pmap ? pmap[jb] : jb;
-  const C<double>* U = U0 + (size_t)prob * m * us;
   const int* cl = cmap ? cmap + (size_t)prob * (m + 1) : nullptr;
   const int mq = cl ? cl[0] : m;  // columns summed (block-uniform)
   if (mq < 1 || mq > m) return;   // (the whole block: before any barrier)
-  const int nx = lv.nx, ny = lv.ny;
-  const size_t N = (size_t)nx * ny;
-  const int nbk = (mq + GB - 1) / GB, nbp = nbk * (nbk + 1) / 2;
-  // per cell the features of mp = nbk GB vectors (zero beyond m), then one or
-  // two spare complex: an odd number of 16-byte slots between cells keeps the
-  // cells a wavefront stages (and the groups read) on different banks
-  const int mp = nbk * GB, cs = gram_cell_slots(mp);
-  C<double>* sf = (C<double>*)smem;                    // [T][cs]
-  double* se = (double*)(sf + (size_t)T * cs);         // [T]
-  const Geo<double> g = make_geo<double>(lv, bl, prob * m);
+  const Geo<double> gg = make_geo<double>(lv, bl, prob * m);
+  GramArgs g;
+  g.U = U0 + (size_t)prob * m * us;
+  g.us = us;
+  g.cl = cl ? cl + 1 : nullptr;
+  g.eta = eta;
+  g.out = part + ((size_t)blockIdx.x * gridDim.y + jb) * 4 * (m * (m + 1) / 2);
+  g.xf = gg.xf;
+  g.yf = gg.yf;
   // the mass factors' weights: sqrt(6 mx) a, sqrt(6 mx) b (x-edges), sqrt(6 my) a, sqrt(6 my) b
-  const double fa_ = 0.5 * (1.0 + 1.0 / sqrt(3.0)), fb_ = 0.5 * (1.0 - 1.0 / sqrt(3.0));
+  const double fa = 0.5 * (1.0 + 1.0 / sqrt(3.0)), fb = 0.5 * (1.0 - 1.0 / sqrt(3.0));
   const double sxm = sqrt(lv.hy / lv.hx), sym = sqrt(lv.hx / lv.hy);
-  const double xa = sxm * fa_, xb = sxm * fb_, ya = sym * fa_, yb = sym * fb_;
-  const int ngrp = (int)blockDim.x / nbp;
-  const int tid = threadIdx.x, grp = tid / nbp, bp = tid % nbp;
-  int A, Bq;
-  pair_ab(bp, A, Bq);
-  const bool act = grp < ngrp;
-  C<double> K[GB][GB], Mm[GB][GB];
-#pragma unroll
-  for (int x = 0; x < GB; x++)
-#pragma unroll
-    for (int y = 0; y < GB; y++) K[x][y] = Mm[x][y] = czero<double>();
-  const int j0 = blockIdx.x * rpb, j1 = j0 + rpb < ny ? j0 + rpb : ny;
-  // items w = tid + r blockDim (r < GRAM_ITEMS, mp T <= GRAM_ITEMS blockDim) of
-  // a full segment: vector a = w / T, cell t = w mod T (consecutive threads on
-  // consecutive cells); a >= mp marks no item
-  int pa[GRAM_ITEMS], pt[GRAM_ITEMS];
-#pragma unroll
-  for (int r = 0; r < GRAM_ITEMS; r++) {
-    const int w = tid + r * (int)blockDim.x;
-    pa[r] = w / T;
-    pt[r] = w - pa[r] * T;
-  }
-  // segments sg = (row j, columns i0 .. i0 + T - 1) of the band, column of
-  // segments by column of segments: rows j and j + 1 of one column follow each
-  // other, so a thread keeps the x-edge value of row j + 1 it loaded for row j
-  // (the curl and the mass factor read x at j and j + 1) and loads one new x
-  // row per segment instead of two.  The loads of segment sg + 1 are issued
-  // before segment sg is summed, so their latency hides behind the products.
-  const int nrow = j1 - j0, nseg = (nx + T - 1) / T, sEnd = nrow * nseg;
-  int ia[GRAM_ITEMS], it[GRAM_ITEMS];
-  C<double> v[GRAM_ITEMS][4];  // x(i,j), y(i,j), x(i,j+1), y(i+1,j), raw
-  // eta of the cell of item 0: the one item of vector 0 a thread can hold
-  // (items r >= 1 have w >= blockDim > T cells)
-  double ev0 = 0.0;
-  // all loads of the thread's items of segment sg (clamped to a real vector,
-  // so every address is valid); with next_row, sg is the row after the
-  // segment whose raw values v holds, in the same column
-  auto load = [&](int sg, bool next_row) {
-    const int j = j0 + sg % nrow, i0 = (sg / nrow) * T;
-    const int cnt = nx - i0 < T ? nx - i0 : T;
-    // the next row; across the periodic boundary with the Bloch factor
-    const long long offp = j + 1 < ny ? nx : -(long long)(ny - 1) * nx;
-#pragma unroll
-    for (int r = 0; r < GRAM_ITEMS; r++) {
-      ia[r] = pa[r];
-      it[r] = pt[r];
-      if (cnt != T) {
-        const int w = tid + r * (int)blockDim.x;
-        ia[r] = w / cnt;
-        it[r] = w - ia[r] * cnt;
-      }
-      const int a = ia[r] < mq ? ia[r] : mq - 1, i = i0 + it[r];
-      const C<double>* ux = U + (size_t)(cl ? cl[1 + a] : a) * us;
-      const C<double>* uy = ux + N;
-      const long long k = i + (long long)j * nx;
-      if (next_row) {
-        // x(i, j) was this item's x(i, j + 1) one row up
-        v[r][0] = v[r][2];
-      } else {
-        v[r][0] = ux[k];
-      }
-      v[r][1] = uy[k];
-      v[r][2] = ux[k + offp];
-      v[r][3] = uy[i + 1 < nx ? k + 1 : k + 1 - nx];
-      if (r == 0) ev0 = eta[k];
-    }
-  };
-  if (sEnd > 0) load(0, false);
-  for (int sg = 0; sg < sEnd; sg++) {
-    const int j = j0 + sg % nrow, i0 = (sg / nrow) * T;
-    const int cnt = nx - i0 < T ? nx - i0 : T;
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < GRAM_ITEMS; r++) {
-      const int a = ia[r], t = it[r], i = i0 + t;
-      if (a >= mp) continue;
-      C<double>* f = sf + (size_t)t * cs + a * 3;
-      if (a >= mq) {
-        f[0] = f[1] = f[2] = czero<double>();
-        continue;
-      }
-      const C<double> x0 = v[r][0], y0 = v[r][1];
-      C<double> xp = v[r][2], yp = v[r][3];
-      if (j + 1 == ny) xp = g.yf * xp;
-      if (i + 1 == nx) yp = g.xf * yp;
-      f[0] = x0 - xp - y0 + yp;
-      f[1] = xa * x0 + xb * xp;
-      f[2] = ya * y0 + yb * yp;
-      if (r == 0 && a == 0) se[t] = ev0;
-    }
-    __syncthreads();
-    if (sg + 1 < sEnd) load(sg + 1, (sg + 1) % nrow != 0);
-    if (act) {
-      for (int t = grp; t < cnt; t += ngrp) {
-        const C<double>* f = sf + (size_t)t * cs;
-        const double et = se[t];
-        C<double> fa[GB][3];
-#pragma unroll
-        for (int ka = 0; ka < GB; ka++) {
-          const int a = A * GB + ka;
-#pragma unroll
-          for (int q = 0; q < 3; q++) fa[ka][q] = f[a * 3 + q];
-        }
-#pragma unroll
-        for (int kb = 0; kb < GB; kb++) {
-          const int b = Bq * GB + kb;
-          const C<double>* fb = f + b * 3;
-          const C<double> ec = et * fb[0], wx = fb[1], wy = fb[2];
-#pragma unroll
-          for (int ka = 0; ka < GB; ka++) {
-            cmac_conj(K[ka][kb], fa[ka][0], ec);
-            cmac_conj(Mm[ka][kb], fa[ka][1], wx);
-            cmac_conj(Mm[ka][kb], fa[ka][2], wy);
-          }
-        }
-      }
-    }
-  }
-  // sum the groups through LDS, one pair of the block at a time
-  const int np = m * (m + 1) / 2;
-  double* out = part + ((size_t)blockIdx.x * gridDim.y + jb) * 4 * np;
-  double* red = smem;  // [blockDim.x][4]
-#pragma unroll
-  for (int ka = 0; ka < GB; ka++)
-#pragma unroll
-    for (int kb = 0; kb < GB; kb++) {
+  g.xa = sxm * fa;
+  g.xb = sxm * fb;
+  g.ya = sym * fa;
+  g.yb = sym * fb;
+  g.nx = lv.nx;
+  g.ny = lv.ny;
+  g.mq = mq;
+  g.j0 = min(lv.ny, (int)blockIdx.x * rpb);
+  g.j1 = min(lv.ny, g.j0 + rpb);
+  // the tiles this problem's columns fill (uniform)
+  switch (min((mq + 7) / 8, NT)) {
+  case 1: gram_rows<1>(g, smem); break;
+  case 2: if constexpr (NT >= 2) gram_rows<2>(g, smem); break;
+  case 3: if constexpr (NT >= 3) gram_rows<3>(g, smem); break;
+  case 4: if constexpr (NT >= 4) gram_rows<4>(g, smem); break;
+  case 5: if constexpr (NT >= 5) gram_rows<5>(g, smem); break;
+  case 6:
+    // both matrices' sums of 21 tile pairs would not fit in registers: one
+    // after the other (the inputs read twice)
+    if constexpr (NT >= 6) {
+      gram_rows<6, 1>(g, smem);
       __syncthreads();
-      red[4 * tid] = K[ka][kb].r;
-      red[4 * tid + 1] = K[ka][kb].i;
-      red[4 * tid + 2] = Mm[ka][kb].r;
-      red[4 * tid + 3] = Mm[ka][kb].i;
-      __syncthreads();
-      if (tid < nbp) {
-        int Ae, Be;
-        pair_ab(tid, Ae, Be);
-        const int a = Ae * GB + ka, b = Be * GB + kb;
-        if (a < mq && b < mq && a >= b) {
-          double v0 = 0, v1 = 0, v2 = 0, v3 = 0;
-          for (int gq = 0; gq < ngrp; gq++) {
-            const double* r = red + 4 * (gq * nbp + tid);
-            v0 += r[0];
-            v1 += r[1];
-            v2 += r[2];
-            v3 += r[3];
-          }
-          double* o = out + 4 * (a * (a + 1) / 2 + b);
-          o[0] = v0;
-          o[1] = v1;
-          o[2] = v2;
-          o[3] = v3;
-        }
-      }
+      gram_rows<6, 2>(g, smem);
     }
+    break;
+  }
 }
 
 // ----------------------------------------------------------------- block combine
@@ -3995,31 +4037,43 @@ static int gram_launch(const mxh_level* lv, const mxh_bloch* bl, int nprob, cons
                        mxh_vecs u, const double* eta64, double* out, void* work, int sets_cap)
 {
   if (m < 1 || m > GRAM_MMAX || nprob < 1 || sets_cap < 1) return (int)hipErrorInvalidValue;
-  const int np = m * (m + 1) / 2;
-  const int nbk = (m + GB - 1) / GB, nbp = nbk * (nbk + 1) / 2;
-  if (nbp > TPB) return (int)hipErrorInvalidValue;
-  // row segment staged per step: T cells of gram_cell_slots(mp) complex and
-  // one double each within 64 KB, mp T <= GRAM_ITEMS TPB items.  The kernel's registers
-  // allow two workgroups per CU, which the LDS of the widest segment still
-  // fits; wider segments (fewer barriers) beat an even spread of cells over
-  // the thread groups (block 12: T = 64 measured 9% faster than T = 50).
-  const int mp = nbk * GB;
-  const size_t cell = (size_t)gram_cell_slots(mp) * sizeof(C<double>) + sizeof(double);
-  int T = GRAM_TILE_MAX;
-  while (T > 1 && (T * cell > 65536 || mp * T > GRAM_ITEMS * TPB)) T--;
-  // row bands: bands * nprob partial sets (sets_cap or nprob) fit the work
-  // buffer; the kernel walks each band's segment columns down the rows, so
-  // taller bands reload fewer x rows (8 rows per band for 32 problems at 512^2)
+  const int np = m * (m + 1) / 2, nt = (m + 7) / 8;
+  // Row bands: bands * nprob partial sets (sets_cap or nprob) fit the work
+  // buffer.  Workgroups run in rounds of `slots` (one to four per compute unit,
+  // by the registers of the tiles' sums) and a band costs its rows and about
+  // one row for its start, so the height minimises rounds x (rows + 1).  36
+  // columns, 16 problems of 512^2: 4, 8, 16, 32 rows measured 2.00, 1.79, 1.69,
+  // 1.66 ms, 64 rows (half the units idle) 3.19.
   const int sets = nprob > sets_cap ? nprob : sets_cap;
-  int bands = sets / nprob;
-  if (bands > lv->ny) bands = lv->ny;
-  if (bands < 1) bands = 1;
-  const int rpb = (lv->ny + bands - 1) / bands;
-  bands = (lv->ny + rpb - 1) / rpb;
-  size_t sh = T * cell;
-  if (sh < TPB * 4 * sizeof(double)) sh = TPB * 4 * sizeof(double);
-  hipLaunchKernelGGL(k_gram, dim3(bands, nprob), dim3(TPB), sh, g_stream, *lv, *bl, m, pmap, cmap,
-                     (const C<double>*)u.p, u.stride, eta64, (double*)work, T, rpb);
+  const long long slots = (long long)mxh_cu_count() * (nt == 1 ? 4 : nt == 2 ? 2 : 1);
+  int rpb = lv->ny;
+  long long cost = -1;
+  for (int r = 1; r <= 64 && r <= lv->ny; r++) {
+    const long long wgs = (long long)((lv->ny + r - 1) / r) * nprob;
+    if (wgs > sets) continue;
+    const long long c = (wgs + slots - 1) / slots * (r + 1);
+    if (cost < 0 || c <= cost) {
+      cost = c;
+      rpb = r;
+    }
+  }
+  const int bands = (lv->ny + rpb - 1) / rpb;
+  const size_t sh = sizeof(double) * 256 * (size_t)(nt * (nt + 1) / 2);
+  const dim3 grid(bands, nprob);
+#define GRAM_CASE(NT)                                                                                       \
+  case NT:                                                                                                  \
+    hipLaunchKernelGGL(k_gram<NT>, grid, dim3(TPB), sh, g_stream, *lv, *bl, m, pmap, cmap,                  \
+                       (const C<double>*)u.p, u.stride, eta64, (double*)work, rpb);                         \
+    break;
+  switch (nt) {
+    GRAM_CASE(1)
+    GRAM_CASE(2)
+    GRAM_CASE(3)
+    GRAM_CASE(4)
+    GRAM_CASE(5)
+    GRAM_CASE(6)
+  }
+#undef GRAM_CASE
   LAUNCH_CHECK();
   int width = 4 * np * nprob;
   hipLaunchKernelGGL(k_reduce_partials, dim3(reduce_blocks(width)), dim3(TPB), 0, g_stream, (const double*)work,
