@@ -66,6 +66,10 @@ void *mxh_malloc(size_t bytes);
 void mxh_free(void *p);
 int mxh_h2d(void *dst, const void *src, size_t bytes);
 int mxh_d2h(void *dst, const void *src, size_t bytes); /* synchronous */
+/* The same for `rows` rows of `row` bytes, dense on the host and a pitch of
+   dst_pitch / src_pitch bytes apart on the device (d2h: synchronous). */
+int mxh_h2d_rows(void *dst, size_t dst_pitch, const void *src, size_t row, int rows);
+int mxh_d2h_rows(void *dst, const void *src, size_t src_pitch, size_t row, int rows);
 /* Stream-ordered device-to-host copy that returns at once; dst must come from
    mxh_host_alloc (pinned) for the copy to overlap the host's work.  Wait for
    it with an event recorded after it. */

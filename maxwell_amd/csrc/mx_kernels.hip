@@ -3620,6 +3620,20 @@ int mxh_d2h(void* dst, const void* src, size_t bytes)
   return (int)hipStreamSynchronize(g_stream);
 }
 
+int mxh_h2d_rows(void* dst, size_t dst_pitch, const void* src, size_t row, int rows)
+{
+  if (dst_pitch == row) return mxh_h2d(dst, src, row * (size_t)rows);
+  return (int)hipMemcpy2DAsync(dst, dst_pitch, src, row, row, rows, hipMemcpyHostToDevice, g_stream);
+}
+
+int mxh_d2h_rows(void* dst, const void* src, size_t src_pitch, size_t row, int rows)
+{
+  if (src_pitch == row) return mxh_d2h(dst, src, row * (size_t)rows);
+  hipError_t e = hipMemcpy2DAsync(dst, row, src, src_pitch, row, rows, hipMemcpyDeviceToHost, g_stream);
+  if (e != hipSuccess) return (int)e;
+  return (int)hipStreamSynchronize(g_stream);
+}
+
 int mxh_d2h_async(void* dst, const void* src, size_t bytes)
 {
   return (int)hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g_stream);
