@@ -107,8 +107,8 @@ int mxh_edge_gs_phase(int prec, const mxh_level *lv, const mxh_bloch *bl, int nv
                       mxh_vecs b, mxh_vecs x, const void *eta, const mxh_coef *cf,
                       int colour);
 
-/* Tile-fused AFW sweeps with operator K + M (alpha = beta = 1), reading x
-   and writing the result to xo (a different buffer: workgroups read halo
+/* Tile-fused AFW sweeps (grids of at most 64 x 64: the whole grid in LDS)
+   with operator K + M (alpha = beta = 1), reading x and writing the result to xo (a different buffer: workgroups read halo
    nodes that other workgroups own).  mode bits:
    1 backward colour order (then nsweep must be 1), 2 x starts at zero,
    4 add P xc_in to x first (coarse correction of the V-cycle),
@@ -118,6 +118,32 @@ int mxh_edge_gs_phase(int prec, const mxh_level *lv, const mxh_bloch *bl, int nv
 int mxh_afw_tile(int prec, const mxh_level *lv, const mxh_bloch *bl, int nv,
                  mxh_vecs b, mxh_vecs x, mxh_vecs xo, const void *eta, int nsweep,
                  int mode, mxh_vecs xc_in, mxh_vecs bc, mxh_vecs xc);
+
+/* The coarse end of a V(nu, nu) cycle in one launch, one workgroup per vector:
+   levels 0 .. n - 1 (each twice the one below, even sizes, the top one of at
+   most 1024 nodes), nu forward sweeps, residual and restriction down, the
+   coarsest level by the inverse of its matrix, prolongation and nu backward
+   sweeps up, with the operators and the sweep order of mxh_afw_tile and
+   mxh_node_tile.  b (b.map honoured by the edge cycle) and x: vectors of the
+   top level; xzero: x is zero on entry (and not read).  W: inverse of the
+   coarsest matrix as mxh_coarse_inverse writes it, of problem g / vpp with
+   per_problem, else one for all.  With b and x of a lower level given
+   (nv = 1) its right-hand side and solution are written there. */
+#define MXH_CYCLE_MAXL 6
+typedef struct {
+  int n;
+  mxh_level lv[MXH_CYCLE_MAXL];
+  const void *eta[MXH_CYCLE_MAXL]; /* edge cycles, in the vector precision */
+  void *b[MXH_CYCLE_MAXL], *x[MXH_CYCLE_MAXL];
+} mxh_cycle;
+int mxh_cycle_supported(int prec, const mxh_cycle *cy);
+int mxh_edge_cycle(int prec, const mxh_cycle *cy, const mxh_bloch *bl, int nv, int nu, mxh_vecs b, mxh_vecs x,
+                   int xzero, const double *W, int per_problem);
+int mxh_node_cycle(int prec, const mxh_cycle *cy, const mxh_bloch *bl, int nv, int nu, mxh_vecs b, mxh_vecs x,
+                   int xzero, const double *W, int per_problem);
+/* W[p] = A[p]^-1 (n x n complex, row-major) from the Cholesky factors L[p] of
+   mxh_coarse_setup or mxh_coarse_solve; n <= 256. */
+int mxh_coarse_inverse(int n, int nprob, const double *L, double *W);
 
 /* Coarse b_v = R (bf_v - (K + M) xf_v); coarse x_v = 0. */
 int mxh_resid_restrict(int prec, const mxh_level *fine, const mxh_bloch *bl,

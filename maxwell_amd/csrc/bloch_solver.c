@@ -46,6 +46,9 @@ struct mx_solver {
   void *ex2[MX_MAXL], *nxv2[MX_MAXL]; /* second x buffers: tile kernels write here, then swap */
   void *lift_table;     /* the direct lifting's table; null: node V-cycles */
   void *rdef;           /* defects of a block step (MG precision, defect slots) */
+  mxh_cycle cyc;        /* levels 0 .. lc of the edge V-cycle, run in one launch */
+  int lc;               /* -1: none (one launch per pass on every level) */
+  double *dAi;          /* inverses of the coarse edge matrices (lc >= 0) */
   double *dbloch, *dAe, *dAn, *dlam, *dnorm, *dgram, *dC, *dwork, *dcoef;
   void *gramwork;
   int ne0, nn0;         /* coarse edge / node unknowns */
@@ -127,6 +130,7 @@ void mx_solver_destroy(mx_solver *s)
   mxh_free(s->dbloch);
   mxh_free(s->dAe);
   mxh_free(s->dAn);
+  mxh_free(s->dAi);
   mxh_free(s->dlam);
   mxh_free(s->dnorm);
   mxh_free(s->dgram);
@@ -243,6 +247,24 @@ int mx_solver_create(const mx_config *cfg, const double *eta, mx_solver **out)
     s->nxv2[l] = dalloc(s, s->csz * (size_t)ndim(s, l) * nv);
     if (!s->eb[l] || !s->ex[l] || !s->nb[l] || !s->nxv[l] || !s->ex2[l] || !s->nxv2[l]) goto nomem;
   }
+  /* the coarse levels that fit one workgroup's LDS run as one launch */
+  s->lc = -1;
+  if (!cfg->phase_kernels && cfg->smoother_steps > 0) {
+    mxh_cycle c;
+    memset(&c, 0, sizeof(c));
+    for (int l = 0; l <= s->L && l < MXH_CYCLE_MAXL; l++) {
+      c.n = l + 1;
+      c.lv[l] = s->lv[l];
+      c.eta[l] = s->etaP[l];
+      if (!mxh_cycle_supported(s->prec, &c)) break;
+      s->cyc = c;
+      s->lc = l;
+    }
+  }
+  if (s->lc >= 0) {
+    s->dAi = (double *)dalloc(s, 16 * (size_t)s->ne0 * s->ne0 * P);
+    if (!s->dAi) goto nomem;
+  }
   s->rdef = dalloc(s, s->csz * (size_t)edim(s, s->L) * nv);
   if (!s->rdef) goto nomem;
   if (!cfg->phase_kernels && mxh_lift_supported(s->prec, &s->lv[s->L])) {
@@ -339,6 +361,7 @@ static int tune_bucket(const mx_solver *s, int nv)
 static int march_rows_of(const mx_solver *s, int node, int l, int nv)
 {
   if (s->lv[l].nx < 8 || s->lv[l].ny < 8) return 0; /* halo of one sweep: 6 */
+  if (!node && l <= s->lc) return 0;                /* run by the coarse cycle */
   if (s->tuned && !(node && s->lift_table)) return s->tune_rows[tune_bucket(s, nv)][node][l];
   if (s->cfg.march_min <= 0) return 0;
   const int rows = s->cfg.march_rows > 0 ? s->cfg.march_rows : 128;
@@ -409,7 +432,7 @@ static int autotune(mx_solver *s, int nv_full, const mxh_bloch *bl)
     if (nv < 1 || (bk > 0 && nv == s->tune_nv[bk - 1])) break;
     s->tune_nv[bk] = nv;
     for (int node = 0; node < (s->lift_table ? 1 : 2) && !err; node++)
-      for (int l = 1; l <= s->L && !err; l++) {
+      for (int l = node || s->lc < 1 ? 1 : s->lc + 1; l <= s->L && !err; l++) {
         const long long n = node ? ndim(s, l) : edim(s, l);
         void **bb = node ? s->nb : s->eb, **xx = node ? s->nxv : s->ex;
         err |= mxh_random(s->prec, n, nv, V(bb[l], n), 7 + l, 0);
@@ -461,7 +484,8 @@ static int vcycle_edge(mx_solver *s, int nv, const mxh_bloch *bl, int xzero, mxh
 {
   const int P = s->prec, nu = s->cfg.smoother_steps;
   const mxh_vecs none = V(NULL, 0);
-  for (int l = s->L; l > 0; l--) {
+  const int lc = s->lc > 0 ? s->lc : 0;
+  for (int l = s->L; l > lc; l--) {
     mxh_vecs b = l == s->L && bfine.p ? bfine : V(s->eb[l], edim(s, l)), x = V(s->ex[l], edim(s, l));
     mxh_vecs bc = V(s->eb[l - 1], edim(s, l - 1)), xc = V(s->ex[l - 1], edim(s, l - 1));
     const int xz = (l < s->L) || xzero;
@@ -482,10 +506,14 @@ static int vcycle_edge(mx_solver *s, int nv, const mxh_bloch *bl, int xzero, mxh
       }
     }
   }
-  CK(mxh_coarse_solve(P, s->ne0, NULL, s->dAe, s->vpp, bl->vmap, nv, V(s->eb[0], edim(s, 0)),
-                      V(s->ex[0], edim(s, 0))));
+  if (s->lc >= 0)
+    CK(mxh_edge_cycle(P, &s->cyc, bl, nv, nu, lc == s->L && bfine.p ? bfine : V(s->eb[lc], edim(s, lc)),
+                      V(s->ex[lc], edim(s, lc)), lc < s->L || xzero, s->dAi, 1));
+  else
+    CK(mxh_coarse_solve(P, s->ne0, NULL, s->dAe, s->vpp, bl->vmap, nv, V(s->eb[0], edim(s, 0)),
+                        V(s->ex[0], edim(s, 0))));
   s->st.launches += 1;
-  for (int l = 1; l <= s->L; l++) {
+  for (int l = lc + 1; l <= s->L; l++) {
     mxh_vecs b = l == s->L && bfine.p ? bfine : V(s->eb[l], edim(s, l)), x = V(s->ex[l], edim(s, l));
     mxh_vecs xc = V(s->ex[l - 1], edim(s, l - 1));
     if (s->cfg.phase_kernels || nu == 0) {
@@ -856,7 +884,7 @@ static int precondition_to(mx_solver *s, int ng, const mxh_bloch *blg, double *E
      were formed, through the set's slot map; otherwise they are gathered */
   mxh_vecs src = V(s->rdef, n), bfine = V(NULL, 0);
   src.map = dbmap;
-  if (!s->cfg.phase_kernels && s->cfg.smoother_steps > 0 && march_rows_of(s, 0, L, ng) > 0) {
+  if (!s->cfg.phase_kernels && s->cfg.smoother_steps > 0 && (s->lc == L || march_rows_of(s, 0, L, ng) > 0)) {
     bfine = src;
   } else {
     CK(mxh_gather(s->prec, n, ng, V(s->eb[L], n), src));
@@ -961,6 +989,7 @@ static int setup_problems(mx_solver *s, int nprob, const double *kx, const doubl
     CK(mxh_d2h(s->hinfo, s->dinfo, sizeof(int) * P));
     for (int p = 0; p < P; p++)
       if (s->hinfo[p]) return MX_ELAPACK;
+    if (s->lc >= 0) CK(mxh_coarse_inverse(ne0, P, s->dAe, s->dAi));
     return MX_OK;
   }
   for (int p = 0; p < P; p++) {
@@ -975,6 +1004,7 @@ static int setup_problems(mx_solver *s, int nprob, const double *kx, const doubl
   }
   CK(mxh_h2d(s->dAe, s->hAe, sizeof(double complex) * (size_t)ne0 * ne0 * P));
   CK(mxh_h2d(s->dAn, s->hAn, sizeof(double complex) * (size_t)nn0 * nn0 * P));
+  if (s->lc >= 0) CK(mxh_coarse_inverse(ne0, P, s->dAe, s->dAi));
   return MX_OK;
 }
 

@@ -267,6 +267,10 @@ __global__ void k_reduce_partials(const double* __restrict__ part, int nblk, int
 
 static const int TPB = 256;
 
+// the LDS of a compute unit, and bytes per complex value
+#define LDS_MAX (160 * 1024)
+static size_t csize(int prec) { return prec == MXH_F64 ? 16 : 8; }
+
 static inline unsigned nblocks(long long n, int tpb = TPB) { return (unsigned)((n + tpb - 1) / tpb); }
 
 // k_reduce_partials over `width` outputs: four outputs per 256-thread block
@@ -2725,6 +2729,696 @@ __global__ __launch_bounds__(1024) void k_node_tile(mxh_level lv, mxh_bloch bl, 
   }
 }
 
+// ----------------------------------------------------------------- whole grids in LDS
+// Grids of at most 64 x 64 (one thread per 2 x 2 node block) are smoothed with
+// the whole periodic vector in LDS: no halo is loaded or computed (the square
+// tiles redo a 64^2 FP64 grid five times over), a colour phase is one patch per
+// thread.  Columns are split by parity, so a phase reads consecutive addresses
+// across a wavefront; the Bloch phase is applied where a block's neighbour lies
+// across the boundary.  What bounds it: vector issue of the patch solves at 64^2,
+// the latency of the phases on smaller grids.  192 vectors of 64^2 in FP64, two
+// sweeps and prolongation: 58.6 -> 34.9 us (square tiles before).
+template <typename T>
+struct GridBlock {
+  int hx, hy, I, J;       // blocks per side, this thread's block
+  int co[4], go[4];       // columns 2I - 1 .. 2I + 2: LDS offset, natural index
+  int ro[4];              // rows 2J - 1 .. 2J + 2, times nx
+  C<T> xf, yf;
+
+  MXH_DEV void set(int nx, int ny, int block)
+  {
+    hx = nx >> 1;
+    hy = ny >> 1;
+    J = block / hx;
+    I = block - J * hx;
+    const int l = I ? I - 1 : hx - 1, r = I + 1 < hx ? I + 1 : 0;
+    co[0] = hx + l;
+    co[1] = I;
+    co[2] = hx + I;
+    co[3] = r;
+    go[0] = 2 * l + 1;
+    go[1] = 2 * I;
+    go[2] = 2 * I + 1;
+    go[3] = 2 * r;
+    ro[0] = (J ? 2 * J - 1 : ny - 1) * nx;
+    ro[1] = 2 * J * nx;
+    ro[2] = (2 * J + 1) * nx;
+    ro[3] = (J + 1 < hy ? 2 * J + 2 : 0) * nx;
+  }
+  // value at node (2I + DI, 2J + DJ) of an array in LDS (parity-split columns)
+  // or, GL, in memory
+  template <int DI, int DJ, bool GL = false>
+  MXH_DEV C<T> get(const C<T>* s) const
+  {
+    C<T> v = s[(GL ? go[DI + 1] : co[DI + 1]) + ro[DJ + 1]];
+    if (DI == -1 && I == 0) v = cconj(xf) * v;
+    if (DI == 2 && I == hx - 1) v = xf * v;
+    if (DJ == -1 && J == 0) v = cconj(yf) * v;
+    if (DJ == 2 && J == hy - 1) v = yf * v;
+    return v;
+  }
+  // the stored value of node (2I + DI, 2J + DJ), which get() returned as v,
+  // plus d (v + d itself where no phase lies between)
+  template <int DI, int DJ>
+  MXH_DEV void put(C<T>* s, C<T> v, C<T> d) const
+  {
+    C<T>* p = s + co[DI + 1] + ro[DJ + 1];
+    const bool wx = DI == -1 && I == 0, wy = DJ == -1 && J == 0;
+    if (wx) d = xf * d;
+    if (wy) d = yf * d;
+    *p = wx || wy ? *p + d : v + d;
+  }
+};
+
+// 1 / (hx hy eps) of the cells (2I - 1 .. 2I + 1) x (2J - 1 .. 2J + 1)
+template <typename T>
+MXH_DEV void grid_eta(const GridBlock<T>& g, const T* eta, T axy, T er[3][3])
+{
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int b = 0; b < 3; b++) er[a][b] = axy * eta[g.go[a] + g.ro[b]];
+}
+
+// The AFW patch of node (2I + CI, 2J + CJ); b in LDS or, BG, in memory.
+template <int CI, int CJ, bool BG, bool RELOAD, typename T>
+MXH_DEV void grid_patch(const GridBlock<T>& g, C<T>* sx, C<T>* sy, const C<T>* bx, const C<T>* by,
+                        const T er[3][3], T mx, T my)
+{
+  const C<T> b0 = g.template get<CI - 1, CJ, BG>(bx), b1 = g.template get<CI, CJ, BG>(bx);
+  const C<T> b2 = g.template get<CI, CJ - 1, BG>(by), b3 = g.template get<CI, CJ, BG>(by);
+  const C<T> xLm = g.template get<CI - 1, CJ - 1>(sx), xL0 = g.template get<CI - 1, CJ>(sx);
+  const C<T> xLp = g.template get<CI - 1, CJ + 1>(sx), xRm = g.template get<CI, CJ - 1>(sx);
+  const C<T> xR0 = g.template get<CI, CJ>(sx), xRp = g.template get<CI, CJ + 1>(sx);
+  const C<T> yLm = g.template get<CI - 1, CJ - 1>(sy), yCm = g.template get<CI, CJ - 1>(sy);
+  const C<T> yRm = g.template get<CI + 1, CJ - 1>(sy), yL0 = g.template get<CI - 1, CJ>(sy);
+  const C<T> yC0 = g.template get<CI, CJ>(sy), yR0 = g.template get<CI + 1, CJ>(sy);
+  T eLL = er[CI][CJ], eRL = er[CI + 1][CJ], eLU = er[CI][CJ + 1], eRU = er[CI + 1][CJ + 1];
+  if (RELOAD) asm volatile("" : "+v"(eLL), "+v"(eRL), "+v"(eLU), "+v"(eRU));
+  const C<T> qLL = eLL * (xLm - xL0 - yLm + yCm), qRL = eRL * (xRm - xR0 - yCm + yRm);
+  const C<T> qLU = eLU * (xL0 - xLp - yL0 + yC0), qRU = eRU * (xR0 - xRp - yC0 + yR0);
+  const C<T> r0 = b0 - (qLU - qLL) - mx * (T(4) * xL0 + xLm + xLp);
+  const C<T> r1 = b1 - (qRU - qRL) - mx * (T(4) * xR0 + xRm + xRp);
+  const C<T> r2 = b2 - (qLL - qRL) - my * (T(4) * yCm + yLm + yRm);
+  const C<T> r3 = b3 - (qLU - qRU) - my * (T(4) * yC0 + yL0 + yR0);
+  C<T> z0, z1, z2, z3;
+  afw_local_solve(eLL, eRL, eLU, eRU, mx, my, r0, r1, r2, r3, z0, z1, z2, z3);
+  g.template put<CI - 1, CJ>(sx, xL0, z0);
+  g.template put<CI, CJ>(sx, xR0, z1);
+  g.template put<CI, CJ - 1>(sy, yCm, z2);
+  g.template put<CI, CJ>(sy, yC0, z3);
+}
+
+// keeps the compiler from lifting the loads through p out of the sweep loop
+// (and, on eta, the coefficients of the local solves)
+template <bool RELOAD, typename T>
+MXH_DEV const T* reload(const T* p)
+{
+  if (RELOAD) asm volatile("" : "+s"(p));
+  return p;
+}
+
+// One four-colour sweep (all threads of the workgroup; act: the thread owns a
+// block).  Up to 256 threads a block's b and the coefficients of its local solves
+// stay in registers over the sweeps; RELOAD: 1024 threads leave no room, b is
+// read and the coefficients are formed again per patch.
+template <bool BWD, bool BG, bool RELOAD = false, int NB = 1, typename T>
+MXH_DEV void grid_sweep(const GridBlock<T> (&g)[NB], const bool (&act)[NB], C<T>* sx, C<T>* sy, const C<T>* bx,
+                        const C<T>* by, const T (&er)[NB][3][3], T mx, T my)
+{
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+#pragma unroll
+    for (int q = 0; q < NB; q++)
+      if (act[q]) {
+        const C<T>*px = reload<RELOAD>(bx), *py = reload<RELOAD>(by);
+        switch (BWD ? 3 - k : k) {
+        case 0: grid_patch<0, 0, BG, RELOAD>(g[q], sx, sy, px, py, er[q], mx, my); break;
+        case 1: grid_patch<1, 0, BG, RELOAD>(g[q], sx, sy, px, py, er[q], mx, my); break;
+        case 2: grid_patch<0, 1, BG, RELOAD>(g[q], sx, sy, px, py, er[q], mx, my); break;
+        case 3: grid_patch<1, 1, BG, RELOAD>(g[q], sx, sy, px, py, er[q], mx, my); break;
+        }
+      }
+    __syncthreads();
+  }
+}
+
+// The residual of the block's nodes, restricted to its coarse node (cx, cy):
+// the block's own part, then (after a barrier) what its neighbours below and
+// to the left lend it, one sum each (px, py, one value per block in LDS).
+template <bool BG, typename T>
+MXH_DEV void grid_restrict_own(const GridBlock<T>& g, bool act, const C<T>* sx, const C<T>* sy, const C<T>* bx,
+                           const C<T>* by, const T er[3][3], T mx, T my, C<T>* px, C<T>* py, C<T>& cx, C<T>& cy)
+{
+  const int k = g.I + g.J * g.hx;
+  if (act) {
+    // x(2I - 1 .. 2I + 1, 2J - 1 .. 2J + 2), y(2I - 1 .. 2I + 2, 2J - 1 .. 2J + 1)
+    const C<T> x00 = g.template get<-1, 0>(sx), x01 = g.template get<-1, 1>(sx), x02 = g.template get<-1, 2>(sx);
+    C<T> X[2][4], Y[4][2];
+    X[0][0] = g.template get<0, -1>(sx);
+    X[0][1] = g.template get<0, 0>(sx);
+    X[0][2] = g.template get<0, 1>(sx);
+    X[0][3] = g.template get<0, 2>(sx);
+    X[1][0] = g.template get<1, -1>(sx);
+    X[1][1] = g.template get<1, 0>(sx);
+    X[1][2] = g.template get<1, 1>(sx);
+    X[1][3] = g.template get<1, 2>(sx);
+    Y[0][0] = g.template get<-1, 0>(sy);
+    Y[0][1] = g.template get<-1, 1>(sy);
+    Y[1][0] = g.template get<0, 0>(sy);
+    Y[1][1] = g.template get<0, 1>(sy);
+    Y[2][0] = g.template get<1, 0>(sy);
+    Y[2][1] = g.template get<1, 1>(sy);
+    Y[3][0] = g.template get<2, 0>(sy);
+    Y[3][1] = g.template get<2, 1>(sy);
+    const C<T> ym0 = g.template get<0, -1>(sy), ym1 = g.template get<1, -1>(sy), ym2 = g.template get<2, -1>(sy);
+    // eta times the curl of the cells (0, 1) x (-1, 0, 1), and of (-1) x (0, 1)
+    C<T> q[2][3];
+    q[0][0] = er[1][0] * (X[0][0] - X[0][1] - ym0 + ym1);
+    q[1][0] = er[2][0] * (X[1][0] - X[1][1] - ym1 + ym2);
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int b = 0; b < 2; b++) q[a][b + 1] = er[a + 1][b + 1] * (X[a][b + 1] - X[a][b + 2] - Y[a + 1][b] + Y[a + 2][b]);
+    const C<T> l0 = er[0][1] * (x00 - x01 - Y[0][0] + Y[1][0]), l1 = er[0][2] * (x01 - x02 - Y[0][1] + Y[1][1]);
+    C<T> rx[2][2], ry[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int b = 0; b < 2; b++) {
+        rx[a][b] = cmk(T(0), T(0)) - (q[a][b + 1] - q[a][b]) - mx * (T(4) * X[a][b + 1] + X[a][b] + X[a][b + 2]);
+        ry[a][b] = cmk(T(0), T(0)) - ((a ? q[0][b + 1] : (b ? l1 : l0)) - q[a][b + 1]) -
+                   my * (T(4) * Y[a + 1][b] + Y[a][b] + Y[a + 2][b]);
+      }
+    rx[0][0] += g.template get<0, 0, BG>(bx);
+    rx[1][0] += g.template get<1, 0, BG>(bx);
+    rx[0][1] += g.template get<0, 1, BG>(bx);
+    rx[1][1] += g.template get<1, 1, BG>(bx);
+    ry[0][0] += g.template get<0, 0, BG>(by);
+    ry[1][0] += g.template get<1, 0, BG>(by);
+    ry[0][1] += g.template get<0, 1, BG>(by);
+    ry[1][1] += g.template get<1, 1, BG>(by);
+    px[k] = rx[0][1] + rx[1][1];
+    py[k] = ry[1][0] + ry[1][1];
+    cx = T(0.5) * (rx[0][0] + rx[1][0]) + T(0.25) * px[k];
+    cy = T(0.5) * (ry[0][0] + ry[0][1]) + T(0.25) * py[k];
+  }
+}
+template <typename T>
+MXH_DEV void grid_restrict_lent(const GridBlock<T>& g, bool act, const C<T>* px, const C<T>* py, C<T>& cx, C<T>& cy)
+{
+  const int k = g.I + g.J * g.hx;
+  if (act) {
+    C<T> d = px[g.J ? k - g.hx : k + (g.hy - 1) * g.hx], l = py[g.I ? k - 1 : k + g.hx - 1];
+    if (g.J == 0) d = cconj(g.yf) * d;
+    if (g.I == 0) l = cconj(g.xf) * l;
+    cx += T(0.25) * d;
+    cy += T(0.25) * l;
+  }
+}
+
+// x += P xc for the block's nodes: c0, c1 = cx(I, J), cx(I, J + 1), d0, d1 =
+// cy(I, J), cy(I + 1, J), the upper and right one with their Bloch factors
+template <typename T>
+MXH_DEV void grid_prolong(const GridBlock<T>& g, C<T>* sx, C<T>* sy, C<T> c0, C<T> c1, C<T> d0, C<T> d1)
+{
+  if (g.J == g.hy - 1) c1 = g.yf * c1;
+  if (g.I == g.hx - 1) d1 = g.xf * d1;
+  const C<T> h = T(0.5) * c0, q = T(0.25) * (c0 + c1), u = T(0.5) * d0, w = T(0.25) * (d0 + d1);
+  sx[g.co[1] + g.ro[1]] += h;
+  sx[g.co[2] + g.ro[1]] += h;
+  sx[g.co[1] + g.ro[2]] += q;
+  sx[g.co[2] + g.ro[2]] += q;
+  sy[g.co[1] + g.ro[1]] += u;
+  sy[g.co[1] + g.ro[2]] += u;
+  sy[g.co[2] + g.ro[1]] += w;
+  sy[g.co[2] + g.ro[2]] += w;
+}
+
+// block's nodes between LDS and memory
+template <typename T>
+MXH_DEV void grid_copy_in(const GridBlock<T>& g, C<T>* s, const C<T>* a)
+{
+#pragma unroll
+  for (int b = 1; b < 3; b++)
+#pragma unroll
+    for (int c = 1; c < 3; c++) s[g.co[c] + g.ro[b]] = a ? a[g.go[c] + g.ro[b]] : czero<T>();
+}
+template <typename T>
+MXH_DEV void grid_copy_out(const GridBlock<T>& g, const C<T>* s, C<T>* a)
+{
+#pragma unroll
+  for (int b = 1; b < 3; b++)
+#pragma unroll
+    for (int c = 1; c < 3; c++) a[g.go[c] + g.ro[b]] = s[g.co[c] + g.ro[b]];
+}
+
+template <typename T> struct GridCfg;
+template <> struct GridCfg<float> { static constexpr int TB = 1024, NB = 1; };
+template <> struct GridCfg<double> { static constexpr int TB = 512, NB = 2; };
+
+// The passes of k_afw_tile (same modes) on a grid that fits; NB blocks per
+// thread (64^2 in FP64: two of 512 threads', in the 256 registers a patch's
+// values and coefficients want).
+template <typename T, int MODE, int TB, int NB>
+__global__ __launch_bounds__(TB) void k_afw_grid(mxh_level lv, mxh_bloch bl, const C<T>* B, long long bs,
+                                                 const C<T>* Xin, C<T>* Xout, long long xs, const T* eta, int nsweep,
+                                                 const C<T>* XCin, C<T>* BC, C<T>* XC, long long cs)
+{
+  extern __shared__ double smem[];
+  const int v = blockIdx.x, nx = lv.nx, ny = lv.ny, N = nx * ny, NC = N >> 2;
+  C<T>*sx = (C<T>*)smem, *sy = sx + N, *px = sy + N, *py = px + NC;  // px, py: MODE 8
+  const Geo<T> geo = make_geo<T>(lv, bl, v);
+  const C<T>*bx = B + (size_t)v * bs, *by = bx + N;
+  const T mx = T(lv.hy / lv.hx / 6.0), my = T(lv.hx / lv.hy / 6.0);
+  GridBlock<T> g[NB];
+  bool act[NB];
+  int kc[NB];
+  T er[NB][3][3];
+#pragma unroll
+  for (int q = 0; q < NB; q++) {
+    const int k = (int)threadIdx.x + q * TB;
+    act[q] = k < NC;
+    g[q].xf = geo.xf;
+    g[q].yf = geo.yf;
+    g[q].set(nx, ny, act[q] ? k : 0);
+    kc[q] = g[q].I + g[q].J * g[q].hx;
+    grid_eta(g[q], eta, T(1.0 / (lv.hx * lv.hy)), er[q]);
+    if (act[q]) {
+      const C<T>* x = (MODE & 2) ? nullptr : Xin + (size_t)v * xs;
+      grid_copy_in(g[q], sx, x);
+      grid_copy_in(g[q], sy, x ? x + N : nullptr);
+      if (MODE & 4) {
+        const C<T>*cx = XCin + (size_t)v * cs, *cy = cx + NC;
+        grid_prolong(g[q], sx, sy, cx[kc[q]], cx[g[q].J + 1 < g[q].hy ? kc[q] + g[q].hx : g[q].I], cy[kc[q]],
+                     cy[g[q].I + 1 < g[q].hx ? kc[q] + 1 : g[q].J * g[q].hx]);
+      }
+    }
+  }
+  __syncthreads();
+  for (int s = 0; s < nsweep; s++)
+    grid_sweep<(MODE & 1) != 0, true, (TB > 256), NB>(g, act, sx, sy, bx, by, er, mx, my);
+#pragma unroll
+  for (int q = 0; q < NB; q++)
+    if (act[q]) {
+      C<T>* x = Xout + (size_t)v * xs;
+      grid_copy_out(g[q], sx, x);
+      grid_copy_out(g[q], sy, x + N);
+    }
+  if (MODE & 8) {
+    C<T> cx[NB], cy[NB];
+#pragma unroll
+    for (int q = 0; q < NB; q++)
+      grid_restrict_own<true>(g[q], act[q], sx, sy, bx, by, er[q], mx, my, px, py, cx[q], cy[q]);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NB; q++) {
+      grid_restrict_lent(g[q], act[q], px, py, cx[q], cy[q]);
+      if (act[q]) {
+        C<T>*bc = BC + (size_t)v * cs, *xc = XC + (size_t)v * cs;
+        bc[kc[q]] = cx[q];
+        bc[NC + kc[q]] = cy[q];
+        xc[kc[q]] = czero<T>();
+        xc[NC + kc[q]] = czero<T>();
+      }
+    }
+  }
+}
+
+// ---- the coarse end of a V-cycle in one launch: levels of at most 32 x 32.
+// One workgroup per vector keeps x of every level, b of the lower ones and the
+// lent sums in LDS; the coarsest level is a product with the inverse of its
+// matrix.  It replaces two launches a level and the triangular solves, all
+// latency-bound at any batch size, as it is: 192 vectors from 32^2 to 4^2 in FP64
+// 51 us against 160, 640 in FP32 85 us against 330 (phases of one wave on 16^2 and
+// 8^2, and the barriers between them).
+#define CYCLE_MAXL 6
+struct CycleLevels {
+  int n;  // levels 0 .. n - 1
+  int nx[CYCLE_MAXL], ny[CYCLE_MAXL];
+  double hx[CYCLE_MAXL], hy[CYCLE_MAXL];
+  const void* eta[CYCLE_MAXL];  // edge cycles
+  void *b[CYCLE_MAXL], *x[CYCLE_MAXL];  // where the lower levels' vectors go (null: nowhere)
+};
+
+// out = W-product of the coarsest level: x_r = sum_c conj(W[c n + r]) b_c over
+// nc = n components laid out as `comp` arrays of nx x ny (parity-split in LDS)
+template <typename T>
+MXH_DEV void cycle_coarse(int n, int nx, int N, const C<double>* W, const C<T>* b, C<T>* x, double* red)
+{
+  const int tid = threadIdx.x, grp = max(1, (int)blockDim.x / n);
+  auto at = [&](int k) {
+    const int c = k / N, q = k - c * N, j = q / nx, i = q - j * nx;
+    return c * N + j * nx + (i & 1) * (nx >> 1) + (i >> 1);
+  };
+  C<double>* part = (C<double>*)red;
+  for (int w = tid; w < grp * n; w += blockDim.x) {
+    const int r = w % n, q = w / n;
+    C<double> s = czero<double>();
+    for (int c = q; c < n; c += grp) s += cconj(W[(size_t)c * n + r]) * ccast<double>(b[at(c)]);
+    part[w] = s;
+  }
+  __syncthreads();
+  for (int r = tid; r < n; r += blockDim.x) {
+    C<double> s = part[r];
+    for (int q = 1; q < grp; q++) s += part[q * n + r];
+    x[at(r)] = ccast<T>(s);
+  }
+  __syncthreads();
+}
+
+template <typename T>
+__global__ __launch_bounds__(256, 2) void k_edge_cycle(CycleLevels cl, mxh_bloch bl, int nu, const C<T>* B, long long bs,
+                                                    const int* bmap, C<T>* X, long long xs, int xzero, const double* W0,
+                                                    int wper)
+{
+  extern __shared__ double smem[];
+  const int v = blockIdx.x, top = cl.n - 1, tid = threadIdx.x;
+  mxh_level lv;
+  lv.nx = cl.nx[top];
+  lv.ny = cl.ny[top];
+  const Geo<T> geo = make_geo<T>(lv, bl, v);
+  const int gv = bl.vmap ? bl.vmap[v] : v;
+  GridBlock<T> gb[1];
+  GridBlock<T>& g = gb[0];
+  g.xf = geo.xf;
+  g.yf = geo.yf;
+  const int NT = lv.nx * lv.ny, n0 = 2 * cl.nx[0] * cl.ny[0];
+  const C<double>* W = (const C<double>*)W0 + (wper ? (size_t)(gv / bl.vpp) * n0 * n0 : 0);
+  // LDS: x of levels top .. 0, b of levels top - 1 .. 0, lent sums, coarse partial sums
+  C<T>* xl = (C<T>*)smem;
+  int xtot = 0;
+  for (int l = 0; l <= top; l++) xtot += 2 * cl.nx[l] * cl.ny[l];
+  C<T>* bl_ = xl + xtot;                 // b of level top - 1 first
+  C<T>* px = bl_ + (xtot - 2 * NT);
+  C<T>* py = px + (NT >> 2);
+  double* red = (double*)(px + (top ? NT >> 1 : 2 * NT));
+  const C<T>*gbx = B + (size_t)(bmap ? bmap[v] : v) * bs, *gby = gbx + NT;
+  C<T>* xout = X + (size_t)v * xs;
+
+  C<T>*x = xl, *b = bl_ - 2 * NT;  // of the current level (b: lower levels)
+  for (int l = top; l > 0; l--) {
+    const int nx = cl.nx[l], ny = cl.ny[l], N = nx * ny;
+    const bool acts[1] = {tid < (N >> 2)}, act = acts[0];
+    g.set(nx, ny, act ? tid : 0);
+    const T axy = T(1.0 / (cl.hx[l] * cl.hy[l]));
+    const T mx = T(cl.hy[l] / cl.hx[l] / 6.0), my = T(cl.hx[l] / cl.hy[l] / 6.0);
+    T er[1][3][3];
+    grid_eta(g, (const T*)cl.eta[l], axy, er[0]);
+    if (act) {
+      const C<T>* src = l == top && !xzero ? xout : nullptr;
+      grid_copy_in(g, x, src);
+      grid_copy_in(g, x + N, src ? src + N : nullptr);
+    }
+    __syncthreads();
+    C<T> cx, cy;
+    if (l == top) {
+      for (int s = 0; s < nu; s++) grid_sweep<false, true>(gb, acts, x, x + N, gbx, gby, er, mx, my);
+      grid_restrict_own<true>(g, act, x, x + N, gbx, gby, er[0], mx, my, px, py, cx, cy);
+    } else {
+      for (int s = 0; s < nu; s++) grid_sweep<false, false>(gb, acts, x, x + N, b, b + N, er, mx, my);
+      grid_restrict_own<false>(g, act, x, x + N, b, b + N, er[0], mx, my, px, py, cx, cy);
+    }
+    __syncthreads();
+    grid_restrict_lent(g, act, px, py, cx, cy);
+    x += 2 * N;
+    b += 2 * N;
+    if (act) {
+      const int NC = N >> 2, k = g.J * g.hx + (g.I & 1) * (g.hx >> 1) + (g.I >> 1);
+      b[k] = cx;
+      b[NC + k] = cy;
+    }
+    __syncthreads();
+  }
+  const int nx0 = cl.nx[0], N0 = nx0 * cl.ny[0];
+  if (top == 0) {  // the coarsest level alone
+    for (int k = tid; k < 2 * N0; k += blockDim.x) {
+      const int c = k / N0, q = k - c * N0, j = q / nx0, i = q - j * nx0;
+      px[c * N0 + j * nx0 + (i & 1) * (nx0 >> 1) + (i >> 1)] = gbx[k];
+    }
+    __syncthreads();
+    b = px;
+  }
+  cycle_coarse(n0, nx0, N0, W, b, x, red);
+  for (int l = 1; l <= top; l++) {
+    const int nx = cl.nx[l], ny = cl.ny[l], N = nx * ny, NC = N >> 2;
+    const bool acts[1] = {tid < NC}, act = acts[0];
+    g.set(nx, ny, act ? tid : 0);
+    const C<T>* xc = x;
+    x -= 2 * N;
+    b -= 2 * N;
+    const T axy = T(1.0 / (cl.hx[l] * cl.hy[l]));
+    const T mx = T(cl.hy[l] / cl.hx[l] / 6.0), my = T(cl.hx[l] / cl.hy[l] / 6.0);
+    T er[1][3][3];
+    grid_eta(g, (const T*)cl.eta[l], axy, er[0]);
+    if (act) {
+      // the coarse vector's columns are split by parity too
+      auto at = [&](int I, int J) { return J * g.hx + (I & 1) * (g.hx >> 1) + (I >> 1); };
+      const int Jp = g.J + 1 < g.hy ? g.J + 1 : 0, Ip = g.I + 1 < g.hx ? g.I + 1 : 0;
+      grid_prolong(g, x, x + N, xc[at(g.I, g.J)], xc[at(g.I, Jp)], xc[NC + at(g.I, g.J)], xc[NC + at(Ip, g.J)]);
+    }
+    __syncthreads();
+    if (l == top)
+      for (int s = 0; s < nu; s++) grid_sweep<true, true>(gb, acts, x, x + N, gbx, gby, er, mx, my);
+    else
+      for (int s = 0; s < nu; s++) grid_sweep<true, false>(gb, acts, x, x + N, b, b + N, er, mx, my);
+  }
+  // out: the top level's x, and the lower levels where asked
+  if (top > 0) {
+    const bool act = tid < (NT >> 2);
+    g.set(lv.nx, lv.ny, act ? tid : 0);
+    if (act) {
+      grid_copy_out(g, xl, xout);
+      grid_copy_out(g, xl + NT, xout + NT);
+    }
+  } else {
+    for (int k = tid; k < 2 * N0; k += blockDim.x) {
+      const int c = k / N0, q = k - c * N0, j = q / nx0, i = q - j * nx0;
+      xout[k] = x[c * N0 + j * nx0 + (i & 1) * (nx0 >> 1) + (i >> 1)];
+    }
+  }
+  C<T>*xk = xl + 2 * NT, *bk = bl_;
+  for (int l = top - 1; l >= 0; l--) {
+    const int nx = cl.nx[l], N = nx * cl.ny[l];
+    C<T>*xo = (C<T>*)cl.x[l], *bo = (C<T>*)cl.b[l];
+    if (xo)
+      for (int k = tid; k < 2 * N; k += blockDim.x) {
+        const int c = k / N, q = k - c * N, j = q / nx, i = q - j * nx;
+        const int s = c * N + j * nx + (i & 1) * (nx >> 1) + (i >> 1);
+        xo[k] = xk[s];
+        bo[k] = bk[s];
+      }
+    xk += 2 * N;
+    bk += 2 * N;
+  }
+}
+
+// W[r n + c] = (A^-1)[r, c] from the Cholesky factor L of A (n x n,
+// column-major, per problem): one workgroup per problem, one thread per column
+// c, forward and back substitution.  work: W itself holds the running column.
+__global__ __launch_bounds__(256) void k_coarse_inverse(int n, const double* L0, double* W0)
+{
+  const C<double>* L = (const C<double>*)L0 + (size_t)blockIdx.x * n * n;
+  C<double>* W = (C<double>*)W0 + (size_t)blockIdx.x * n * n;
+  const int c = threadIdx.x;
+  if (c >= n) return;
+  for (int r = 0; r < n; r++) {
+    C<double> t = cmk(r == c ? 1.0 : 0.0, 0.0);
+    for (int k = c; k < r; k++) t -= L[r + (size_t)k * n] * W[(size_t)k * n + c];
+    const double d = L[r + (size_t)r * n].r;
+    W[(size_t)r * n + c] = cmk(t.r / d, t.i / d);
+  }
+  for (int r = n - 1; r >= 0; r--) {
+    C<double> t = W[(size_t)r * n + c];
+    for (int k = r + 1; k < n; k++) t -= cconj(L[k + (size_t)r * n]) * W[(size_t)k * n + c];
+    const double d = L[r + (size_t)r * n].r;
+    W[(size_t)r * n + c] = cmk(t.r / d, t.i / d);
+  }
+}
+
+// ---- the nodal counterpart: Gauss-Seidel for the Q1 Laplacian
+template <int CI, int CJ, typename T>
+MXH_DEV C<T> grid_node_off(const GridBlock<T>& g, const C<T>* s, const NodeCoef<T>& nc)
+{
+  return nc.ax * (g.template get<CI - 1, CJ>(s) + g.template get<CI + 1, CJ>(s)) +
+         nc.ay * (g.template get<CI, CJ - 1>(s) + g.template get<CI, CJ + 1>(s)) +
+         nc.ad * (g.template get<CI - 1, CJ - 1>(s) + g.template get<CI + 1, CJ - 1>(s) +
+                  g.template get<CI - 1, CJ + 1>(s) + g.template get<CI + 1, CJ + 1>(s));
+}
+template <int CI, int CJ, bool BG, typename T>
+MXH_DEV void grid_node_update(const GridBlock<T>& g, bool act, C<T>* s, const C<T>* b, const NodeCoef<T>& nc, T iac)
+{
+  if (act) s[g.co[CI + 1] + g.ro[CJ + 1]] = iac * (g.template get<CI, CJ, BG>(b) - grid_node_off<CI, CJ>(g, s, nc));
+  __syncthreads();
+}
+template <bool BWD, bool BG, typename T>
+MXH_DEV void grid_node_sweep(const GridBlock<T>& g, bool act, C<T>* s, const C<T>* b, const NodeCoef<T>& nc, T iac)
+{
+  if (BWD) {
+    grid_node_update<1, 1, BG>(g, act, s, b, nc, iac);
+    grid_node_update<0, 1, BG>(g, act, s, b, nc, iac);
+    grid_node_update<1, 0, BG>(g, act, s, b, nc, iac);
+    grid_node_update<0, 0, BG>(g, act, s, b, nc, iac);
+  } else {
+    grid_node_update<0, 0, BG>(g, act, s, b, nc, iac);
+    grid_node_update<1, 0, BG>(g, act, s, b, nc, iac);
+    grid_node_update<0, 1, BG>(g, act, s, b, nc, iac);
+    grid_node_update<1, 1, BG>(g, act, s, b, nc, iac);
+  }
+}
+// the residual restricted to the block's coarse node; p: three lent values per block
+template <bool BG, typename T>
+MXH_DEV C<T> grid_node_restrict(const GridBlock<T>& g, bool act, const C<T>* s, const C<T>* b, const NodeCoef<T>& nc,
+                                C<T>* p)
+{
+  const int NC = g.hx * g.hy, k = g.I + g.J * g.hx;
+  C<T> acc = czero<T>();
+  if (act) {
+    const C<T> r00 = g.template get<0, 0, BG>(b) - nc.ac * g.template get<0, 0>(s) - grid_node_off<0, 0>(g, s, nc);
+    const C<T> r10 = g.template get<1, 0, BG>(b) - nc.ac * g.template get<1, 0>(s) - grid_node_off<1, 0>(g, s, nc);
+    const C<T> r01 = g.template get<0, 1, BG>(b) - nc.ac * g.template get<0, 1>(s) - grid_node_off<0, 1>(g, s, nc);
+    const C<T> r11 = g.template get<1, 1, BG>(b) - nc.ac * g.template get<1, 1>(s) - grid_node_off<1, 1>(g, s, nc);
+    p[k] = r10;
+    p[NC + k] = r01;
+    p[2 * NC + k] = r11;
+    acc = r00 + T(0.5) * (r10 + r01) + T(0.25) * r11;
+  }
+  __syncthreads();
+  if (act) {
+    const int kl = g.I ? k - 1 : k + g.hx - 1, kd = g.J ? k - g.hx : k + (g.hy - 1) * g.hx;
+    const int kld = g.J ? kl - g.hx : kl + (g.hy - 1) * g.hx;
+    C<T> l = T(0.5) * p[kl] + T(0.25) * p[2 * NC + kl], d = T(0.5) * p[NC + kd] + T(0.25) * p[2 * NC + kd];
+    C<T> ld = T(0.25) * p[2 * NC + kld];
+    if (g.I == 0) {
+      l = cconj(g.xf) * l;
+      ld = cconj(g.xf) * ld;
+    }
+    if (g.J == 0) {
+      d = cconj(g.yf) * d;
+      ld = cconj(g.yf) * ld;
+    }
+    acc += l + d + ld;
+  }
+  return acc;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_node_cycle(CycleLevels cl, mxh_bloch bl, int nu, const C<T>* B, long long bs,
+                                                    C<T>* X, long long xs, int xzero, const double* W0, int wper)
+{
+  extern __shared__ double smem[];
+  const int v = blockIdx.x, top = cl.n - 1, tid = threadIdx.x;
+  mxh_level lv;
+  lv.nx = cl.nx[top];
+  lv.ny = cl.ny[top];
+  const Geo<T> geo = make_geo<T>(lv, bl, v);
+  const int gv = bl.vmap ? bl.vmap[v] : v;
+  GridBlock<T> g;
+  g.xf = geo.xf;
+  g.yf = geo.yf;
+  const int NT = lv.nx * lv.ny, n0 = cl.nx[0] * cl.ny[0];
+  const C<double>* W = (const C<double>*)W0 + (wper ? (size_t)(gv / bl.vpp) * n0 * n0 : 0);
+  C<T>* xl = (C<T>*)smem;
+  int xtot = 0;
+  for (int l = 0; l <= top; l++) xtot += cl.nx[l] * cl.ny[l];
+  C<T>*bl_ = xl + xtot, *p = bl_ + (xtot - NT);
+  double* red = (double*)(p + NT);
+  const C<T>* gb = B + (size_t)v * bs;
+  C<T>* xout = X + (size_t)v * xs;
+  auto coef = [&](int l) {
+    mxh_level q;
+    q.hx = cl.hx[l];
+    q.hy = cl.hy[l];
+    return node_coef<T>(q, 1.0);
+  };
+  C<T>*x = xl, *b = bl_ - NT;
+  for (int l = top; l > 0; l--) {
+    const int nx = cl.nx[l], ny = cl.ny[l], N = nx * ny;
+    const bool act = tid < (N >> 2);
+    g.set(nx, ny, act ? tid : 0);
+    const NodeCoef<T> nc = coef(l);
+    const T iac = T(1) / nc.ac;
+    if (act) grid_copy_in(g, x, l == top && !xzero ? (const C<T>*)xout : nullptr);
+    __syncthreads();
+    C<T> c;
+    if (l == top) {
+      for (int s = 0; s < nu; s++) grid_node_sweep<false, true>(g, act, x, gb, nc, iac);
+      c = grid_node_restrict<true>(g, act, x, gb, nc, p);
+    } else {
+      for (int s = 0; s < nu; s++) grid_node_sweep<false, false>(g, act, x, b, nc, iac);
+      c = grid_node_restrict<false>(g, act, x, b, nc, p);
+    }
+    x += N;
+    b += N;
+    if (act) b[g.J * g.hx + (g.I & 1) * (g.hx >> 1) + (g.I >> 1)] = c;
+    __syncthreads();
+  }
+  const int nx0 = cl.nx[0];
+  auto split = [&](int k) {
+    const int j = k / nx0, i = k - j * nx0;
+    return j * nx0 + (i & 1) * (nx0 >> 1) + (i >> 1);
+  };
+  if (top == 0) {
+    for (int k = tid; k < n0; k += blockDim.x) p[split(k)] = gb[k];
+    __syncthreads();
+    b = p;
+  }
+  cycle_coarse(n0, nx0, n0, W, b, x, red);
+  for (int l = 1; l <= top; l++) {
+    const int nx = cl.nx[l], ny = cl.ny[l], N = nx * ny;
+    const bool act = tid < (N >> 2);
+    g.set(nx, ny, act ? tid : 0);
+    const C<T>* xc = x;
+    x -= N;
+    b -= N;
+    const NodeCoef<T> nc = coef(l);
+    const T iac = T(1) / nc.ac;
+    if (act) {
+      auto at = [&](int I, int J) { return J * g.hx + (I & 1) * (g.hx >> 1) + (I >> 1); };
+      const int Jp = g.J + 1 < g.hy ? g.J + 1 : 0, Ip = g.I + 1 < g.hx ? g.I + 1 : 0;
+      const C<T> c00 = xc[at(g.I, g.J)];
+      C<T> c10 = xc[at(Ip, g.J)], c01 = xc[at(g.I, Jp)], c11 = xc[at(Ip, Jp)];
+      if (Ip == 0) {
+        c10 = g.xf * c10;
+        c11 = g.xf * c11;
+      }
+      if (Jp == 0) {
+        c01 = g.yf * c01;
+        c11 = g.yf * c11;
+      }
+      x[g.co[1] + g.ro[1]] += c00;
+      x[g.co[2] + g.ro[1]] += T(0.5) * (c00 + c10);
+      x[g.co[1] + g.ro[2]] += T(0.5) * (c00 + c01);
+      x[g.co[2] + g.ro[2]] += T(0.25) * (c00 + c10 + c01 + c11);
+    }
+    __syncthreads();
+    if (l == top)
+      for (int s = 0; s < nu; s++) grid_node_sweep<true, true>(g, act, x, gb, nc, iac);
+    else
+      for (int s = 0; s < nu; s++) grid_node_sweep<true, false>(g, act, x, b, nc, iac);
+  }
+  if (top > 0) {
+    const bool act = tid < (NT >> 2);
+    g.set(lv.nx, lv.ny, act ? tid : 0);
+    if (act) grid_copy_out(g, xl, xout);
+  } else {
+    for (int k = tid; k < n0; k += blockDim.x) xout[k] = x[split(k)];
+  }
+  C<T>*xk = xl + NT, *bk = bl_;
+  for (int l = top - 1; l >= 0; l--) {
+    const int nx = cl.nx[l], N = nx * cl.ny[l];
+    C<T>*xo = (C<T>*)cl.x[l], *bo = (C<T>*)cl.b[l];
+    if (xo)
+      for (int k = tid; k < N; k += blockDim.x) {
+        const int j = k / nx, i = k - j * nx, s = j * nx + (i & 1) * (nx >> 1) + (i >> 1);
+        xo[k] = xk[s];
+        bo[k] = bk[s];
+      }
+    xk += N;
+    bk += N;
+  }
+}
+
 // ----------------------------------------------------------------- row-marching smoothers
 // A workgroup smooths an owned block of W x Hgt nodes of one vector.  It reads
 // the (W + 2H) x (Hgt + 2H) region around it row by row, from the bottom, and
@@ -3547,6 +4241,8 @@ __global__ __launch_bounds__(MarchCfg<NSW>::THREADS) void k_node_march(mxh_level
 // ================================================================= launchers
 #define LAUNCH_CHECK() do { hipError_t _e = hipGetLastError(); if (_e != hipSuccess) return (int)_e; } while (0)
 
+static int grid_attrs();
+
 extern "C" {
 
 int mxh_init(void)
@@ -3571,11 +4267,14 @@ int mxh_init(void)
   const void* big[] = {(const void*)k_fft_solve<double>, (const void*)k_fft_solve<float>,
                        (const void*)k_fft_cols<double>, (const void*)k_fft_cols<float>,
                        (const void*)k_fft_rows<double, -1>, (const void*)k_fft_rows<double, 1>,
-                       (const void*)k_fft_rows<float, -1>, (const void*)k_fft_rows<float, 1>};
+                       (const void*)k_fft_rows<float, -1>, (const void*)k_fft_rows<float, 1>,
+                       (const void*)k_edge_cycle<double>, (const void*)k_edge_cycle<float>,
+                       (const void*)k_node_cycle<double>, (const void*)k_node_cycle<float>};
   for (const void* f : big) {
-    e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     if (e != hipSuccess) return (int)e;
   }
+  if (grid_attrs()) return (int)hipErrorInvalidValue;
   e = hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     g_stream = nullptr;
@@ -3765,6 +4464,158 @@ static int launch_tile_mode(int mode, dim3 grid, dim3 block, const mxh_level* lv
 }
 }  // extern "C++"
 
+extern "C++" {
+// grids smoothed whole in LDS: one thread per 2 x 2 block (1024 at most), the
+// vector and the lent sums within 160 KB (64 x 64 in both precisions)
+static bool afw_grid_fits(int prec, const mxh_level* lv)
+{
+  const long long N = (long long)lv->nx * lv->ny;
+  return N <= 4096 && (prec == MXH_F64 ? 40 : 20) * N <= LDS_MAX && lv->nx >= 4 && lv->ny >= 4;
+}
+
+template <typename T, int MODE>
+static void launch_grid(const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs b, mxh_vecs x, mxh_vecs xo,
+                        const void* eta, int nsweep, mxh_vecs xc_in, mxh_vecs bc, mxh_vecs xc, long long cs)
+{
+  const int N = lv->nx * lv->ny, blocks = N / 4;
+  const size_t sh = sizeof(C<T>) * (2 * (size_t)N + ((MODE & 8) ? N / 2 : 0));
+  auto go = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(nv), dim3(threads), sh, g_stream, *lv, *bl, (const C<T>*)b.p, b.stride,
+                       (const C<T>*)x.p, (C<T>*)xo.p, x.stride, (const T*)eta, nsweep, (const C<T>*)xc_in.p,
+                       (C<T>*)bc.p, (C<T>*)xc.p, cs);
+  };
+  if (blocks <= 256) go(k_afw_grid<T, MODE, 256, 1>, (blocks + 63) / 64 * 64);
+  else go(k_afw_grid<T, MODE, GridCfg<T>::TB, GridCfg<T>::NB>, GridCfg<T>::TB);
+}
+
+template <typename T>
+static int launch_grid_mode(int mode, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs b, mxh_vecs x,
+                            mxh_vecs xo, const void* eta, int nsweep, mxh_vecs xc_in, mxh_vecs bc, mxh_vecs xc)
+{
+  const long long cs = (mode & 8) ? bc.stride : (mode & 4) ? xc_in.stride : 0;
+#define GRID_CASE(M)                                                                     \
+  case M:                                                                                \
+    launch_grid<T, M>(lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc, cs);             \
+    break;
+  switch (mode) {
+    GRID_CASE(0)
+    GRID_CASE(1)
+    GRID_CASE(2)
+    GRID_CASE(5)
+    GRID_CASE(8)
+    GRID_CASE(10)
+  default: return (int)hipErrorInvalidValue;
+  }
+#undef GRID_CASE
+  LAUNCH_CHECK();
+  return 0;
+}
+
+template <typename T, int MODE>
+static int grid_attr()
+{
+  const void* f[] = {(const void*)k_afw_grid<T, MODE, 256, 1>,
+                     (const void*)k_afw_grid<T, MODE, GridCfg<T>::TB, GridCfg<T>::NB>};
+  for (const void* q : f) {
+    const hipError_t e = hipFuncSetAttribute(q, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
+    if (e != hipSuccess) return (int)e;
+  }
+  return 0;
+}
+
+}  // extern "C++"
+static int grid_attrs()
+{
+  return grid_attr<double, 0>() | grid_attr<double, 1>() | grid_attr<double, 2>() | grid_attr<double, 5>() |
+         grid_attr<double, 8>() | grid_attr<double, 10>() | grid_attr<float, 0>() | grid_attr<float, 1>() |
+         grid_attr<float, 2>() | grid_attr<float, 5>() | grid_attr<float, 8>() | grid_attr<float, 10>();
+}
+extern "C++" {
+static bool cycle_levels(const mxh_cycle* cy, CycleLevels* cl)
+{
+  if (cy->n < 1 || cy->n > CYCLE_MAXL) return false;
+  cl->n = cy->n;
+  for (int l = 0; l < cy->n; l++) {
+    const mxh_level* v = &cy->lv[l];
+    if (v->nx < 2 || v->ny < 2 || (v->nx & 1) || (v->ny & 1)) return false;
+    if (l && (v->nx != 2 * cy->lv[l - 1].nx || v->ny != 2 * cy->lv[l - 1].ny)) return false;
+    cl->nx[l] = v->nx;
+    cl->ny[l] = v->ny;
+    cl->hx[l] = v->hx;
+    cl->hy[l] = v->hy;
+    cl->eta[l] = cy->eta[l];
+    cl->b[l] = cy->b[l];
+    cl->x[l] = cy->x[l];
+    if ((cl->b[l] != nullptr) != (cl->x[l] != nullptr)) return false;
+  }
+  return cl->nx[cy->n - 1] * cl->ny[cy->n - 1] <= 1024;
+}
+// LDS of a cycle: x of all levels, b of the lower ones, the lent sums (or the
+// coarsest b where it is the only level), 4 KB of partial sums
+static size_t cycle_lds(int prec, const CycleLevels& cl, int comp)
+{
+  size_t tot = 0;
+  const size_t top = (size_t)cl.nx[cl.n - 1] * cl.ny[cl.n - 1];
+  for (int l = 0; l < cl.n; l++) tot += (size_t)comp * cl.nx[l] * cl.ny[l];
+  const size_t lent = comp == 1 ? top : cl.n > 1 ? top / 2 : 2 * top;
+  return csize(prec) * (2 * tot - comp * top + lent) + 16 * 256;
+}
+}  // extern "C++"
+
+int mxh_cycle_supported(int prec, const mxh_cycle* cy)
+{
+  CycleLevels cl;
+  return cycle_levels(cy, &cl) && 2 * cl.nx[0] * cl.ny[0] <= 256 && cycle_lds(prec, cl, 2) <= LDS_MAX;
+}
+
+int mxh_coarse_inverse(int n, int nprob, const double* L, double* W)
+{
+  if (n < 1 || n > 256 || nprob < 1) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_coarse_inverse, dim3(nprob), dim3((n + 63) / 64 * 64), 0, g_stream, n, L, W);
+  LAUNCH_CHECK();
+  return 0;
+}
+
+int mxh_edge_cycle(int prec, const mxh_cycle* cy, const mxh_bloch* bl, int nv, int nu, mxh_vecs b, mxh_vecs x,
+                   int xzero, const double* W, int per_problem)
+{
+  CycleLevels cl;
+  if (!W || nu < 1 || nv < 1 || !mxh_cycle_supported(prec, cy) || !cycle_levels(cy, &cl))
+    return (int)hipErrorInvalidValue;
+  if (nv > 1 && cl.x[0]) return (int)hipErrorInvalidValue;  // lower levels are returned for one vector
+  const int blocks = cl.nx[cl.n - 1] * cl.ny[cl.n - 1] / 4;
+  const dim3 tb(blocks <= 64 ? 64 : blocks <= 128 ? 128 : 256);
+  const size_t sh = cycle_lds(prec, cl, 2);
+  if (prec == MXH_F64)
+    hipLaunchKernelGGL(k_edge_cycle<double>, dim3(nv), tb, sh, g_stream, cl, *bl, nu, (const C<double>*)b.p, b.stride,
+                       b.map, (C<double>*)x.p, x.stride, xzero, W, per_problem);
+  else
+    hipLaunchKernelGGL(k_edge_cycle<float>, dim3(nv), tb, sh, g_stream, cl, *bl, nu, (const C<float>*)b.p, b.stride,
+                       b.map, (C<float>*)x.p, x.stride, xzero, W, per_problem);
+  LAUNCH_CHECK();
+  return 0;
+}
+
+int mxh_node_cycle(int prec, const mxh_cycle* cy, const mxh_bloch* bl, int nv, int nu, mxh_vecs b, mxh_vecs x,
+                   int xzero, const double* W, int per_problem)
+{
+  CycleLevels cl;
+  if (!W || nu < 1 || nv < 1 || !mxh_cycle_supported(prec, cy) || !cycle_levels(cy, &cl))
+    return (int)hipErrorInvalidValue;
+  if (nv > 1 && cl.x[0]) return (int)hipErrorInvalidValue;
+  const int blocks = cl.nx[cl.n - 1] * cl.ny[cl.n - 1] / 4;
+  const dim3 tb(blocks <= 64 ? 64 : blocks <= 128 ? 128 : 256);
+  const size_t sh = cycle_lds(prec, cl, 1);
+  if (prec == MXH_F64)
+    hipLaunchKernelGGL(k_node_cycle<double>, dim3(nv), tb, sh, g_stream, cl, *bl, nu, (const C<double>*)b.p, b.stride,
+                       (C<double>*)x.p, x.stride, xzero, W, per_problem);
+  else
+    hipLaunchKernelGGL(k_node_cycle<float>, dim3(nv), tb, sh, g_stream, cl, *bl, nu, (const C<float>*)b.p, b.stride,
+                       (C<float>*)x.p, x.stride, xzero, W, per_problem);
+  LAUNCH_CHECK();
+  return 0;
+}
+
 int mxh_afw_tile(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs b, mxh_vecs x, mxh_vecs xo,
                  const void* eta, int nsweep, int mode, mxh_vecs xc_in, mxh_vecs bc, mxh_vecs xc)
 {
@@ -3776,6 +4627,9 @@ int mxh_afw_tile(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh
     return (int)hipErrorInvalidValue;
   if ((mode & 4) && !xc_in.p) return (int)hipErrorInvalidValue;
   if ((mode & 8) && (!bc.p || !xc.p || bc.stride != xc.stride)) return (int)hipErrorInvalidValue;
+  if (afw_grid_fits(prec, lv))
+    return prec == MXH_F64 ? launch_grid_mode<double>(mode, lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc)
+                           : launch_grid_mode<float>(mode, lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc);
   const int R = prec == MXH_F64 ? TileCfg<double>::R : TileCfg<float>::R, TT = R - 2 * TILE_H;
   const int ntx = (lv->nx + TT - 1) / TT, nty = (lv->ny + TT - 1) / TT;
   dim3 grid(ntx * nty, nv), block((R / 2) * (R / 2));
@@ -4440,28 +5294,26 @@ static bool fft_plan(int n, FftPlan* p)
   return p->ns <= FFT_MAXS;
 }
 
-#define FFT_LDS_MAX (160 * 1024)
-static size_t fft_csz(int prec) { return prec == MXH_F64 ? 16 : 8; }
 // LDS of the one-launch solve: the vector, the phases and the mode terms
 static size_t fft_solve_lds(int prec, const mxh_level* lv)
 {
-  const size_t c = fft_csz(prec), s = (size_t)lv->nx + lv->ny;
+  const size_t c = csize(prec), s = (size_t)lv->nx + lv->ny;
   return c * ((size_t)lv->ny * (lv->nx | 1) + s) + c / 2 * s;
 }
 // columns per workgroup: 128-byte row segments, fewer where the columns are
 // long (at least 32 bytes of a row; 0: columns too long for LDS)
 static int fft_cols(int prec, const mxh_level* lv)
 {
-  const size_t c = fft_csz(prec);
+  const size_t c = csize(prec);
   int cb = (int)(128 / c);
-  while (cb * c >= 32 && c * cb * lv->ny + c / 2 * (lv->ny + cb) > FFT_LDS_MAX) cb >>= 1;
+  while (cb * c >= 32 && c * cb * lv->ny + c / 2 * (lv->ny + cb) > LDS_MAX) cb >>= 1;
   return cb * c >= 32 ? cb : 0;
 }
 // rows per workgroup: about 36 KB, so that four workgroups share a CU
 static int fft_rows(int prec, const mxh_level* lv)
 {
   int rb = 64;
-  while (rb > 1 && (rb >= 2 * lv->ny || fft_csz(prec) * rb * (size_t)(lv->nx | 1) > 36 * 1024)) rb >>= 1;
+  while (rb > 1 && (rb >= 2 * lv->ny || csize(prec) * rb * (size_t)(lv->nx | 1) > 36 * 1024)) rb >>= 1;
   return rb;
 }
 
@@ -4469,12 +5321,12 @@ int mxh_lift_supported(int prec, const mxh_level* lv)
 {
   FftPlan p;
   return fft_plan(lv->nx, &p) && fft_plan(lv->ny, &p) && fft_cols(prec, lv) > 0 &&
-         fft_csz(prec) * (2 * (size_t)lv->nx + 2) <= 64 * 1024;
+         csize(prec) * (2 * (size_t)lv->nx + 2) <= 64 * 1024;
 }
 
-int mxh_lift_launches(int prec, const mxh_level* lv) { return fft_solve_lds(prec, lv) <= FFT_LDS_MAX ? 6 : 8; }
+int mxh_lift_launches(int prec, const mxh_level* lv) { return fft_solve_lds(prec, lv) <= LDS_MAX ? 6 : 8; }
 
-size_t mxh_lift_table_bytes(int prec, const mxh_level* lv) { return fft_csz(prec) * ((size_t)lv->nx + lv->ny); }
+size_t mxh_lift_table_bytes(int prec, const mxh_level* lv) { return csize(prec) * ((size_t)lv->nx + lv->ny); }
 
 int mxh_lift_table(int prec, const mxh_level* lv, void* table)
 {
@@ -4502,7 +5354,7 @@ static int node_direct(int prec, const mxh_level* lv, const mxh_bloch* bl, int n
   const C<T>* B = (const C<T>*)b.p;
   C<T>* X = (C<T>*)x.p;
   const size_t one = fft_solve_lds(prec, lv);
-  if (one <= FFT_LDS_MAX) {
+  if (one <= LDS_MAX) {
     const long long N = (long long)lv->nx * lv->ny;
     hipLaunchKernelGGL(k_fft_solve<T>, dim3(nv), dim3(N >= 8192 ? 1024 : N >= 2048 ? 512 : 256), one, g_stream, *lv,
                        *bl, px, py, twx, twy, B, b.stride, X, x.stride);
