@@ -213,6 +213,17 @@ int mxh_gram_cols(const mxh_level *lv, const mxh_bloch *bl, int nprob, const int
                   const int *cmap, int m, mxh_vecs u, const double *eta64, double *out,
                   void *work);
 
+/* The Rayleigh-Ritz step's small eigenproblems, block j being problem q =
+   pmap ? pmap[j] : j: A c = lam B c with A = sk K + M, B = M from the sums of
+   mxh_gram (basis = 0: m columns, C_j m x m column-major) or mxh_gram_cols
+   (basis > 0 columns at most, cmap as there; C_j basis x 2m: the Ritz vectors,
+   then the same without rows 0 .. m - 1).  Columns are taken in order, scaled to
+   unit M-norm, and kept only if the squared sine of their angle to those kept
+   before exceeds pivot.  lam[q vpp + i], i < m: the lowest values, ascending.
+   status[j]: 0, 1 a sum is not finite, 2 fewer than m columns kept (C_j = 0). */
+int mxh_ritz(int m, int basis, int nprob, const int *pmap, const int *cmap, const double *gram, double sk,
+             double pivot, double *C, double *lam, int vpp, int *status);
+
 /* Per block j (problem q = pmap ? pmap[j] : j): E_j = sum_i C_j[i + j m] U_i
    over the problem's m FP64 vectors; C: device complex, m*m per block.
    n = complex values per vector. */

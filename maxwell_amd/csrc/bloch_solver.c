@@ -9,8 +9,7 @@
  *   [Gamma point: remove the constant fields, test_block2d.c:217-220]
  *   Ar = U^H (K+M) U, Mr = U^H M U; hegv; E = U C
  *   b = (K + (1 - lam) M) e and its norms     convergence test + next defect
- * Every kernel launch covers all vectors of all problems of the batch; the
- * small Ritz problems are solved on the host in FP64.
+ * Every kernel launch covers all vectors of all problems of the batch.
  */
 #include "maxwell_amd.h"
 
@@ -53,15 +52,16 @@ struct mx_solver {
   void *gramwork;
   int ne0, nn0;         /* coarse edge / node unknowns */
   /* host scratch */
-  double complex *hAe, *hAn, *hMr, *hC; /* hMr, hC: m x m per problem (PINVIT);
-                                           hC: 3m x 2m per problem (LOBPCG) */
+  double complex *hAe, *hAn;
   int *hwvalid;         /* LOBPCG: vector's W column written this step */
   int pvalid;           /* LOBPCG: the P columns hold a search direction
                            (from the second Ritz step of the loop on) */
   int *hcols, *dcols;   /* LOBPCG: the Gram's column list per problem (vpp + 1
                            ints: count, then columns of [E W P]) */
-  double *hgram, *hnorm, *hlam, *hbloch; /* hgram: pinned */
-  void *ev_gram[2];                      /* Gram sums of each half on the host */
+  /* what a block step tells the host, one copy: norms (2 per vector), Ritz
+     values (vpp per problem), Ritz status (per listed problem); host: pinned */
+  double *hnorm, *hlam, *hbloch;
+  int *dstat, *hstat;
   int *gamma;
   int *hlist, *hslot;   /* host index lists (problems, vectors, maps) */
   int *dlist;           /* device copies of the lists */
@@ -131,7 +131,6 @@ void mx_solver_destroy(mx_solver *s)
   mxh_free(s->dAe);
   mxh_free(s->dAn);
   mxh_free(s->dAi);
-  mxh_free(s->dlam);
   mxh_free(s->dnorm);
   mxh_free(s->dgram);
   mxh_free(s->dC);
@@ -140,24 +139,25 @@ void mx_solver_destroy(mx_solver *s)
   mxh_free(s->gramwork);
   free(s->hAe);
   free(s->hAn);
-  free(s->hMr);
-  free(s->hC);
   free(s->hwvalid);
-  mxh_host_free(s->hgram);
-  for (int h = 0; h < 2; h++)
-    if (s->ev_gram[h]) mxh_event_destroy(s->ev_gram[h]);
-  free(s->hnorm);
-  free(s->hlam);
+  mxh_host_free(s->hnorm);
   free(s->hbloch);
   free(s->gamma);
-  free(s->hlist);
+  mxh_host_free(s->hlist);
   free(s->hslot);
   mxh_free(s->dlist);
-  free(s->hcols);
+  mxh_host_free(s->hcols);
   mxh_free(s->dcols);
   mxh_free(s->dinfo);
   free(s->hinfo);
   free(s);
+}
+
+/* the buffer of a block step's results (dnorm, dlam, dstat) */
+static size_t step_bytes(const mx_solver *s)
+{
+  return sizeof(double) * (2 * (size_t)s->nvmax + (size_t)s->vpp * s->cfg.max_problems) +
+         sizeof(int) * (size_t)s->cfg.max_problems;
 }
 
 /* device allocation counted into the solver's footprint */
@@ -278,36 +278,33 @@ int mx_solver_create(const mx_config *cfg, const double *eta, mx_solver **out)
   s->dbloch = (double *)dalloc(s, sizeof(double) * 4 * P);
   s->dAe = (double *)dalloc(s, 16 * (size_t)s->ne0 * s->ne0 * P);
   s->dAn = (double *)dalloc(s, 16 * (size_t)s->nn0 * s->nn0 * P);
-  s->dlam = (double *)dalloc(s, sizeof(double) * (size_t)vpp * P);
-  s->dnorm = (double *)dalloc(s, sizeof(double) * 2 * nv);
+  s->dnorm = (double *)dalloc(s, step_bytes(s));
+  s->dlam = s->dnorm + 2 * (size_t)nv;
+  s->dstat = (int *)(s->dlam + (size_t)vpp * P);
   s->dgram = (double *)dalloc(s, sizeof(double) * 4 * (size_t)vpp * vpp * P);
   s->dC = (double *)dalloc(s, 16 * (size_t)vpp * m * 2 * P);
   s->dwork = (double *)dalloc(s, sizeof(double) * (513 * 4 * (size_t)nv + 1024));
   s->dcoef = (double *)dalloc(s, sizeof(double) * 2 * (size_t)nv);
   s->gramwork = dalloc(s, mxh_gram_work_bytes(vpp, P));
-  if (!s->dE || !s->dU || !s->dbloch || !s->dAe || !s->dAn || !s->dlam || !s->dnorm || !s->dgram || !s->dC ||
+  if (!s->dE || !s->dU || !s->dbloch || !s->dAe || !s->dAn || !s->dnorm || !s->dgram || !s->dC ||
       !s->dwork || !s->dcoef || !s->gramwork)
     goto nomem;
   s->hAe = (double complex *)malloc(sizeof(double complex) * (size_t)s->ne0 * s->ne0 * P);
   s->hAn = (double complex *)malloc(sizeof(double complex) * (size_t)s->nn0 * s->nn0 * P);
-  s->hMr = (double complex *)malloc(sizeof(double complex) * (size_t)m * m * P);
-  s->hC = (double complex *)malloc(sizeof(double complex) * (size_t)vpp * m * 2 * P);
   s->hwvalid = (int *)calloc((size_t)nv, sizeof(int));
-  s->hgram = (double *)mxh_host_alloc(sizeof(double) * 4 * (size_t)vpp * vpp * P);
-  for (int h = 0; h < 2; h++)
-    if (mxh_event_create(&s->ev_gram[h])) s->ev_gram[h] = NULL;
-  s->hnorm = (double *)malloc(sizeof(double) * 2 * nv);
-  s->hlam = (double *)malloc(sizeof(double) * (size_t)vpp * P);
+  s->hnorm = (double *)mxh_host_alloc(step_bytes(s));
+  s->hlam = s->hnorm + 2 * (size_t)nv;
+  s->hstat = (int *)(s->hlam + (size_t)vpp * P);
   s->hbloch = (double *)malloc(sizeof(double) * 4 * P);
   s->gamma = (int *)calloc(P, sizeof(int));
-  s->hlist = (int *)malloc(sizeof(int) * (P + 4 * (size_t)nv));
+  s->hlist = (int *)mxh_host_alloc(sizeof(int) * (P + 4 * (size_t)nv));
   s->hslot = (int *)malloc(sizeof(int) * (size_t)vpp * P);
   s->dlist = (int *)dalloc(s, sizeof(int) * (P + 4 * (size_t)nv));
-  s->hcols = (int *)malloc(sizeof(int) * (size_t)(vpp + 1) * P);
+  s->hcols = (int *)mxh_host_alloc(sizeof(int) * (size_t)(vpp + 1) * P);
   s->dcols = (int *)dalloc(s, sizeof(int) * (size_t)(vpp + 1) * P);
   s->dinfo = (int *)dalloc(s, sizeof(int) * P);
   s->hinfo = (int *)malloc(sizeof(int) * P);
-  if (!s->hAe || !s->hAn || !s->hMr || !s->hC || !s->hwvalid || !s->hgram || !s->ev_gram[0] || !s->ev_gram[1] || !s->hnorm || !s->hlam || !s->hbloch ||
+  if (!s->hAe || !s->hAn || !s->hwvalid || !s->hnorm || !s->hbloch ||
       !s->gamma || !s->hlist || !s->hslot || !s->dlist || !s->dinfo || !s->hinfo || !s->hcols || !s->dcols)
     goto nomem;
   if (mxh_sync()) goto dev;
@@ -651,134 +648,17 @@ static int lift(mx_solver *s, int nv, const mxh_bloch *bl, double *E, const void
   return lift_to(s, nv, bl, E, X, gmap, NULL, NULL);
 }
 
-/* The small generalised eigenproblems Ar c = lam Mr c (Ar = U^H (K+M) U,
-   Mr = U^H M U, from the Gram sums in hgram) of the list's problems
-   j0 <= j < j1: eigenvectors to hC, Ritz values (of K+M) to hlam. */
-static int ritz_host(mx_solver *s, int j0, int j1, const int *plist)
-{
-  const int m = s->cfg.block, L = s->L, np = m * (m + 1) / 2;
-  const double sk = 1.0 / (s->lv[L].hx * s->lv[L].hy);
-  for (int j = j0; j < j1; j++) {
-    const int p = plist ? plist[j] : j;
-    const double *g = s->hgram + 4 * (size_t)np * j;
-    double complex *Ar = s->hC + (size_t)j * m * m, *Mr = s->hMr + (size_t)j * m * m;
-    for (int q = 0; q < 4 * np; q++)
-      if (!isfinite(g[q])) return MX_ENOTFINITE;
-    for (int a = 0; a < m; a++)
-      for (int c = 0; c <= a; c++) {
-        const double *q = g + 4 * (a * (a + 1) / 2 + c);
-        double complex gk = q[0] + I * q[1], gm = q[2] + I * q[3];
-        Ar[a + c * m] = sk * gk + gm;
-        Mr[a + c * m] = gm;
-        Ar[c + a * m] = conj(Ar[a + c * m]);
-        Mr[c + a * m] = conj(gm);
-      }
-    /* Ar becomes the eigenvectors C of the problem.  Mr must be definite
-       to well above rounding: a pivot of its Cholesky factor below 1e-13 of
-       its diagonal entry means block vectors that are dependent to FP64
-       precision (repeated or zero start vectors), whose Ritz values would be
-       rounding noise */
-    if (mxd_hegv_rel(m, Ar, Mr, s->hlam + (size_t)p * s->vpp, 1e-13)) return MX_ELAPACK;
-  }
-  return MX_OK;
-}
-
-/* LOBPCG Rayleigh-Ritz of the list's problems j0 <= j < j1 over the basis
-   [E | W | P] (3m columns; the Gram sums of all pairs in hgram): the columns
-   are scaled to unit M-norm and taken in the order E, W, P, each kept only
-   if the squared sine of its angle to the span of the columns kept before it
-   exceeds LOBPCG_PIVOT (pivot of a Cholesky factorisation of the scaled
-   M-Gram), so that W and P columns that are zero (no step yet, or a locked
-   vector's W, which is not written while the vector is locked) or
-   numerically dependent drop out.  The kept basis then has a scaled Gram of
-   condition below about 3m / LOBPCG_PIVOT, which bounds what the rounding of
-   the Gram sums (eps relative) does to the M-orthonormality of the new block
-   (about eps times that condition).  At least m columns must stay.  The
-   lowest m Ritz pairs of the kept pencil give hlam and two coefficient blocks
-   per problem in hC (3m x 2m, column-major): E_new = [E W P] C_E and the next
-   search direction P_new = [W P] C_WP (the W and P rows of C_E). */
+/* Pivot below which a column of the Ritz basis counts as dependent on those
+   before it (squared sine of its angle to their span; mxh_ritz).  PINVIT: a
+   block vector dependent to FP64 precision (repeated or zero start vectors),
+   whose Ritz values would be rounding noise; all m have to stay.  LOBPCG, over
+   [E | W | P] in this order: W and P columns that are zero or numerically
+   dependent drop out.  The kept basis then has a scaled Gram of condition below
+   about 3m / LOBPCG_PIVOT, which bounds what the rounding of the Gram sums (eps
+   relative) does to the M-orthonormality of the new block (about eps times that
+   condition). */
+#define PINVIT_PIVOT 1e-13
 #define LOBPCG_PIVOT 1e-7
-static int lobpcg_problem(mx_solver *s, int j, int p)
-{
-  const int m = s->cfg.block, L = s->L, k = 3 * m, np = k * (k + 1) / 2;
-  const double sk = 1.0 / (s->lv[L].hx * s->lv[L].hy);
-  double w[48], dsc[48];
-  int keep[48];
-  double complex A[48 * 48], B[48 * 48], Lf[48 * 48], As[48 * 48], Bs[48 * 48];
-  const double *g = s->hgram + 4 * (size_t)np * j;
-  /* the Gram holds the problem's listed columns (E, the W of its unlocked
-     vectors, P once it holds a direction) at list positions 0 .. kc - 1 */
-  const int *cl = s->hcols + (size_t)p * (k + 1), kc = cl[0];
-  for (int q = 0; q < 2 * kc * (kc + 1); q++)
-    if (!isfinite(g[q])) return MX_ENOTFINITE;
-  for (int a = 0; a < kc; a++)
-    for (int c = 0; c <= a; c++) {
-      const double *q = g + 4 * (a * (a + 1) / 2 + c);
-      const double complex gk = q[0] + I * q[1], gm = q[2] + I * q[3];
-      A[a + c * k] = sk * gk + gm;
-      B[a + c * k] = gm;
-      A[c + a * k] = conj(A[a + c * k]);
-      B[c + a * k] = conj(gm);
-    }
-  /* greedy column selection by a Cholesky factorisation of the scaled B */
-  int kk = 0;
-  for (int c = 0; c < kc; c++) {
-    const double bcc = creal(B[c + c * k]);
-    if (!(bcc > 0.0) || !isfinite(bcc)) continue;
-    const double d = 1.0 / sqrt(bcc);
-    /* row kk of the factor of the scaled B restricted to the kept columns */
-    double piv = 1.0;
-    for (int t = 0; t < kk; t++) {
-      double complex z = B[c + keep[t] * k] * d * dsc[t];
-      for (int u = 0; u < t; u++) z -= Lf[kk + u * 48] * conj(Lf[t + u * 48]);
-      z /= creal(Lf[t + t * 48]);
-      Lf[kk + t * 48] = z;
-      piv -= creal(z * conj(z));
-    }
-    if (!(piv > LOBPCG_PIVOT)) continue;
-    Lf[kk + kk * 48] = sqrt(piv);
-    keep[kk] = c;
-    dsc[kk] = d;
-    kk++;
-  }
-  if (kk < m) return MX_ELAPACK;
-  for (int t = 0; t < kk; t++)
-    for (int u = 0; u < kk; u++) {
-      As[t + u * kk] = A[keep[t] + keep[u] * k] * dsc[t] * dsc[u];
-      Bs[t + u * kk] = B[keep[t] + keep[u] * k] * dsc[t] * dsc[u];
-    }
-  if (mxd_hegv(kk, As, Bs, w)) return MX_ELAPACK;
-  double complex *Cp = s->hC + (size_t)j * k * 2 * m;
-  for (int q = 0; q < k * 2 * m; q++) Cp[q] = 0.0;
-  for (int i = 0; i < m; i++) {
-    s->hlam[(size_t)p * s->vpp + i] = w[i];
-    for (int t = 0; t < kk; t++) {
-      const int c = cl[1 + keep[t]];
-      const double complex cf = As[t + i * kk] * dsc[t];
-      Cp[c + (size_t)i * k] = cf;
-      if (c >= m) Cp[c + (size_t)(m + i) * k] = cf;
-    }
-  }
-  return MX_OK;
-}
-
-/* The problems are independent (each writes its own hC block and hlam
-   entries), so a team of host threads shares them: at 3m = 36 one
-   eigensolve takes about 2 ms, against a few ms of GPU work per half-batch
-   that it has to hide behind. */
-static int ritz_host_lobpcg(mx_solver *s, int j0, int j1, const int *plist)
-{
-  int status = MX_OK;
-#pragma omp parallel for schedule(dynamic, 1) if (j1 - j0 > 1)
-  for (int j = j0; j < j1; j++) {
-    const int e = lobpcg_problem(s, j, plist ? plist[j] : j);
-    if (e) {
-#pragma omp critical(mx_ritz_status)
-      if (!status) status = e;
-    }
-  }
-  return status;
-}
 
 /* Launches the defects (K + (1 - lam) M) e of nv listed vectors (dvlist:
    device, null = 0..nv-1) into slots slot0 .. slot0 + nv - 1 of r (next
@@ -799,28 +679,26 @@ static int defect_launch(mx_solver *s, int nv, const int *dvlist, double *E, voi
 }
 
 /* Rayleigh-Ritz over the blocks of the listed problems (plist on the host,
-   dplist on the device; null: problems 0..na-1): Gram sums, the small
-   eigenproblems on the host, Eout = Ein C; then the defects of Eout's
-   vectors (the m of each listed problem in list order: dvlist, nvl = na m)
-   to r and their norms to hnorm.  With device lists and two or more
-   problems the list is done in two halves, so that the host's eigensolves
-   of one half run while the GPU sums the other half's Gram products or
-   updates and checks the first half. */
+   dplist on the device): Gram sums, the small eigenproblems (mxh_ritz),
+   Eout = Ein C; then the defects of Eout's vectors (the m of each listed
+   problem in list order: dvlist, nvl = na m) to r.  Norms, Ritz values and
+   statuses come back in one copy, the step's only wait.  On the host the
+   eigenproblems (12 x 12: 20-40 us each, 36 x 36: 1 ms) held the GPU up: 64^2 FP64,
+   16 problems, 680 us a step against 450 us of kernels. */
 static int ritz_defect(mx_solver *s, int na, const int *plist, const int *dplist, int nvl, const int *dvlist,
                        double *Ein, double *Eout, void *r)
 {
-  const int m = s->cfg.block, L = s->L, mg = s->vpp, np = mg * (mg + 1) / 2;
-  const size_t csz = s->lobpcg ? (size_t)mg * 2 * m : (size_t)m * m; /* coefficients per problem */
+  const int m = s->cfg.block, L = s->L, mg = s->vpp;
   const long long n = edim(s, L);
+  const double sk = 1.0 / (s->lv[L].hx * s->lv[L].hy);
   mxh_bloch bl = batch_bloch(s);
-  const int split = na >= 2 && dplist && dvlist;
-  const int nh[2] = {split ? (na + 1) / 2 : na, split ? na / 2 : 0};
+  int e;
   if (s->lobpcg) {
     /* the Gram's columns per problem: E, the W of the vectors preconditioned
        this step (a locked vector's W slot is not written) and P once it holds
        a direction; the Ritz step never uses the products it leaves out */
     for (int j = 0; j < na; j++) {
-      const int p = plist ? plist[j] : j;
+      const int p = plist[j];
       int *cl = s->hcols + (size_t)p * (mg + 1), c = 0;
       for (int i = 0; i < m; i++) cl[1 + c++] = i;
       for (int i = 0; i < m; i++)
@@ -830,42 +708,25 @@ static int ritz_defect(mx_solver *s, int na, const int *plist, const int *dplist
       cl[0] = c;
     }
     CK(mxh_h2d(s->dcols, s->hcols, sizeof(int) * (size_t)(mg + 1) * s->last_nprob));
+    CK(mxh_gram_cols(&s->lv[L], &bl, na, dplist, s->dcols, mg, V(Ein, s->es), s->eta64[L], s->dgram, s->gramwork));
+    CK(mxh_ritz(m, mg, na, dplist, s->dcols, s->dgram, sk, LOBPCG_PIVOT, s->dC, s->dlam, mg, s->dstat));
+  } else {
+    CK(mxh_gram(&s->lv[L], &bl, na, dplist, mg, V(Ein, s->es), s->eta64[L], s->dgram, s->gramwork));
+    CK(mxh_ritz(m, 0, na, dplist, NULL, s->dgram, sk, PINVIT_PIVOT, s->dC, s->dlam, mg, s->dstat));
   }
-  for (int h = 0, j0 = 0; h < 2 && nh[h]; j0 += nh[h], h++) {
-    const int *pm = dplist ? dplist + j0 : NULL;
-    double *gout = s->dgram + 4 * (size_t)np * j0;
-    CK(s->lobpcg ? mxh_gram_cols(&s->lv[L], &bl, nh[h], pm, s->dcols, mg, V(Ein, s->es), s->eta64[L], gout, s->gramwork)
-                 : mxh_gram(&s->lv[L], &bl, nh[h], pm, mg, V(Ein, s->es), s->eta64[L], gout, s->gramwork));
-    CK(mxh_d2h_async(s->hgram + 4 * (size_t)np * j0, s->dgram + 4 * (size_t)np * j0,
-                     sizeof(double) * 4 * (size_t)np * nh[h]));
-    CK(mxh_event_record(s->ev_gram[h]));
-    s->st.launches += 3;
-  }
-  for (int h = 0, j0 = 0; h < 2 && nh[h]; j0 += nh[h], h++) {
-    CK(mxh_event_sync(s->ev_gram[h]));
-    int e = s->lobpcg ? ritz_host_lobpcg(s, j0, j0 + nh[h], plist) : ritz_host(s, j0, j0 + nh[h], plist);
-    if (e) {
-      mxh_sync();
-      return e;
-    }
-    CK(mxh_h2d(s->dC + 2 * (size_t)j0 * csz, s->hC + (size_t)j0 * csz, sizeof(double complex) * csz * nh[h]));
-    CK(mxh_h2d(s->dlam, s->hlam, sizeof(double) * (size_t)mg * s->last_nprob));
-    if (s->lobpcg && !(m & 1)) /* [E W P] -> E_new (slots 0..m-1), P_new (slots 2m..3m-1) */
-      CK(mxh_lobpcg_combine(n, nh[h], dplist ? dplist + j0 : NULL, m, V(Ein, s->es), V(Eout, s->es),
-                            s->dC + 2 * (size_t)j0 * csz));
-    else if (s->lobpcg)
-      CK(mxh_combine_x(n, nh[h], dplist ? dplist + j0 : NULL, mg, 2 * m, m, m, V(Ein, s->es), mg, V(Eout, s->es), mg,
-                       s->dC + 2 * (size_t)j0 * csz));
-    else if (m > 16)  /* every input read once */
-      CK(mxh_combine_x(n, nh[h], dplist ? dplist + j0 : NULL, m, m, m, 0, V(Ein, s->es), m, V(Eout, s->es), m,
-                       s->dC + 2 * (size_t)j0 * csz));
-    else
-      CK(mxh_block_combine(n, nh[h], dplist ? dplist + j0 : NULL, m, V(Ein, s->es), V(Eout, s->es),
-                           s->dC + 2 * (size_t)j0 * csz));
-    s->st.launches++;
-    if ((e = defect_launch(s, nh[h] * m, dvlist ? dvlist + j0 * m : NULL, Eout, r, j0 * m))) return e;
-  }
-  CK(mxh_d2h(s->hnorm, s->dnorm, sizeof(double) * 2 * nvl));
+  if (s->lobpcg && !(m & 1)) /* [E W P] -> E_new (slots 0..m-1), P_new (slots 2m..3m-1) */
+    CK(mxh_lobpcg_combine(n, na, dplist, m, V(Ein, s->es), V(Eout, s->es), s->dC));
+  else if (s->lobpcg)
+    CK(mxh_combine_x(n, na, dplist, mg, 2 * m, m, m, V(Ein, s->es), mg, V(Eout, s->es), mg, s->dC));
+  else if (m > 16)  /* every input read once */
+    CK(mxh_combine_x(n, na, dplist, m, m, m, 0, V(Ein, s->es), m, V(Eout, s->es), m, s->dC));
+  else
+    CK(mxh_block_combine(n, na, dplist, m, V(Ein, s->es), V(Eout, s->es), s->dC));
+  s->st.launches += 4;
+  if ((e = defect_launch(s, nvl, dvlist, Eout, r, 0))) return e;
+  CK(mxh_d2h(s->hnorm, s->dnorm, step_bytes(s)));
+  for (int j = 0; j < na; j++)
+    if (s->hstat[j]) return s->hstat[j] == 1 ? MX_ENOTFINITE : MX_ELAPACK;
   return MX_OK;
 }
 

@@ -1083,6 +1083,287 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gram(mxh_level lv, mxh
   }
 }
 
+// ----------------------------------------------------------------- Ritz problems
+// The small generalised eigenproblems of the Rayleigh-Ritz step, one workgroup
+// per problem, from the Gram sums of k_gram: A = sk K + M and B = M over the
+// problem's n columns (at most 48).  The columns are scaled to unit M-norm and
+// taken in order, each kept only if its pivot in the Cholesky factorisation of
+// the scaled B (the squared sine of its angle to the columns kept before it)
+// exceeds pivot; then C = L^-1 A L^-H, cyclic Jacobi with the rotations of a
+// round-robin round (n / 2 disjoint pairs) applied together, and X = L^-H Y.
+// The lowest m pairs give lam and the coefficient block, with basis > 0 (the
+// LOBPCG basis of `basis` columns) basis x 2m: the Ritz vectors and once more
+// without their first m rows.  status: 0, 1 a sum is not finite, 2 fewer than
+// m columns kept; the coefficients are then 0.
+//
+// Everything stays in LDS in FP64; a step of a factorisation or substitution
+// has one barrier, a Jacobi round two.  What bounds it is that chain (per round
+// a rotation's square roots, a barrier, the LDS reads and writes of A and V, a
+// barrier): 54 us for 16 problems of 9 columns and 638 us for 64 of 36, of
+// which all run at once.  On the host the same problems took 0.5 to 1 ms
+// between device steps that wait for them (64^2 grids in FP64, 16 problems: a
+// solve of 80 ms against 56) and needed two transfers; at 512^2 and 36 columns,
+// where the host could work beside the device, both ways are alike (720 ms
+// against 728).
+#define RITZ_MAX 48
+
+MXH_DEV double rsqrt64(double a)
+{
+  double r = __builtin_amdgcn_rsq(a);
+  r = r * fma(-0.5 * a * r, r, 1.5);
+  return r * fma(-0.5 * a * r, r, 1.5);
+}
+
+__global__ __launch_bounds__(1024) void k_ritz(int m, int basis, const int* pmap, const int* cmap, const double* gram,
+                                              double sk, double pivot, double* Cout, double* lam,
+                                              int vpp, int* status)
+{
+  extern __shared__ double smem[];
+  const int jb = blockIdx.x, prob = pmap ? pmap[jb] : jb, tid = threadIdx.x, bd = blockDim.x;
+  const int k = basis ? basis : m, np = k * (k + 1) / 2;
+  const int* cl = cmap ? cmap + (size_t)prob * (k + 1) : nullptr;
+  const int n = cl ? min(cl[0], k) : k;
+  C<double>*A = (C<double>*)smem, *B = A + n * n, *Vv = B + n * n;
+  __shared__ double dsc[RITZ_MAX], w[RITZ_MAX], rc[RITZ_MAX / 2], rs[RITZ_MAX / 2], red[16];
+  __shared__ C<double> re[RITZ_MAX / 2];
+  __shared__ int keep[RITZ_MAX], ord[RITZ_MAX], bad;
+  const double* g = gram + 4 * (size_t)np * jb;
+  const int csz = basis ? basis * 2 * m : m * m;
+  C<double>* Cj = (C<double>*)Cout + (size_t)jb * csz;
+  if (tid == 0) bad = 0;
+  for (int e = tid; e < csz; e += bd) Cj[e] = czero<double>();
+  __syncthreads();
+  // column-major A and B, lower triangle of the sums mirrored
+  for (int e = tid; e < n * n; e += bd) {
+    const int c = e / n, a = e - c * n, hi = max(a, c), lo = min(a, c);
+    const double* q = g + 4 * (hi * (hi + 1) / 2 + lo);
+    const double q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
+    if (!(isfinite(q0) && isfinite(q1) && isfinite(q2) && isfinite(q3))) bad = 1;
+    const double s = a >= c ? 1.0 : -1.0;
+    B[e] = cmk(q2, a == c ? 0.0 : s * q3);
+    A[e] = cmk(sk * q0 + q2, a == c ? 0.0 : s * (sk * q1 + q3));
+  }
+  __syncthreads();
+  if (bad) {
+    if (tid == 0) status[jb] = 1;
+    return;
+  }
+  if (tid < n) {
+    const double b = B[tid + tid * n].r;
+    dsc[tid] = b > 0.0 ? 1.0 / sqrt(b) : 0.0;  // 0: never kept
+  }
+  __syncthreads();
+  for (int e = tid; e < n * n; e += bd) {
+    const int c = e / n, a = e - c * n;
+    const double s = dsc[a] * dsc[c];
+    A[e] = s * A[e];
+    B[e] = s * B[e];
+  }
+  // pivots in order; a kept column's multiples leave the rest (right-looking)
+  const int ti = tid & 15, tj = tid >> 4, sj = bd >> 4;
+  int kk = 0;
+  for (int c = 0; c < n; c++) {
+    __syncthreads();
+    const double piv = B[c + c * n].r;
+    if (!(piv > pivot)) continue;  // uniform
+    if (tid == 0) keep[kk] = c;
+    kk++;
+    const double inv = 1.0 / piv;
+    for (int j = c + 1 + tj; j < n; j += sj) {
+      const C<double> f = inv * cconj(B[j + c * n]);
+      for (int i = j + ti; i < n; i += 16) B[i + j * n] -= B[i + c * n] * f;
+    }
+  }
+  __syncthreads();
+  if (kk < m) {
+    if (tid == 0) status[jb] = 2;
+    return;
+  }
+  // the kept rows and columns, with leading dimension kk: the factor L (lower)
+  // and the matrix
+  for (int e = tid; e < kk * kk; e += bd) {
+    const int u = e / kk, t = e - u * kk, ku = keep[u], kt = keep[t];
+    Vv[e] = t > u ? (1.0 / sqrt(B[ku + ku * n].r)) * B[kt + ku * n]
+                  : (t == u ? cmk(sqrt(B[ku + ku * n].r), 0.0) : czero<double>());
+  }
+  __syncthreads();
+  for (int e = tid; e < kk * kk; e += bd) B[e] = Vv[e];
+  __syncthreads();
+  for (int e = tid; e < kk * kk; e += bd) {
+    const int u = e / kk, t = e - u * kk;
+    Vv[e] = A[keep[t] + keep[u] * n];
+  }
+  __syncthreads();
+  for (int e = tid; e < kk * kk; e += bd) A[e] = Vv[e];
+  // A <- L^-1 A (rows, divided by the diagonal at the end), then A L^-H
+  for (int r = 0; r < kk; r++) {
+    __syncthreads();
+    const double inv = 1.0 / B[r + r * kk].r;
+    for (int j = tj; j < kk; j += sj) {
+      const C<double> f = inv * A[r + j * kk];
+      for (int i = r + 1 + ti; i < kk; i += 16) A[i + j * kk] -= B[i + r * kk] * f;
+    }
+  }
+  for (int r = 0; r < kk; r++) {
+    __syncthreads();
+    const double inv = 1.0 / B[r + r * kk].r;
+    for (int j = r + 1 + tj; j < kk; j += sj) {
+      const C<double> f = inv * cconj(B[j + r * kk]);
+      for (int i = ti; i < kk; i += 16) A[i + j * kk] -= A[i + r * kk] * f;
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < kk * kk; e += bd) {
+    const int j = e / kk, i = e - j * kk;
+    const C<double> a = A[i + j * kk], b = cconj(A[j + i * kk]);
+    Vv[e] = (0.5 / (B[i + i * kk].r * B[j + j * kk].r)) * (a + b);
+  }
+  __syncthreads();
+  for (int e = tid; e < kk * kk; e += bd) {
+    const int j = e / kk, i = e - j * kk;
+    A[e] = i == j ? cmk(Vv[e].r, 0.0) : Vv[e];
+    Vv[e] = cmk(i == j ? 1.0 : 0.0, 0.0);
+  }
+  // Jacobi
+  const int h = (kk + 1) / 2, ne = 2 * h;
+  // this thread's items of a round: 2 x 2 blocks (slots P, K), then rows i of V
+  // for slot K (P = -1 - i); none: K < 0.  At most two (mxh_ritz)
+  int itP[2], itK[2];
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int x = tid + u * bd, y = x - h * h;
+    itK[u] = x >= h * h + kk * h ? -1 : (y < 0 ? x / h : y / kk);
+    itP[u] = y < 0 ? x % h : -1 - y % kk;
+  }
+  for (int sweep = 0; sweep < 64; sweep++) {
+    __syncthreads();
+    double off = 0.0, dia = 0.0;
+    for (int e = tid; e < kk * kk; e += bd) {
+      const double t = A[e].r * A[e].r + A[e].i * A[e].i;
+      if (e / kk == e % kk) dia += t;
+      else off += t;
+    }
+    off = wave_sum(off);
+    dia = wave_sum(dia);
+    if ((tid & 63) == 0) {
+      // one slot pair per wave (at most 16 waves)
+      w[tid >> 6] = off;
+      red[tid >> 6] = dia;
+    }
+    __syncthreads();
+    off = dia = 0.0;
+    for (int q = 0; q < bd >> 6; q++) {
+      off += w[q];
+      dia += red[q];
+    }
+    if (off <= 1e-32 * dia) break;  // uniform
+    for (int round = 0; round < ne - 1; round++) {
+      // round-robin pairs: index ne - 1 stays, the others rotate (slot 0 holds
+      // it); an index >= kk is the dummy of an odd count
+      auto first = [&](int slot) {
+        const int a = round + slot;
+        return slot == 0 ? ne - 1 : (a >= ne - 1 ? a - (ne - 1) : a);
+      };
+      auto second = [&](int slot) {
+        const int a = round - slot;
+        return slot == 0 ? round : (a < 0 ? a + ne - 1 : a);
+      };
+      if (tid < h) {
+        const int p = first(tid), q = second(tid);
+        double cs = 1.0, sn = 0.0;
+        C<double> e = cmk(1.0, 0.0);
+        if (p < kk) {
+          const C<double> z = A[p + q * kk];
+          const double z2 = z.r * z.r + z.i * z.i;
+          if (z2 > 1e-290) {
+            const double ri = rsqrt64(z2), r = z2 * ri, d = A[q + q * kk].r - A[p + p * kk].r;
+            const double s2 = d * d + 4.0 * z2;
+            const double t = copysign(2.0 * r, d) * recip(fabs(d) + s2 * rsqrt64(s2));
+            cs = rsqrt64(1.0 + t * t);
+            sn = t * cs;
+            e = ri * cconj(z);
+          }
+        }
+        rc[tid] = cs;
+        rs[tid] = sn;
+        re[tid] = e;
+      }
+      __syncthreads();
+      // A <- J^H A J on the 2 x 2 blocks of pairs, V <- V J: an item's slots
+      // are fixed, its rows and columns follow from the round
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        if (itK[u] < 0) continue;
+        const int K = itK[u], s = first(K), t = second(K);
+        const double cK = rc[K], sK = rs[K];
+        const C<double> eK = re[K], z0 = czero<double>();
+        const bool ok_s = s < kk;
+        if (itP[u] >= 0) {
+          const int P = itP[u], p = first(P), q = second(P);
+          const bool ok_p = p < kk;
+          C<double> a = ok_p && ok_s ? A[p + s * kk] : z0, b = ok_p ? A[p + t * kk] : z0;
+          C<double> c = ok_s ? A[q + s * kk] : z0, d = A[q + t * kk];
+          // columns: s' = cs s - sn e t, t' = sn s + cs e t
+          const double cP = rc[P], sP = rs[P];
+          const C<double> eP = cconj(re[P]), eb = eK * b, ed = eK * d;
+          const C<double> a1 = cK * a - sK * eb, b1 = sK * a + cK * eb, c1 = cK * c - sK * ed, d1 = sK * c + cK * ed;
+          // rows: p' = cs p - sn conj(e) q, q' = sn p + cs conj(e) q
+          const C<double> ec = eP * c1, ef = eP * d1;
+          a = cP * a1 - sP * ec;
+          c = sP * a1 + cP * ec;
+          b = cP * b1 - sP * ef;
+          d = sP * b1 + cP * ef;
+          if (P == K) {
+            a.i = d.i = 0.0;
+            b = c = z0;
+          }
+          if (ok_p && ok_s) A[p + s * kk] = a;
+          if (ok_p) A[p + t * kk] = b;
+          if (ok_s) A[q + s * kk] = c;
+          A[q + t * kk] = d;
+        } else if (ok_s) {
+          const int i = -1 - itP[u];
+          const C<double> a = Vv[i + s * kk], b = eK * Vv[i + t * kk];
+          Vv[i + s * kk] = cK * a - sK * b;
+          Vv[i + t * kk] = sK * a + cK * b;
+        }
+      }
+      __syncthreads();
+    }
+  }
+  __syncthreads();
+  if (tid < kk) {
+    const double v = A[tid + tid * kk].r;
+    int r = 0;
+    for (int j = 0; j < kk; j++) {
+      const double u = A[j + j * kk].r;
+      r += u < v || (u == v && j < tid);
+    }
+    ord[r] = tid;
+    w[r] = v;
+  }
+  __syncthreads();
+  for (int i = tid; i < m; i += bd) lam[(size_t)prob * vpp + i] = w[i];
+  // X = L^-H Y for the lowest m (rows divided by the diagonal at the end)
+  for (int r = kk - 1; r >= 0; r--) {
+    __syncthreads();
+    const double inv = 1.0 / B[r + r * kk].r;
+    for (int j = tj; j < m; j += sj) {
+      C<double>* y = Vv + ord[j] * kk;
+      const C<double> f = inv * y[r];
+      for (int i = ti; i < r; i += 16) y[i] -= cconj(B[r + i * kk]) * f;
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < kk * m; e += bd) {
+    const int i = e / kk, t = e - i * kk, pos = keep[t], c = cl ? cl[1 + pos] : pos;
+    const C<double> z = (dsc[pos] / B[t + t * kk].r) * Vv[t + ord[i] * kk];
+    Cj[c + (size_t)i * k] = z;
+    if (basis && c >= m) Cj[c + (size_t)(m + i) * k] = z;
+  }
+  if (tid == 0) status[jb] = 0;
+}
+
 // ----------------------------------------------------------------- block combine
 // Per problem: out_j = sum_a C[a + j nin] in_a over nin input vectors, for
 // nout outputs, every input read once.  Output j goes to slot j of the
@@ -4274,7 +4555,10 @@ int mxh_init(void)
     e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     if (e != hipSuccess) return (int)e;
   }
-  if (grid_attrs()) return (int)hipErrorInvalidValue;
+  // (static LDS counts too)
+  e = hipFuncSetAttribute((const void*)k_ritz, hipFuncAttributeMaxDynamicSharedMemorySize,
+                          3 * sizeof(C<double>) * RITZ_MAX * RITZ_MAX);
+  if (e != hipSuccess || grid_attrs()) return (int)hipErrorInvalidValue;
   e = hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     g_stream = nullptr;
@@ -4976,6 +5260,20 @@ int mxh_gram_static(const mxh_level* lv, const mxh_bloch* bl, int nprob, const i
   if ((size_t)nprob > cap) return MXH_ESCRATCH;
   const int sets_cap = cap < (size_t)GRAM_SETS ? (int)cap : GRAM_SETS;
   return gram_launch(lv, bl, nprob, pmap, nullptr, m, u, eta64, out, g_scratch_ptr[g_device], sets_cap);
+}
+
+int mxh_ritz(int m, int basis, int nprob, const int* pmap, const int* cmap, const double* gram, double sk,
+             double pivot, double* Cm, double* lam, int vpp, int* status)
+{
+  const int k = basis ? basis : m;
+  if (m < 1 || k < m || k > RITZ_MAX || nprob < 1) return (int)hipErrorInvalidValue;
+  // threads: the items of a Jacobi round, k^2 / 4 blocks and k^2 / 2 rows, in at
+  // most two goes
+  hipLaunchKernelGGL(k_ritz, dim3(nprob), dim3(k <= 12 ? 128 : k <= 16 ? 256 : k <= 24 ? 512 : 1024),
+                     3 * sizeof(C<double>) * (size_t)k * k, g_stream, m, basis, pmap, cmap, gram, sk, pivot, Cm, lam,
+                     vpp, status);
+  LAUNCH_CHECK();
+  return 0;
 }
 
 int mxh_block_combine(long long n, int nprob, const int* pmap, int m, mxh_vecs u, mxh_vecs e, const double* Cm)
