@@ -18,6 +18,7 @@
 #include <assert.h>
 #include <math.h>
 #include <omp.h>
+#include <pthread.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -62,6 +63,7 @@ typedef struct {
   double *out;   /* small device result buffer */
   field *tmp;    /* scratch edge vector */
   size_t ntmp;
+  field *sweep;  /* the smoothers' second buffer (one edge vector), under sweep_lock */
 } griddev;
 
 static griddev *gdev(const grid2d *gr)
@@ -114,7 +116,8 @@ static mxh_coef coef(field a, field b)
 }
 
 static long long en(const edge2d *x) { return 2LL * x->gr->nx * x->gr->ny; }
-static long long nn(const node2d *x) { return (long long)x->gr->nx * x->gr->ny; }
+static long long nodes(const grid2d *gr) { return (long long)gr->nx * gr->ny; }
+static long long nn(const node2d *x) { return nodes(x->gr); }
 
 static field *scratch_edge(const grid2d *gr)
 {
@@ -253,6 +256,7 @@ void del_grid2d(grid2d *gr)
     mxh_free(g->work);
     mxh_free(g->out);
     mxh_free(g->tmp);
+    mxh_free(g->sweep);
     free(g);
   }
   free(gr->eps);
@@ -710,13 +714,19 @@ typedef struct {
   uint64_t sum;
   int n;
   double *dev;
+  double *inv;   /* inverse of the factored matrix, in room for nroom rows */
+  int nroom, inv_valid;
 } factor_cache;
 
-static uint64_t fnv(const void *p, size_t bytes)
+/* FNV-1a over 64-bit words (n even: complex doubles) */
+static uint64_t fnv(const void *p, size_t words)
 {
-  const unsigned char *c = (const unsigned char *)p;
-  uint64_t h = 1469598103934665603ULL;
-  for (size_t k = 0; k < bytes; k++) h = (h ^ c[k]) * 1099511628211ULL;
+  uint64_t h = 1469598103934665603ULL, w;
+  for (size_t k = 0; k < words; k++) {
+    memcpy(&w, (const char *)p + 8 * k, 8);
+    h = (h ^ w) * 1099511628211ULL;
+    h ^= h >> 32;
+  }
   return h;
 }
 
@@ -724,7 +734,7 @@ static const double *device_factor(factor_cache *fc, const matrix *A)
 {
   field *p = packed(A);
   size_t bytes = sizeof(field) * (size_t)A->rows * A->rows;
-  uint64_t h = fnv(p, bytes);
+  uint64_t h = fnv(p, bytes / 8);
   if (fc->key != A || fc->sum != h || fc->n != A->rows) {
     if (fc->n != A->rows) {
       mxh_free(fc->dev);
@@ -735,12 +745,93 @@ static const double *device_factor(factor_cache *fc, const matrix *A)
     fc->key = A;
     fc->sum = h;
     fc->n = A->rows;
+    fc->inv_valid = 0;
   }
   if (p != A->a) free(p);
   return fc->dev;
 }
 
+static const double *device_inverse(factor_cache *fc, const matrix *A)
+{
+  const double *L = device_factor(fc, A);
+  if (!fc->inv_valid) {
+    if (fc->nroom < A->rows) {
+      mxh_free(fc->inv);
+      fc->inv = (double *)mxh_malloc(sizeof(field) * (size_t)A->rows * A->rows);
+      if (!fc->inv) die("factor allocation", 0);
+      fc->nroom = A->rows;
+    }
+    HIPCK(mxh_coarse_inverse(A->rows, 1, L, fc->inv));
+    fc->inv_valid = 1;
+  }
+  return fc->inv;
+}
+
 static factor_cache edge_fc, node_fc;
+
+/* ---- V-cycles through the fused smoothers: a level's sweeps, its residual
+   and restriction (down) or prolongation (up) in passes of at most two sweeps
+   that alternate between x and the grid's second buffer, and the levels of at
+   most 32 x 32 nodes in one launch (mxh_edge_cycle, mxh_node_cycle).  A cycle
+   of one vector is bound by launches and their latency: of 108 launches of an
+   edge cycle on 256 x 256 with 4 x 4 coarse nodes 39 remain, of a node cycle 7.
+   The operators, the order of the sweeps and every level's b and x on return
+   are those of one launch per colour, which stays for nu < 1 and for edge
+   levels above 64 x 64: the square tiles smooth copies of the nodes across the
+   periodic boundary, which round differently there, and that excites gradient
+   fields (a step on 256 x 256: error 6e-11 against 3e-12; 18 launches of a
+   level 60 us, two passes 40). */
+#define EDGE_PASS_MAX 4096 /* nodes mxh_afw_tile keeps whole in LDS */
+typedef struct {
+  int fused;   /* the passes below can be used */
+  int lc;      /* levels 0 .. lc in one launch (< 1: level 0 by itself) */
+  mxh_cycle cy;
+  const double *W;
+} cycle_plan;
+
+/* the second buffers are shared by every vector of a grid: held over the
+   launches of a cycle (the library's stream then runs them in order) */
+static pthread_mutex_t sweep_lock = PTHREAD_MUTEX_INITIALIZER;
+
+static field *sweep_buffer(const grid2d *gr)
+{
+  griddev *g = gdev(gr);
+  if (!g->sweep) g->sweep = (field *)mxh_malloc(sizeof(field) * 2 * (size_t)gr->nx * gr->ny);
+  if (!g->sweep) die("scratch allocation", 0);
+  return g->sweep;
+}
+
+/* grids and vectors of levels 0 .. L (comp components per node) */
+static void plan_cycle(cycle_plan *p, int L, int nu, const matrix *Ac, int comp, factor_cache *fc,
+                       const grid2d *(*grid)(void **, int), field *(*data)(void **, int), void **b, void **x)
+{
+  memset(p, 0, sizeof(*p));
+  p->lc = -1;
+  p->fused = nu > 0 && L > 0;
+  for (int l = 0; l <= L && p->fused; l++) {
+    const grid2d *g = grid(x, l), *h = grid(b, l);
+    if (h->nx != g->nx || h->ny != g->ny) p->fused = 0;
+    if (l && (g->nx != 2 * grid(x, l - 1)->nx || g->ny != 2 * grid(x, l - 1)->ny)) p->fused = 0;
+  }
+  if (!p->fused || !Ac || Ac->rows != comp * grid(x, 0)->nx * grid(x, 0)->ny || Ac->rows > 256) return;
+  for (int l = 0; l <= L && l < MXH_CYCLE_MAXL; l++) {
+    const grid2d *g = grid(x, l);
+    if (g->xfactor != grid(x, 0)->xfactor || g->yfactor != grid(x, 0)->yfactor) break;
+    mxh_cycle t = p->cy;
+    t.n = l + 1;
+    t.lv[l] = level_of(g);
+    t.eta[l] = gdev(g)->eta;
+    t.b[l] = t.x[l] = NULL;
+    if (l) {
+      t.b[l - 1] = data(b, l - 1);
+      t.x[l - 1] = data(x, l - 1);
+    }
+    if (l && !mxh_cycle_supported(MXH_F64, &t)) break;
+    p->cy = t;
+    p->lc = l;
+  }
+  if (p->lc > 0) p->W = device_inverse(fc, Ac);
+}
 
 /* x = Ac^{-1} b on the coarsest level with the Cholesky factor in Ac
    (potrf_matrix output) */
@@ -760,16 +851,56 @@ static void edge_coarse_solve(const matrix *Ac, const edge2d *b, edge2d *x)
   }
 }
 
-static void vcycle_edge_impl(int L, int nu, const matrix *Ac, edge2d **b, edge2d **x)
+static const grid2d *edge_grid(void **v, int l) { return ((edge2d **)v)[l]->gr; }
+static field *edge_data(void **v, int l) { return ((edge2d **)v)[l]->x; }
+
+static void plan_edge(cycle_plan *p, int L, int nu, const matrix *Ac, edge2d **b, edge2d **x)
 {
-  for (int l = L; l > 0; l--) {
+  plan_cycle(p, L, nu, Ac, 2, &edge_fc, edge_grid, edge_data, (void **)b, (void **)x);
+}
+
+/* one level's way down (to < l: nu forward sweeps, residual, restriction) or up
+   (prolongation, nu backward sweeps) */
+static void edge_passes(int nu, int up, int xzero, const edge2d *b, edge2d *x, edge2d *bc, edge2d *xc)
+{
+  const mxh_level lv = level_of(x->gr);
+  const mxh_bloch bl = bloch_of(x->gr);
+  const long long n = en(x), nc = en(xc);
+  const mxh_vecs none = VV(NULL, 0);
+  /* the way down starts at x, the way up where that ended: after an even number of passes in all, at x */
+  const int passes = (nu + 1) / 2;
+  field *buf[2] = {x->x, sweep_buffer(x->gr)};
+  int cur = up ? passes & 1 : 0;
+  for (int i = 0; i < passes; i++, cur ^= 1) {
+    const int first = i == 0, last = i == passes - 1, sweeps = last ? nu - 2 * i : 2;
+    const int mode = up ? 1 + (first ? 4 : 0) : (first && xzero ? 2 : 0) + (last ? 8 : 0);
+    HIPCK(mxh_afw_tile(MXH_F64, &lv, &bl, 1, VV(b->x, n), VV(buf[cur], n), VV(buf[cur ^ 1], n), gdev(x->gr)->eta,
+                       sweeps, mode, mode & 4 ? VV(xc->x, nc) : none, mode & 8 ? VV(bc->x, nc) : none,
+                       mode & 8 ? VV(xc->x, nc) : none));
+  }
+}
+
+static void vcycle_edge_impl(int L, int nu, const matrix *Ac, edge2d **b, edge2d **x, const cycle_plan *p, int xzero)
+{
+  if (xzero && (!p->fused || nodes(x[L]->gr) > EDGE_PASS_MAX)) HIPCK(mxh_memset(x[L]->x, 0, sizeof(field) * en(x[L])));
+  const int lc = p->lc > 0 ? p->lc : 0;
+  if (p->fused) pthread_mutex_lock(&sweep_lock);
+  for (int l = L; l > lc; l--) {
+    if (p->fused && nodes(x[l]->gr) <= EDGE_PASS_MAX) {
+      edge_passes(nu, 0, xzero && l == L, b[l], x[l], b[l - 1], x[l - 1]);
+      continue;
+    }
     for (int i = 0; i < nu; i++) gs_edge(1.0, 1.0, b[l], x[l], 0);
     mxh_level lv = level_of(x[l]->gr);
     mxh_bloch bl = bloch_of(x[l]->gr);
     HIPCK(mxh_resid_restrict(MXH_F64, &lv, &bl, 1, VV(b[l]->x, en(b[l])), VV(x[l]->x, en(x[l])),
                              gdev(x[l]->gr)->eta, VV(b[l - 1]->x, en(b[l - 1])), VV(x[l - 1]->x, en(x[l - 1]))));
   }
-  if (Ac) {
+  if (lc > 0) {
+    const mxh_bloch bl = bloch_of(x[lc]->gr);
+    HIPCK(mxh_edge_cycle(MXH_F64, &p->cy, &bl, 1, nu, VV(b[lc]->x, en(b[lc])), VV(x[lc]->x, en(x[lc])),
+                         lc < L || xzero, p->W, 0));
+  } else if (Ac) {
     edge_coarse_solve(Ac, b[0], x[0]);
   } else {
     for (int i = 0; i < nu; i++) {
@@ -777,17 +908,26 @@ static void vcycle_edge_impl(int L, int nu, const matrix *Ac, edge2d **b, edge2d
       gs_edge(1.0, 1.0, b[0], x[0], 1);
     }
   }
-  for (int l = 1; l <= L; l++) {
+  for (int l = lc + 1; l <= L; l++) {
+    if (p->fused && nodes(x[l]->gr) <= EDGE_PASS_MAX) {
+      edge_passes(nu, 1, 0, b[l], x[l], b[l - 1], x[l - 1]);
+      continue;
+    }
     prolong_edge_impl(1.0, x[l - 1], x[l]);
     for (int i = 0; i < nu; i++) gs_edge(1.0, 1.0, b[l], x[l], 1);
   }
+  if (p->fused) pthread_mutex_unlock(&sweep_lock);
 }
 
 void vcycle_edge2d(int L, int nu, const matrix *Ac, edge2d **b, edge2d **x, edge2d **d)
 {
   (void)d; /* residuals are formed inside the restriction kernel */
 #pragma omp single
-  vcycle_edge_impl(L, nu, Ac, b, x);
+  {
+    cycle_plan p;
+    plan_edge(&p, L, nu, Ac, b, x);
+    vcycle_edge_impl(L, nu, Ac, b, x, &p, 0);
+  }
 }
 
 /* ---- pointwise edge Gauss-Seidel (edge2d.c:3892-5600).  The reference
@@ -1228,17 +1368,53 @@ void adjgradient_node2d(field alpha, const edge2d *x, node2d *y)
   }
 }
 
-static void vcycle_node_impl(int L, int nu, const matrix *Ac, node2d **b, node2d **x)
+static const grid2d *node_grid(void **v, int l) { return ((node2d **)v)[l]->gr; }
+static field *node_data(void **v, int l) { return ((node2d **)v)[l]->v; }
+
+static void plan_node(cycle_plan *p, int L, int nu, const matrix *Ac, node2d **b, node2d **x)
 {
-  for (int l = L; l > 0; l--) {
+  plan_cycle(p, L, nu, Ac, 1, &node_fc, node_grid, node_data, (void **)b, (void **)x);
+}
+
+static void node_passes(int nu, int up, const node2d *b, node2d *x, node2d *bc, node2d *xc)
+{
+  const mxh_level lv = level_of(x->gr);
+  const mxh_bloch bl = bloch_of(x->gr);
+  const long long n = nn(x), nc = nn(xc);
+  const mxh_vecs none = VV(NULL, 0);
+  const int passes = (nu + 1) / 2;
+  field *buf[2] = {x->v, sweep_buffer(x->gr)};
+  int cur = up ? passes & 1 : 0;
+  for (int i = 0; i < passes; i++, cur ^= 1) {
+    const int first = i == 0, last = i == passes - 1, sweeps = last ? nu - 2 * i : 2;
+    const int mode = up ? 1 + (first ? 4 : 0) : (last ? 8 : 0);
+    HIPCK(mxh_node_tile(MXH_F64, &lv, &bl, 1, VV(b->v, n), VV(buf[cur], n), VV(buf[cur ^ 1], n), sweeps, mode,
+                        mode & 4 ? VV(xc->v, nc) : none, mode & 8 ? VV(bc->v, nc) : none,
+                        mode & 8 ? VV(xc->v, nc) : none));
+  }
+}
+
+static void vcycle_node_impl(int L, int nu, const matrix *Ac, node2d **b, node2d **x, const cycle_plan *p)
+{
+  const int lc = p->lc > 0 ? p->lc : 0;
+  if (p->fused) pthread_mutex_lock(&sweep_lock);
+  for (int l = L; l > lc; l--) {
+    if (p->fused) {
+      node_passes(nu, 0, b[l], x[l], b[l - 1], x[l - 1]);
+      continue;
+    }
     for (int i = 0; i < nu; i++) gs_node(1.0, b[l], x[l], 0);
     mxh_level lv = level_of(x[l]->gr);
     mxh_bloch bl = bloch_of(x[l]->gr);
     HIPCK(mxh_node_resid_restrict(MXH_F64, &lv, &bl, 1, VV(b[l]->v, nn(b[l])), VV(x[l]->v, nn(x[l])),
                                   VV(b[l - 1]->v, nn(b[l - 1])), VV(x[l - 1]->v, nn(x[l - 1]))));
   }
-  if (Ac) {
-    assert(Ac->rows == x[0]->gr->nx * x[0]->gr->ny);
+  if (Ac) assert(Ac->rows == x[0]->gr->nx * x[0]->gr->ny);
+  if (lc > 0) {
+    const mxh_bloch bl = bloch_of(x[lc]->gr);
+    HIPCK(mxh_node_cycle(MXH_F64, &p->cy, &bl, 1, nu, VV(b[lc]->v, nn(b[lc])), VV(x[lc]->v, nn(x[lc])), lc < L, p->W,
+                         0));
+  } else if (Ac) {
     if (Ac->rows <= 256) {
       const double *L0 = device_factor(&node_fc, Ac);
       HIPCK(mxh_coarse_solve(MXH_F64, Ac->rows, L0, NULL, 1, NULL, 1, VV(b[0]->v, nn(b[0])), VV(x[0]->v, nn(x[0]))));
@@ -1256,19 +1432,28 @@ static void vcycle_node_impl(int L, int nu, const matrix *Ac, node2d **b, node2d
       gs_node(1.0, b[0], x[0], 1);
     }
   }
-  for (int l = 1; l <= L; l++) {
+  for (int l = lc + 1; l <= L; l++) {
+    if (p->fused) {
+      node_passes(nu, 1, b[l], x[l], b[l - 1], x[l - 1]);
+      continue;
+    }
     mxh_level lv = level_of(x[l]->gr);
     mxh_bloch bl = bloch_of(x[l]->gr);
     HIPCK(mxh_node_prolong(MXH_F64, &lv, &bl, 1, VV(x[l - 1]->v, nn(x[l - 1])), VV(x[l]->v, nn(x[l])), 1.0, 0.0));
     for (int i = 0; i < nu; i++) gs_node(1.0, b[l], x[l], 1);
   }
+  if (p->fused) pthread_mutex_unlock(&sweep_lock);
 }
 
 void vcycle_node2d(int L, int nu, const matrix *Ac, node2d **b, node2d **x, node2d **d)
 {
   (void)d;
 #pragma omp single
-  vcycle_node_impl(L, nu, Ac, b, x);
+  {
+    cycle_plan p;
+    plan_node(&p, L, nu, Ac, b, x);
+    vcycle_node_impl(L, nu, Ac, b, x, &p);
+  }
 }
 
 /* ---- conjugate gradients for the Q1 Laplacian preconditioned by one nodal
@@ -1333,13 +1518,16 @@ void pinvit_edge2d(int l, int smoother_steps, int prec_steps, int gradient_steps
     mxh_coef cf = coef(1.0, 1.0 - lambda);
     const long long n = en(e), N = n / 2;
     HIPCK(mxh_addeval(MXH_F64, &lv, &bl, 1, VV(e->x, n), VV(b[l]->x, n), gdev(gr)->eta, &cf, 0));
-    HIPCK(mxh_memset(x[l]->x, 0, sizeof(field) * n));
-    for (int j = 0; j < prec_steps; j++) vcycle_edge_impl(l, smoother_steps, Ae, b, x);
+    cycle_plan pe, pn;
+    plan_edge(&pe, l, smoother_steps, Ae, b, x);
+    plan_node(&pn, l, smoother_steps, An, bg, xg);
+    if (prec_steps < 1) HIPCK(mxh_memset(x[l]->x, 0, sizeof(field) * n));
+    for (int j = 0; j < prec_steps; j++) vcycle_edge_impl(l, smoother_steps, Ae, b, x, &pe, j == 0);
     /* lifting right-hand side of u = e - x, then e <- u - G xg in place (u
        is formed from e and x by both kernels, never stored) */
     HIPCK(mxh_lift_rhs(MXH_F64, &lv, &bl, 1, VV(e->x, n), VV(x[l]->x, n), VV(NULL, n), VV(bg[l]->v, N),
                        VV(xg[l]->v, N), NULL, NULL));
-    for (int j = 0; j < gradient_steps; j++) vcycle_node_impl(l, smoother_steps, An, bg, xg);
+    for (int j = 0; j < gradient_steps; j++) vcycle_node_impl(l, smoother_steps, An, bg, xg, &pn);
     HIPCK(mxh_lift_apply(MXH_F64, &lv, &bl, 1, VV(xg[l]->v, N), VV(e->x, n), VV(x[l]->x, n), VV(e->x, n), -1.0,
                          NULL, NULL));
   }

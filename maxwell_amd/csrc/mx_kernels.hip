@@ -3495,12 +3495,51 @@ __global__ __launch_bounds__(256, 2) void k_edge_cycle(CycleLevels cl, mxh_bloch
 }
 
 // W[r n + c] = (A^-1)[r, c] from the Cholesky factor L of A (n x n,
-// column-major, per problem): one workgroup per problem, one thread per column
-// c, forward and back substitution.  work: W itself holds the running column.
+// column-major, per problem): one workgroup per problem, forward and back
+// substitution of the unit vectors.  n <= COARSE_LDS_N: L and W in LDS, a row's
+// multiples leave all other rows at once, one barrier a row (a chain of 2 n
+// barriers).  Larger: one thread per column, W itself holds the running column.
+#define COARSE_LDS_N 64
 __global__ __launch_bounds__(256) void k_coarse_inverse(int n, const double* L0, double* W0)
 {
+  extern __shared__ double smem[];
   const C<double>* L = (const C<double>*)L0 + (size_t)blockIdx.x * n * n;
   C<double>* W = (C<double>*)W0 + (size_t)blockIdx.x * n * n;
+  if (n <= COARSE_LDS_N) {
+    C<double>*l = (C<double>*)smem, *w = l + n * n;
+    const int tc = threadIdx.x & 15, tr = threadIdx.x >> 4, nr = blockDim.x >> 4;
+    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
+      l[e] = L[e];
+      w[e] = cmk(e / n == e % n ? 1.0 : 0.0, 0.0);
+    }
+    for (int k = 0; k < n; k++) {
+      __syncthreads();
+      const double inv = 1.0 / l[k + k * n].r;
+      for (int r = k + 1 + tr; r < n; r += nr) {
+        const C<double> f = inv * l[r + k * n];
+        for (int c = tc; c <= k; c += 16) w[r * n + c] -= f * w[k * n + c];
+      }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
+      const int r = e / n;
+      w[e] = (1.0 / l[r + r * n].r) * w[e];
+    }
+    for (int k = n - 1; k >= 0; k--) {
+      __syncthreads();
+      const double inv = 1.0 / l[k + k * n].r;
+      for (int r = tr; r < k; r += nr) {
+        const C<double> f = inv * cconj(l[k + r * n]);
+        for (int c = tc; c < n; c += 16) w[r * n + c] -= f * w[k * n + c];
+      }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
+      const int r = e / n;
+      W[e] = (1.0 / l[r + r * n].r) * w[e];
+    }
+    return;
+  }
   const int c = threadIdx.x;
   if (c >= n) return;
   for (int r = 0; r < n; r++) {
@@ -4550,7 +4589,8 @@ int mxh_init(void)
                        (const void*)k_fft_rows<double, -1>, (const void*)k_fft_rows<double, 1>,
                        (const void*)k_fft_rows<float, -1>, (const void*)k_fft_rows<float, 1>,
                        (const void*)k_edge_cycle<double>, (const void*)k_edge_cycle<float>,
-                       (const void*)k_node_cycle<double>, (const void*)k_node_cycle<float>};
+                       (const void*)k_node_cycle<double>, (const void*)k_node_cycle<float>,
+                       (const void*)k_coarse_inverse};
   for (const void* f : big) {
     e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     if (e != hipSuccess) return (int)e;
@@ -4855,7 +4895,9 @@ int mxh_cycle_supported(int prec, const mxh_cycle* cy)
 int mxh_coarse_inverse(int n, int nprob, const double* L, double* W)
 {
   if (n < 1 || n > 256 || nprob < 1) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_coarse_inverse, dim3(nprob), dim3((n + 63) / 64 * 64), 0, g_stream, n, L, W);
+  const bool lds = n <= COARSE_LDS_N;
+  hipLaunchKernelGGL(k_coarse_inverse, dim3(nprob), dim3(lds ? 256 : (n + 63) / 64 * 64),
+                     lds ? 2 * sizeof(C<double>) * n * n : 0, g_stream, n, L, W);
   LAUNCH_CHECK();
   return 0;
 }
