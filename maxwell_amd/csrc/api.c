@@ -116,8 +116,7 @@ static mxh_coef coef(field a, field b)
 }
 
 static long long en(const edge2d *x) { return 2LL * x->gr->nx * x->gr->ny; }
-static long long nodes(const grid2d *gr) { return (long long)gr->nx * gr->ny; }
-static long long nn(const node2d *x) { return nodes(x->gr); }
+static long long nn(const node2d *x) { return (long long)x->gr->nx * x->gr->ny; }
 
 static field *scratch_edge(const grid2d *gr)
 {
@@ -773,15 +772,10 @@ static factor_cache edge_fc, node_fc;
    and restriction (down) or prolongation (up) in passes of at most two sweeps
    that alternate between x and the grid's second buffer, and the levels of at
    most 32 x 32 nodes in one launch (mxh_edge_cycle, mxh_node_cycle).  A cycle
-   of one vector is bound by launches and their latency: of 108 launches of an
-   edge cycle on 256 x 256 with 4 x 4 coarse nodes 39 remain, of a node cycle 7.
-   The operators, the order of the sweeps and every level's b and x on return
-   are those of one launch per colour, which stays for nu < 1 and for edge
-   levels above 64 x 64: the square tiles smooth copies of the nodes across the
-   periodic boundary, which round differently there, and that excites gradient
-   fields (a step on 256 x 256: error 6e-11 against 3e-12; 18 launches of a
-   level 60 us, two passes 40). */
-#define EDGE_PASS_MAX 4096 /* nodes mxh_afw_tile keeps whole in LDS */
+   of one vector is bound by launches and their latency: of 108 launches on 256 x
+   256 with 4 x 4 coarse nodes 7 remain.  The operators, the order of the sweeps
+   and every level's b and x on return are those of one launch per colour, which
+   stays for nu < 1. */
 typedef struct {
   int fused;   /* the passes below can be used */
   int lc;      /* levels 0 .. lc in one launch (< 1: level 0 by itself) */
@@ -882,11 +876,11 @@ static void edge_passes(int nu, int up, int xzero, const edge2d *b, edge2d *x, e
 
 static void vcycle_edge_impl(int L, int nu, const matrix *Ac, edge2d **b, edge2d **x, const cycle_plan *p, int xzero)
 {
-  if (xzero && (!p->fused || nodes(x[L]->gr) > EDGE_PASS_MAX)) HIPCK(mxh_memset(x[L]->x, 0, sizeof(field) * en(x[L])));
+  if (xzero && !p->fused) HIPCK(mxh_memset(x[L]->x, 0, sizeof(field) * en(x[L])));
   const int lc = p->lc > 0 ? p->lc : 0;
   if (p->fused) pthread_mutex_lock(&sweep_lock);
   for (int l = L; l > lc; l--) {
-    if (p->fused && nodes(x[l]->gr) <= EDGE_PASS_MAX) {
+    if (p->fused) {
       edge_passes(nu, 0, xzero && l == L, b[l], x[l], b[l - 1], x[l - 1]);
       continue;
     }
@@ -909,7 +903,7 @@ static void vcycle_edge_impl(int L, int nu, const matrix *Ac, edge2d **b, edge2d
     }
   }
   for (int l = lc + 1; l <= L; l++) {
-    if (p->fused && nodes(x[l]->gr) <= EDGE_PASS_MAX) {
+    if (p->fused) {
       edge_passes(nu, 1, 0, b[l], x[l], b[l - 1], x[l - 1]);
       continue;
     }

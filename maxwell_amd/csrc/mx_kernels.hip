@@ -2897,13 +2897,14 @@ __global__ __launch_bounds__((R / 2) * (R / 2)) __attribute__((amdgpu_waves_per_
 // ----------------------------------------------------------------- tile-fused nodal GS
 // The nodal counterpart of k_afw_tile: pointwise Gauss-Seidel for the Q1
 // Laplacian in four colours; a sweep moves the exact region inward by 4.
-// x and b of the R x R region (R = 64) live in LDS.
-template <typename T, int MODE>
-__global__ __launch_bounds__(1024) void k_node_tile(mxh_level lv, mxh_bloch bl, const C<T>* B, long long bs,
+// x and b of the R x R region live in LDS.  R = 64, and FEW_R where a launch has
+// few tiles (as k_afw_few).
+#define FEW_R 32
+template <typename T, int MODE, int R>
+__global__ __launch_bounds__(R* R / 4) void k_node_tile(mxh_level lv, mxh_bloch bl, const C<T>* B, long long bs,
                                                     const C<T>* Xin, C<T>* Xout, long long xs, int nsweep,
                                                     const C<T>* XCin, C<T>* BC, C<T>* XC, long long cs, int ntx)
 {
-  constexpr int R = 64;
   __shared__ C<T> sx[R * R];
   __shared__ C<T> sb[R * R];
   const int v = blockIdx.y;
@@ -3019,11 +3020,18 @@ __global__ __launch_bounds__(1024) void k_node_tile(mxh_level lv, mxh_bloch bl, 
 // across the boundary.  What bounds it: vector issue of the patch solves at 64^2,
 // the latency of the phases on smaller grids.  192 vectors of 64^2 in FP64, two
 // sweeps and prolongation: 58.6 -> 34.9 us (square tiles before).
+MXH_DEV int wrap_index(int i, int n)
+{
+  i %= n;
+  return i < 0 ? i + n : i;
+}
+
 template <typename T>
 struct GridBlock {
   int hx, hy, I, J;       // blocks per side, this thread's block
   int co[4], go[4];       // columns 2I - 1 .. 2I + 2: LDS offset, natural index
-  int ro[4];              // rows 2J - 1 .. 2J + 2, times nx
+  int ro[4], gr[4];       // rows 2J - 1 .. 2J + 2: LDS offset, times nx
+  bool wl, wr, wd, wu;    // the left, right, lower, upper neighbour lies across the boundary
   C<T> xf, yf;
 
   MXH_DEV void set(int nx, int ny, int block)
@@ -3045,17 +3053,52 @@ struct GridBlock {
     ro[1] = 2 * J * nx;
     ro[2] = (2 * J + 1) * nx;
     ro[3] = (J + 1 < hy ? 2 * J + 2 : 0) * nx;
+#pragma unroll
+    for (int a = 0; a < 4; a++) gr[a] = ro[a];
+    wl = I == 0;
+    wr = I == hx - 1;
+    wd = J == 0;
+    wu = J == hy - 1;
+  }
+  // block (I, J) of a region of R x R nodes whose first is (ox, oy), even, of the
+  // periodic nx x ny grid; the region's rim has no patches
+  template <int R>
+  MXH_DEV void set_tile(int nx, int ny, int ox, int oy, int block)
+  {
+    constexpr int H = R / 2;
+    hx = hy = H;
+    J = block / H;
+    I = block - J * H;
+    co[0] = H + max(I - 1, 0);
+    co[1] = I;
+    co[2] = H + I;
+    co[3] = min(I + 1, H - 1);
+#pragma unroll
+    for (int a = 0; a < 4; a++) ro[a] = min(max(2 * J - 1 + a, 0), R - 1) * R;
+    const int x = wrap_index(ox + 2 * I, nx), y = wrap_index(oy + 2 * J, ny);
+    wl = x == 0;
+    wr = x == nx - 2;
+    wd = y == 0;
+    wu = y == ny - 2;
+    go[0] = wl ? nx - 1 : x - 1;
+    go[1] = x;
+    go[2] = x + 1;
+    go[3] = wr ? 0 : x + 2;
+    gr[0] = (wd ? ny - 1 : y - 1) * nx;
+    gr[1] = y * nx;
+    gr[2] = (y + 1) * nx;
+    gr[3] = (wu ? 0 : y + 2) * nx;
   }
   // value at node (2I + DI, 2J + DJ) of an array in LDS (parity-split columns)
   // or, GL, in memory
   template <int DI, int DJ, bool GL = false>
   MXH_DEV C<T> get(const C<T>* s) const
   {
-    C<T> v = s[(GL ? go[DI + 1] : co[DI + 1]) + ro[DJ + 1]];
-    if (DI == -1 && I == 0) v = cconj(xf) * v;
-    if (DI == 2 && I == hx - 1) v = xf * v;
-    if (DJ == -1 && J == 0) v = cconj(yf) * v;
-    if (DJ == 2 && J == hy - 1) v = yf * v;
+    C<T> v = s[GL ? go[DI + 1] + gr[DJ + 1] : co[DI + 1] + ro[DJ + 1]];
+    if (DI == -1 && wl) v = cconj(xf) * v;
+    if (DI == 2 && wr) v = xf * v;
+    if (DJ == -1 && wd) v = cconj(yf) * v;
+    if (DJ == 2 && wu) v = yf * v;
     return v;
   }
   // the stored value of node (2I + DI, 2J + DJ), which get() returned as v,
@@ -3064,7 +3107,7 @@ struct GridBlock {
   MXH_DEV void put(C<T>* s, C<T> v, C<T> d) const
   {
     C<T>* p = s + co[DI + 1] + ro[DJ + 1];
-    const bool wx = DI == -1 && I == 0, wy = DJ == -1 && J == 0;
+    const bool wx = DI == -1 && wl, wy = DJ == -1 && wd;
     if (wx) d = xf * d;
     if (wy) d = yf * d;
     *p = wx || wy ? *p + d : v + d;
@@ -3078,7 +3121,7 @@ MXH_DEV void grid_eta(const GridBlock<T>& g, const T* eta, T axy, T er[3][3])
 #pragma unroll
   for (int a = 0; a < 3; a++)
 #pragma unroll
-    for (int b = 0; b < 3; b++) er[a][b] = axy * eta[g.go[a] + g.ro[b]];
+    for (int b = 0; b < 3; b++) er[a][b] = axy * eta[g.go[a] + g.gr[b]];
 }
 
 // The AFW patch of node (2I + CI, 2J + CJ); b in LDS or, BG, in memory.
@@ -3223,8 +3266,8 @@ MXH_DEV void grid_restrict_lent(const GridBlock<T>& g, bool act, const C<T>* px,
 template <typename T>
 MXH_DEV void grid_prolong(const GridBlock<T>& g, C<T>* sx, C<T>* sy, C<T> c0, C<T> c1, C<T> d0, C<T> d1)
 {
-  if (g.J == g.hy - 1) c1 = g.yf * c1;
-  if (g.I == g.hx - 1) d1 = g.xf * d1;
+  if (g.wu) c1 = g.yf * c1;
+  if (g.wr) d1 = g.xf * d1;
   const C<T> h = T(0.5) * c0, q = T(0.25) * (c0 + c1), u = T(0.5) * d0, w = T(0.25) * (d0 + d1);
   sx[g.co[1] + g.ro[1]] += h;
   sx[g.co[2] + g.ro[1]] += h;
@@ -3243,7 +3286,7 @@ MXH_DEV void grid_copy_in(const GridBlock<T>& g, C<T>* s, const C<T>* a)
 #pragma unroll
   for (int b = 1; b < 3; b++)
 #pragma unroll
-    for (int c = 1; c < 3; c++) s[g.co[c] + g.ro[b]] = a ? a[g.go[c] + g.ro[b]] : czero<T>();
+    for (int c = 1; c < 3; c++) s[g.co[c] + g.ro[b]] = a ? a[g.go[c] + g.gr[b]] : czero<T>();
 }
 template <typename T>
 MXH_DEV void grid_copy_out(const GridBlock<T>& g, const C<T>* s, C<T>* a)
@@ -3251,7 +3294,7 @@ MXH_DEV void grid_copy_out(const GridBlock<T>& g, const C<T>* s, C<T>* a)
 #pragma unroll
   for (int b = 1; b < 3; b++)
 #pragma unroll
-    for (int c = 1; c < 3; c++) a[g.go[c] + g.ro[b]] = s[g.co[c] + g.ro[b]];
+    for (int c = 1; c < 3; c++) a[g.go[c] + g.gr[b]] = s[g.co[c] + g.ro[b]];
 }
 
 template <typename T> struct GridCfg;
@@ -3322,6 +3365,87 @@ __global__ __launch_bounds__(TB) void k_afw_grid(mxh_level lv, mxh_bloch bl, con
         xc[kc[q]] = czero<T>();
         xc[NC + kc[q]] = czero<T>();
       }
+    }
+  }
+}
+
+// The passes of k_afw_tile for launches that leave most of the chip idle (a
+// vector or a few): regions of 32 x 32 with 12 x 12 owned nodes, one patch per
+// thread and colour and one wave per SIMD, so that a launch is as short as its
+// chain of eight phases allows (two sweeps of a vector of 128^2 in FP64 10 us,
+// the larger tiles 17).  Copies of nodes across the boundary keep the values of the nodes they copy -- the
+// Bloch phase is applied where a patch reaches over it, as in k_afw_grid -- so
+// every copy is the same to the last bit and the residuals of a cell's edges
+// see one curl: with copies in the tile's frame the difference in rounding
+// excites gradient fields (error of a PINVIT step 6e-11 instead of 3e-12).
+#define FEW_T (FEW_R - 2 * TILE_H)
+template <typename T, int MODE>
+__global__ __launch_bounds__(FEW_R* FEW_R / 4) void k_afw_few(mxh_level lv, mxh_bloch bl, const C<T>* B, long long bs,
+                                                             const C<T>* Xin, C<T>* Xout, long long xs, const T* eta,
+                                                             int nsweep, const C<T>* XCin, C<T>* BC, C<T>* XC,
+                                                             long long cs, int ntx)
+{
+  constexpr int R = FEW_R, H = R / 2;
+  __shared__ C<T> sx[R * R], sy[R * R], px[H * H], py[H * H];
+  const int v = blockIdx.y, nx = lv.nx, ny = lv.ny, tid = threadIdx.x;
+  const size_t N = (size_t)nx * ny, NC = N >> 2;
+  const int tileX = blockIdx.x % ntx, tileY = blockIdx.x / ntx;
+  const int ox = tileX * FEW_T - TILE_H, oy = tileY * FEW_T - TILE_H;
+  const Geo<T> geo = make_geo<T>(lv, bl, v);
+  const C<T>*bx = B + (size_t)v * bs, *by = bx + N;
+  const T mx = T(lv.hy / lv.hx / 6.0), my = T(lv.hx / lv.hy / 6.0);
+  GridBlock<T> g;
+  g.xf = geo.xf;
+  g.yf = geo.yf;
+  g.template set_tile<R>(nx, ny, ox, oy, tid);
+  T er[3][3];
+  grid_eta(g, eta, T(1.0 / (lv.hx * lv.hy)), er);
+  const C<T>* x = (MODE & 2) ? nullptr : Xin + (size_t)v * xs;
+  grid_copy_in(g, sx, x);
+  grid_copy_in(g, sy, x ? x + N : nullptr);
+  const int GI = g.go[1] >> 1, GJ = g.gr[1] / (2 * nx), cnx = nx >> 1;
+  if (MODE & 4) {
+    const C<T>*cx = XCin + (size_t)v * cs, *cy = cx + NC;
+    const int k = GI + GJ * cnx;
+    grid_prolong(g, sx, sy, cx[k], cx[g.wu ? GI : k + cnx], cy[k], cy[g.wr ? GJ * cnx : k + 1]);
+  }
+  __syncthreads();
+  const bool l = g.I > 0, d = g.J > 0;
+  for (int s = 0; s < nsweep; s++)
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      switch ((MODE & 1) ? 3 - k : k) {
+      case 0: if (l && d) grid_patch<0, 0, true, false>(g, sx, sy, bx, by, er, mx, my); break;
+      case 1: if (g.I < H - 1 && d) grid_patch<1, 0, true, false>(g, sx, sy, bx, by, er, mx, my); break;
+      case 2: if (l && g.J < H - 1) grid_patch<0, 1, true, false>(g, sx, sy, bx, by, er, mx, my); break;
+      case 3: if (g.I < H - 1 && g.J < H - 1) grid_patch<1, 1, true, false>(g, sx, sy, bx, by, er, mx, my); break;
+      }
+      __syncthreads();
+    }
+  // owned blocks: the last tiles of a row and column may pass the grid's end
+  const bool own = g.I >= TILE_H / 2 && g.I < H - TILE_H / 2 && g.J >= TILE_H / 2 && g.J < H - TILE_H / 2 &&
+                   ox + 2 * g.I < nx && oy + 2 * g.J < ny;
+  if (own) {
+    C<T>* xo = Xout + (size_t)v * xs;
+    grid_copy_out(g, sx, xo);
+    grid_copy_out(g, sy, xo + N);
+  }
+  if (MODE & 8) {
+    C<T> cx, cy;
+    const bool act = l && d && g.I < H - 1 && g.J < H - 1;
+    grid_restrict_own<true>(g, act, sx, sy, bx, by, er, mx, my, px, py, cx, cy);
+    __syncthreads();
+    if (own) {
+      const int k = g.I + g.J * H;
+      C<T> dn = px[k - H], lf = py[k - 1];
+      if (g.wd) dn = cconj(g.yf) * dn;
+      if (g.wl) lf = cconj(g.xf) * lf;
+      C<T>*bc = BC + (size_t)v * cs, *xc = XC + (size_t)v * cs;
+      const size_t kc = GI + (size_t)GJ * cnx;
+      bc[kc] = cx + T(0.25) * dn;
+      bc[NC + kc] = cy + T(0.25) * lf;
+      xc[kc] = czero<T>();
+      xc[NC + kc] = czero<T>();
     }
   }
 }
@@ -4797,6 +4921,31 @@ static bool afw_grid_fits(int prec, const mxh_level* lv)
   return N <= 4096 && (prec == MXH_F64 ? 40 : 20) * N <= LDS_MAX && lv->nx >= 4 && lv->ny >= 4;
 }
 
+// Launches of few tiles: k_afw_few and the small tiles of k_node_tile.  Up to
+// two tiles per compute unit they are the shorter launch (us, two sweeps and
+// residual, FP64 edges / nodes, against the large tiles: 128^2 one vector 10 / 6
+// against 17 / 10, four 16 / 8 against 19 / 11; 256^2 one 15 / 8 against 19 / 10,
+// two 23 / 11 both; FP32 128^2 four 10 against 16), beyond they repeat
+// the halo's work.  One vector takes them at any size for their rounding (512^2
+// 45 us both).  Edge grids of up to 32 x 32 nodes stay whole in LDS (32
+// vectors: 10 us against 14).
+#define FEW_MAX 512
+static bool few_fits(const mxh_level* lv, int nv)
+{
+  const long long t = (long long)((lv->nx + FEW_T - 1) / FEW_T) * ((lv->ny + FEW_T - 1) / FEW_T);
+  return nv == 1 || t * nv <= FEW_MAX;
+}
+
+template <typename T, int MODE>
+static void launch_few(const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs b, mxh_vecs x, mxh_vecs xo,
+                       const void* eta, int nsweep, mxh_vecs xc_in, mxh_vecs bc, mxh_vecs xc, long long cs)
+{
+  const int ntx = (lv->nx + FEW_T - 1) / FEW_T, nty = (lv->ny + FEW_T - 1) / FEW_T;
+  hipLaunchKernelGGL((k_afw_few<T, MODE>), dim3(ntx * nty, nv), dim3(FEW_R * FEW_R / 4), 0, g_stream, *lv, *bl,
+                     (const C<T>*)b.p, b.stride, (const C<T>*)x.p, (C<T>*)xo.p, x.stride, (const T*)eta, nsweep,
+                     (const C<T>*)xc_in.p, (C<T>*)bc.p, (C<T>*)xc.p, cs, ntx);
+}
+
 template <typename T, int MODE>
 static void launch_grid(const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs b, mxh_vecs x, mxh_vecs xo,
                         const void* eta, int nsweep, mxh_vecs xc_in, mxh_vecs bc, mxh_vecs xc, long long cs)
@@ -4813,13 +4962,14 @@ static void launch_grid(const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_ve
 }
 
 template <typename T>
-static int launch_grid_mode(int mode, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs b, mxh_vecs x,
-                            mxh_vecs xo, const void* eta, int nsweep, mxh_vecs xc_in, mxh_vecs bc, mxh_vecs xc)
+static int launch_grid_mode(bool few, int mode, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs b,
+                            mxh_vecs x, mxh_vecs xo, const void* eta, int nsweep, mxh_vecs xc_in, mxh_vecs bc,
+                            mxh_vecs xc)
 {
   const long long cs = (mode & 8) ? bc.stride : (mode & 4) ? xc_in.stride : 0;
-#define GRID_CASE(M)                                                                     \
-  case M:                                                                                \
-    launch_grid<T, M>(lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc, cs);             \
+#define GRID_CASE(M)                                                            \
+  case M:                                                                       \
+    (few ? launch_few<T, M> : launch_grid<T, M>)(lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc, cs); \
     break;
   switch (mode) {
     GRID_CASE(0)
@@ -4953,9 +5103,10 @@ int mxh_afw_tile(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh
     return (int)hipErrorInvalidValue;
   if ((mode & 4) && !xc_in.p) return (int)hipErrorInvalidValue;
   if ((mode & 8) && (!bc.p || !xc.p || bc.stride != xc.stride)) return (int)hipErrorInvalidValue;
-  if (afw_grid_fits(prec, lv))
-    return prec == MXH_F64 ? launch_grid_mode<double>(mode, lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc)
-                           : launch_grid_mode<float>(mode, lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc);
+  const bool few = few_fits(lv, nv) && (long long)lv->nx * lv->ny > 1024;
+  if (few || afw_grid_fits(prec, lv))
+    return prec == MXH_F64 ? launch_grid_mode<double>(few, mode, lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc)
+                           : launch_grid_mode<float>(few, mode, lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc);
   const int R = prec == MXH_F64 ? TileCfg<double>::R : TileCfg<float>::R, TT = R - 2 * TILE_H;
   const int ntx = (lv->nx + TT - 1) / TT, nty = (lv->ny + TT - 1) / TT;
   dim3 grid(ntx * nty, nv), block((R / 2) * (R / 2));
@@ -4969,26 +5120,26 @@ int mxh_afw_tile(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh
 }
 
 extern "C++" {
-template <typename T, int MODE>
+template <typename T, int MODE, int R>
 static void launch_ntile(dim3 grid, const mxh_level* lv, const mxh_bloch* bl, mxh_vecs b, mxh_vecs x, mxh_vecs xo,
                          int nsweep, mxh_vecs xc_in, mxh_vecs bc, mxh_vecs xc, long long cs, int ntx)
 {
-  hipLaunchKernelGGL((k_node_tile<T, MODE>), grid, dim3(1024), 0, g_stream, *lv, *bl, (const C<T>*)b.p, b.stride,
+  hipLaunchKernelGGL((k_node_tile<T, MODE, R>), grid, dim3(R * R / 4), 0, g_stream, *lv, *bl, (const C<T>*)b.p, b.stride,
                      (const C<T>*)x.p, (C<T>*)xo.p, x.stride, nsweep, (const C<T>*)xc_in.p, (C<T>*)bc.p,
                      (C<T>*)xc.p, cs, ntx);
 }
 
-template <typename T>
+template <typename T, int R>
 static int launch_ntile_mode(int mode, dim3 grid, const mxh_level* lv, const mxh_bloch* bl, mxh_vecs b, mxh_vecs x,
                              mxh_vecs xo, int nsweep, mxh_vecs xc_in, mxh_vecs bc, mxh_vecs xc, long long cs, int ntx)
 {
   switch (mode) {
-  case 0: launch_ntile<T, 0>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
-  case 2: launch_ntile<T, 2>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
-  case 8: launch_ntile<T, 8>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
-  case 10: launch_ntile<T, 10>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
-  case 1: launch_ntile<T, 1>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
-  case 5: launch_ntile<T, 5>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
+  case 0: launch_ntile<T, 0, R>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
+  case 2: launch_ntile<T, 2, R>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
+  case 8: launch_ntile<T, 8, R>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
+  case 10: launch_ntile<T, 10, R>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
+  case 1: launch_ntile<T, 1, R>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
+  case 5: launch_ntile<T, 5, R>(grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx); break;
   default: return (int)hipErrorInvalidValue;
   }
   return 0;
@@ -5007,12 +5158,19 @@ int mxh_node_tile(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mx
     return (int)hipErrorInvalidValue;
   if ((mode & 4) && !xc_in.p) return (int)hipErrorInvalidValue;
   if ((mode & 8) && (!bc.p || !xc.p || bc.stride != xc.stride)) return (int)hipErrorInvalidValue;
-  const int TT = 64 - 2 * TILE_H;
+  const bool few = few_fits(lv, nv);
+  const int TT = (few ? FEW_R : 64) - 2 * TILE_H;
   const int ntx = (lv->nx + TT - 1) / TT, nty = (lv->ny + TT - 1) / TT;
   dim3 grid(ntx * nty, nv);
   long long cs = (mode & 8) ? bc.stride : (mode & 4) ? xc_in.stride : 0;
-  int e = prec == MXH_F64 ? launch_ntile_mode<double>(mode, grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx)
-                          : launch_ntile_mode<float>(mode, grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx);
+  int e;
+  if (few)
+    e = prec == MXH_F64
+            ? launch_ntile_mode<double, FEW_R>(mode, grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx)
+            : launch_ntile_mode<float, FEW_R>(mode, grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx);
+  else
+    e = prec == MXH_F64 ? launch_ntile_mode<double, 64>(mode, grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx)
+                        : launch_ntile_mode<float, 64>(mode, grid, lv, bl, b, x, xo, nsweep, xc_in, bc, xc, cs, ntx);
   if (e) return e;
   LAUNCH_CHECK();
   return 0;
