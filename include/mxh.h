@@ -253,13 +253,18 @@ int mxh_gather(int prec, long long n, int nv, mxh_vecs dst, mxh_vecs src);
 /* Householder M-orthonormalisation of k FP64 edge vectors (orthonormalize_edge2d,
    edge2d.c:6154-6296) entirely on the device: X holds the k inputs back to back
    (2 nx ny complex each) and receives the Householder vectors; V receives the
-   M-orthonormal outputs V_i = H_0 ... H_i unit_i; tmp is one vector of
-   scratch; tau receives the k complex tau_i (device); work is device scratch of
-   mxh_orthonormalize_work_bytes(k).  Bloch factors xf = xr + i xi, yf = yr + i yi;
-   eta64: 1/eps per cell.  k <= nx (ny / 2) unit vectors exist. */
+   M-orthonormal outputs V_i = H_0 ... H_i unit_i; tau receives the k complex
+   tau_i (device); work is device scratch of mxh_orthonormalize_work_bytes(k).
+   Bloch factors xf = xr + i xi, yf = yr + i yi.  k <= nx (ny / 2) unit vectors
+   exist.  eta64 and tmp are not used. */
 size_t mxh_orthonormalize_work_bytes(int k);
 int mxh_orthonormalize(const mxh_level *lv, double xr, double xi, double yr, double yi, const double *eta64,
                        int k, double *X, double *V, double *tmp, double *tau, double *work);
+/* The same in place over k vectors of their own, x[0] .. x[k - 1] (device
+   pointers; the array is read as the stream gets there: pinned, or kept until
+   the stream has run); tau: k complex the device can write (pinned). */
+int mxh_orthonormalize_vecs(const mxh_level *lv, double xr, double xi, double yr, double yi, int k,
+                            void *const *x, double *tau, double *work);
 
 /* ---- node space ---- */
 /* Tile-fused nodal Gauss-Seidel sweeps (alpha = 1), same modes as
@@ -355,6 +360,14 @@ int mxh_axpy(int prec, long long n, int nv, mxh_vecs x, mxh_vecs y, double ar,
    out[v] = x_v^H y_v (complex, device doubles 2 nv) */
 int mxh_dot(int prec, long long n, int nv, mxh_vecs x, mxh_vecs y, double *out,
             double *work);
+/* One launch: out = y^H x over n complex FP64 values, or y^H (alpha K + beta M) x
+   over edge vectors, written to out[0], out[1] and then mark to out[2], in
+   pinned memory: valid once the mark is seen there, or after mxh_sync.  work:
+   MXH_PRODUCT_WORK bytes, zero before the first use, of one product at a time. */
+#define MXH_PRODUCT_WORK (8 * (8 + 2 * 256))
+int mxh_product(long long n, const void *x, const void *y, double *work, double *out, double mark);
+int mxh_product_edge(const mxh_level *lv, const mxh_bloch *bl, const void *x, const void *y, const double *eta,
+                     const mxh_coef *cf, double *work, double *out, double mark);
 /* out[v] = |x_v|_2^2 or max |x_v| (kind 0/1) */
 int mxh_norm(int prec, long long n, int nv, mxh_vecs x, int kind, double *out,
              double *work);

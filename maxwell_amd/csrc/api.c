@@ -57,6 +57,74 @@ static void ensure_init(void)
   }
 }
 
+/* Places for results that a kernel writes where the host reads them, and for
+   the device scratch of the launches that make them: one per call in flight,
+   kept for the next (CALL_SLOTS at most; scratch above CALL_KEEP goes back to
+   the device after the call). */
+#define CALL_SLOTS 16
+#define CALL_HOST 8192
+#define CALL_KEEP ((size_t)1 << 20)
+typedef struct {
+  int busy;
+  double *count; /* MXH_PRODUCT_WORK bytes of mxh_product */
+  double *host;  /* CALL_HOST bytes, pinned */
+  double mark;   /* of the last product */
+  void *dev;
+  size_t ndev;
+} call_slot;
+
+static call_slot call_slots[CALL_SLOTS];
+static pthread_mutex_t call_lock = PTHREAD_MUTEX_INITIALIZER;
+static pthread_cond_t call_free = PTHREAD_COND_INITIALIZER;
+
+static call_slot *take_slot(void)
+{
+  call_slot *s = NULL;
+  pthread_mutex_lock(&call_lock);
+  while (!s) {
+    for (int k = 0; k < CALL_SLOTS && !s; k++)
+      if (!call_slots[k].busy) s = &call_slots[k];
+    if (!s) pthread_cond_wait(&call_free, &call_lock);
+  }
+  s->busy = 1;
+  pthread_mutex_unlock(&call_lock);
+  if (!s->count) {
+    double *c = (double *)mxh_malloc(MXH_PRODUCT_WORK);
+    s->host = (double *)mxh_host_alloc(CALL_HOST);
+    if (!c || !s->host) die("result allocation", 0);
+    HIPCK(mxh_memset(c, 0, MXH_PRODUCT_WORK));
+    s->count = c;
+    s->host[2] = s->mark = 0.0;
+  }
+  return s;
+}
+
+/* at least `bytes` of device scratch in the slot */
+static void *slot_scratch(call_slot *s, size_t bytes)
+{
+  if (s->ndev < bytes) {
+    mxh_free(s->dev);
+    s->dev = mxh_malloc(bytes);
+    if (!s->dev) die("scratch allocation", 0);
+    s->ndev = bytes;
+  }
+  return s->dev;
+}
+
+/* after the stream has been waited for */
+static void give_slot(call_slot *s)
+{
+  if (s->ndev > CALL_KEEP) {
+    mxh_free(s->dev);
+    s->dev = NULL;
+    s->ndev = 0;
+  }
+  pthread_mutex_lock(&call_lock);
+  s->busy = 0;
+  pthread_cond_signal(&call_free);
+  pthread_mutex_unlock(&call_lock);
+}
+
 typedef struct {
   double *eta;   /* device copy of gr->eps (FP64) */
   double *work;  /* reduction scratch */
@@ -131,13 +199,38 @@ static field *scratch_edge(const grid2d *gr)
   return g->tmp;
 }
 
-static field dot_dev(int prec, const grid2d *gr, long long n, const void *x, const void *y)
+/* the product under way: the mark arrives some microseconds before the stream
+   reports the launch as done (a 32^2 product 12 us against 18); a wait of more than
+   a few dozen is left to the stream, which also reports errors */
+static field product_result(call_slot *s)
 {
-  griddev *g = gdev(gr);
-  double r[2];
-  HIPCK(mxh_dot(prec, n, 1, VV(x, n), VV(y, n), g->out, g->work));
-  HIPCK(mxh_d2h(r, g->out, sizeof(r)));
-  return r[0] + I * r[1];
+  s->mark += 1.0;
+  const volatile double *m = s->host + 2;
+  int spins = 0;
+  while (*m != s->mark && ++spins < 20000) __builtin_ia32_pause();
+  if (*m != s->mark) HIPCK(mxh_sync());
+  __atomic_thread_fence(__ATOMIC_ACQUIRE);
+  const field r = s->host[0] + I * s->host[1];
+  give_slot(s);
+  return r;
+}
+
+static field dot_dev(long long n, const void *x, const void *y)
+{
+  call_slot *s = take_slot();
+  HIPCK(mxh_product(n, y, x, s->count, s->host, s->mark + 1.0));
+  return product_result(s);
+}
+
+/* y^H (alpha K + beta M) x */
+static field operator_dot(field alpha, field beta, const edge2d *x, const edge2d *y)
+{
+  const mxh_level lv = level_of(x->gr);
+  const mxh_bloch bl = bloch_of(x->gr);
+  const mxh_coef cf = coef(alpha, beta);
+  call_slot *s = take_slot();
+  HIPCK(mxh_product_edge(&lv, &bl, x->x, y->x, gdev(x->gr)->eta, &cf, s->count, s->host, s->mark + 1.0));
+  return product_result(s);
 }
 
 static double norm_dev(const grid2d *gr, long long n, const void *x, int kind)
@@ -526,7 +619,7 @@ field dotprod_edge2d(const edge2d *x, const edge2d *y)
   assert(x->gr == y->gr);
   field r = 0.0;
 #pragma omp single copyprivate(r)
-  r = dot_dev(MXH_F64, x->gr, en(x), x->x, y->x);
+  r = dot_dev(en(x), x->x, y->x);
   return r;
 }
 
@@ -541,10 +634,10 @@ static void half_sums(const edge2d *x, field *sx, field *sy)
   if (!h) die("host allocation", 0);
   for (long long k = 0; k < 2 * N; k++) h[k] = (k < N) ? 1.0 : 0.0;
   HIPCK(mxh_h2d(ones, h, sizeof(field) * 2 * N));
-  *sx = dot_dev(MXH_F64, x->gr, 2 * N, ones, x->x);
+  *sx = dot_dev(2 * N, ones, x->x);
   for (long long k = 0; k < 2 * N; k++) h[k] = (k < N) ? 0.0 : 1.0;
   HIPCK(mxh_h2d(ones, h, sizeof(field) * 2 * N));
-  *sy = dot_dev(MXH_F64, x->gr, 2 * N, ones, x->x);
+  *sy = dot_dev(2 * N, ones, x->x);
   free(h);
 }
 
@@ -606,14 +699,7 @@ field energyprod_edge2d(field alpha, field beta, const edge2d *x, const edge2d *
   assert(x->gr == y->gr);
   field r = 0.0;
 #pragma omp single copyprivate(r)
-  {
-    mxh_level lv = level_of(x->gr);
-    mxh_bloch bl = bloch_of(x->gr);
-    mxh_coef cf = coef(alpha, beta);
-    field *t = scratch_edge(x->gr);
-    HIPCK(mxh_addeval(MXH_F64, &lv, &bl, 1, VV(x->x, en(x)), VV(t, en(x)), gdev(x->gr)->eta, &cf, 0));
-    r = conj(dot_dev(MXH_F64, x->gr, en(x), y->x, t));
-  }
+  r = conj(operator_dot(alpha, beta, x, y));
   return r;
 }
 
@@ -622,14 +708,7 @@ field massprod_edge2d(const edge2d *x, const edge2d *y)
   assert(x->gr == y->gr);
   field r = 0.0;
 #pragma omp single copyprivate(r)
-  {
-    mxh_level lv = level_of(x->gr);
-    mxh_bloch bl = bloch_of(x->gr);
-    mxh_coef cf = coef(0.0, 1.0);
-    field *t = scratch_edge(x->gr);
-    HIPCK(mxh_addeval(MXH_F64, &lv, &bl, 1, VV(x->x, en(x)), VV(t, en(x)), gdev(x->gr)->eta, &cf, 0));
-    r = conj(dot_dev(MXH_F64, x->gr, en(x), y->x, t));
-  }
+  r = conj(operator_dot(0.0, 1.0, x, y));
   return r;
 }
 
@@ -1135,37 +1214,35 @@ void applyhouseholder_edge2d(const edge2d *v, field tau, edge2d *x)
 }
 
 /* The whole orthonormalisation runs on the device as one sequence of
-   launches over a contiguous copy of the k vectors (mxh_orthonormalize: per
-   Householder step a batched M-product row, one rank-one update of all later
-   vectors and their unit-entry fix; the outputs H_0 ... H_i unit_i are built
-   for all i together), with no host round trip until tau is copied back.
-   Outputs go to x[0..k-1]; v (scratch in the reference) receives x[0]'s
-   output, as the reference's last back-substitution leaves it. */
+   launches over the vectors in place (mxh_orthonormalize_vecs: two per
+   Householder step, then the outputs H_0 ... H_i unit_i of all i together),
+   with no host round trip until tau is back.  v (scratch in the reference)
+   receives x[0]'s output, as the reference's last back-substitution leaves it. */
 void orthonormalize_edge2d(int k, edge2d **x, field *tau, edge2d *v)
 {
   assert(k >= 1);
 #pragma omp single
   {
     const grid2d *gr = x[0]->gr;
-    const size_t n = en(x[0]);
-    mxh_level lv = level_of(gr);
-    field *blk = (field *)mxh_malloc(sizeof(field) * n * (2 * (size_t)k + 1));
-    double *dtau = (double *)mxh_malloc(sizeof(double) * 2 * (size_t)k);
-    double *work = (double *)mxh_malloc(mxh_orthonormalize_work_bytes(k));
-    if (!blk || !dtau || !work) die("orthonormalize allocation", 0);
-    field *X = blk, *Vv = blk + (size_t)k * n, *tmp = blk + 2 * (size_t)k * n;
+    const mxh_level lv = level_of(gr);
+    const size_t per = sizeof(void *) + sizeof(field);
+    call_slot *s = take_slot();
+    double *work = (double *)slot_scratch(s, mxh_orthonormalize_work_bytes(k));
+    double *host = per * k <= CALL_HOST ? s->host : (double *)mxh_host_alloc(per * k);
+    if (!host) die("orthonormalize allocation", 0);
+    void **table = (void **)(host + 2 * (size_t)k);
     for (int i = 0; i < k; i++) {
       assert(x[i]->gr == gr);
-      HIPCK(mxh_d2d(X + (size_t)i * n, x[i]->x, sizeof(field) * n));
+      table[i] = x[i]->x;
     }
-    HIPCK(mxh_orthonormalize(&lv, creal(gr->xfactor), cimag(gr->xfactor), creal(gr->yfactor), cimag(gr->yfactor),
-                             gdev(gr)->eta, k, (double *)X, (double *)Vv, (double *)tmp, dtau, work));
-    for (int i = 0; i < k; i++) HIPCK(mxh_d2d(x[i]->x, Vv + (size_t)i * n, sizeof(field) * n));
-    if (v) HIPCK(mxh_d2d(v->x, Vv, sizeof(field) * n));
-    HIPCK(mxh_d2h(tau, dtau, sizeof(field) * (size_t)k));
-    mxh_free(blk);
-    mxh_free(dtau);
-    mxh_free(work);
+    HIPCK(mxh_orthonormalize_vecs(&lv, creal(gr->xfactor), cimag(gr->xfactor), creal(gr->yfactor),
+                                  cimag(gr->yfactor), k, table, host, work));
+    if (v) HIPCK(mxh_d2d(v->x, x[0]->x, sizeof(field) * en(x[0])));
+    HIPCK(mxh_sync());
+    memcpy(tau, host, sizeof(field) * (size_t)k);
+    if (host != s->host) mxh_host_free(host);
+    else s->host[2] = s->mark = 0.0;
+    give_slot(s);
   }
 }
 
@@ -1255,7 +1332,7 @@ field dotprod_node2d(const node2d *x, const node2d *y)
   assert(x->gr == y->gr);
   field r = 0.0;
 #pragma omp single copyprivate(r)
-  r = dot_dev(MXH_F64, x->gr, nn(x), x->v, y->v);
+  r = dot_dev(nn(x), x->v, y->v);
   return r;
 }
 
@@ -1269,7 +1346,7 @@ void center_node2d(node2d *x)
     field *h = (field *)malloc(sizeof(field) * n);
     for (long long k = 0; k < n; k++) h[k] = 1.0;
     HIPCK(mxh_h2d(ones, h, sizeof(field) * n));
-    field s = dot_dev(MXH_F64, x->gr, n, ones, x->v) / (double)n;
+    field s = dot_dev(n, ones, x->v) / (double)n;
     HIPCK(mxh_axpy(MXH_F64, n, 1, VV(ones, n), VV(x->v, n), -creal(s), -cimag(s)));
     HIPCK(mxh_sync());
     free(h);

@@ -267,6 +267,12 @@ __global__ void k_reduce_partials(const double* __restrict__ part, int nblk, int
 
 static const int TPB = 256;
 
+__global__ __launch_bounds__(256) void k_copy(size_t n, const uint4* src, uint4* dst)
+{
+  const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) dst[k] = src[k];
+}
+
 // the LDS of a compute unit, and bytes per complex value
 #define LDS_MAX (160 * 1024)
 static size_t csize(int prec) { return prec == MXH_F64 ? 16 : 8; }
@@ -1531,74 +1537,229 @@ MXH_DEV C<double> unit_mprod(const C<double>* y, int i, int j, int nx, int ny, d
   return sqrt(0.25 * mx) * (4.0 * y[i + (size_t)j * nx] + y[i + (size_t)(j - 1) * nx] + up);
 }
 
-// Step idx of the forward pass, one thread: x = x_idx, a = x^H M x (device),
-// mx_ = M x (device, all entries).  Builds the Householder vector in place
-// (edge2d.c:6238-6262): alpha = |x|_M with the sign of Re(beta), beta =
-// unit^H M x, x += alpha unit, tau = 1 / (alpha^2 + beta alpha) (0 when x
-// = 0), and updates M x by alpha M unit (three entries) so that mx_ is the
-// Householder vector's M-image.
-__global__ void k_hh_build(mxh_level lv, C<double> yf, int idx, C<double>* x, C<double>* mx_, const double* a,
-                           double* tau)
+// Forward pass, two launches a reflection.  k_hh_row(i) sums x_i^H M x_j over
+// every later vector and x_i^H M v_j over every finished one, and p_j = unit_i^H M
+// of each; k_hh_update(i) turns the sums into reflection i (edge2d.c:6238-6262):
+// alpha = |x_i|_M with the sign of Re(beta), beta = p_i, v_i = x_i + alpha
+// unit_i, tau = 1 / (alpha^2 + beta alpha) (0 when x_i = 0), and applies it to the
+// later vectors, whose component along unit_i then goes (edge2d.c:6273-6285).
+// Every workgroup finishes the sums it needs itself, so that nothing but the
+// end of a launch orders the two; v_i stays x_i in memory until the next
+// k_hh_row adds alpha unit_i to its one entry.
+//
+// The outputs V_i = H_0 ... H_i unit_i (H_j = I - conj(tau_j) v_j v_j^H M) all at
+// once: with S_jl = v_j^H M v_l (j < l) and w = (v_j^H M unit_i)_j, V_i = unit_i
+// - sum_j v_j c_j where c_j = conj(tau_j) (w_j - sum_{l > j} S_jl c_l), l <= i.
+//
+// Bound by the chain of 2 k launches on the drivers' grids: 24 vectors of 128^2
+// 1.28 -> 0.45 ms against one launch per product, update and fix of both passes.
+#define HH_NB 64  // partial sums per vector at most (one wave's lanes)
+struct HhVecs {
+  C<double>* base;  // vector j at base + j stride, or, with a table, table[j]
+  long long stride;
+  C<double>* const* table;
+  MXH_DEV C<double>* at(int j) const { return table ? table[j] : base + (size_t)j * stride; }
+};
+// work: [hh: alpha, tau, unused per vector | p | partial sums | S | W -> c]
+struct HhWork {
+  double *hh, *p, *part, *S, *W;
+};
+static HhWork hh_work(double* w, int k)
 {
-  const int nx = lv.nx, ny = lv.ny;
-  int i, j;
-  unit_ij(idx, nx, i, j);
-  const double mxc = lv.hy / lv.hx / 6.0, sc = sqrt(0.25 / mxc);
-  double alpha = sqrt(a[0]);
-  if (alpha == 0.0) {
-    tau[2 * idx] = tau[2 * idx + 1] = 0.0;
+  HhWork h;
+  h.hh = w;
+  h.p = h.hh + 4 * (size_t)k;
+  h.part = h.p + 2 * (size_t)k;
+  h.S = h.part + 2 * HH_NB * (size_t)k;
+  h.W = h.S + 2 * (size_t)k * k;
+  return h;
+}
+
+__global__ __launch_bounds__(256) void k_hh_row(mxh_level lv, C<double> xf, C<double> yf, int idx, HhVecs X,
+                                                HhWork wk)
+{
+  __shared__ double sh[4];
+  const int nx = lv.nx, ny = lv.ny, j = blockIdx.y, tid = threadIdx.x;
+  const size_t N = (size_t)nx * ny;
+  const double mx = lv.hy / lv.hx / 6.0, my = lv.hx / lv.hy / 6.0;
+  const C<double>*x = X.at(idx), *y = x + N;
+  C<double>* u = X.at(j);
+  int i0, j0;
+  size_t fix = ~(size_t)0;  // v_{idx - 1}: alpha unit still to be added
+  double add = 0.0;
+  if (idx > 0 && j == idx - 1) {
+    unit_ij(j, nx, i0, j0);
+    fix = i0 + (size_t)j0 * nx;
+    add = wk.hh[4 * j] * sqrt(0.25 / mx);
+  }
+  double sr = 0.0, si = 0.0;
+  for (size_t e = (size_t)blockIdx.x * blockDim.x + tid; e < N; e += (size_t)gridDim.x * blockDim.x) {
+    const int r = (int)((unsigned)e / (unsigned)nx), c = (int)e - r * nx;
+    const C<double> dn = r ? x[e - nx] : cconj(yf) * x[e + N - nx], up = r + 1 < ny ? x[e + nx] : yf * x[c];
+    const C<double> lf = c ? y[e - 1] : cconj(xf) * y[e + nx - 1], rt = c + 1 < nx ? y[e + 1] : xf * y[e - c];
+    const C<double> a = mx * (4.0 * x[e] + dn + up), b = my * (4.0 * y[e] + lf + rt);
+    C<double> p = u[e];
+    const C<double> q = u[N + e];
+    if (e == fix) {
+      p.r += add;
+      u[e] = p;
+    }
+    sr += a.r * p.r + a.i * p.i + b.r * q.r + b.i * q.i;
+    si += a.r * p.i - a.i * p.r + b.r * q.i - b.i * q.r;
+  }
+  sr = block_sum256(sr, sh);
+  si = block_sum256(si, sh);
+  if (tid == 0) {
+    double* o = wk.part + 2 * ((size_t)j * HH_NB + blockIdx.x);
+    o[0] = sr;
+    o[1] = si;
+    if (blockIdx.x == 0) {
+      unit_ij(idx, nx, i0, j0);
+      const C<double> p = unit_mprod(u, i0, j0, nx, ny, mx, yf);
+      wk.p[2 * j] = p.r;
+      wk.p[2 * j + 1] = p.i;
+    }
+  }
+}
+
+// the sum of vector j's nb partial sums (whole waves)
+MXH_DEV C<double> hh_sum(const HhWork& wk, int j, int nb)
+{
+  const int l = threadIdx.x & 63;
+  const double* q = wk.part + 2 * ((size_t)j * HH_NB + l);
+  return cmk(wave_sum(l < nb ? q[0] : 0.0), wave_sum(l < nb ? q[1] : 0.0));
+}
+
+// grid (blocks, k - idx): vector idx + blockIdx.y; nb: blocks of k_hh_row
+__global__ __launch_bounds__(256) void k_hh_update(mxh_level lv, int idx, int k, int nb, HhVecs X, HhWork wk)
+{
+  const int nx = lv.nx, tid = threadIdx.x, j = idx + blockIdx.y;
+  const size_t E = 2 * (size_t)nx * lv.ny;
+  if (j == idx && blockIdx.x) return;
+  const double sc = sqrt(0.25 / (lv.hy / lv.hx / 6.0));
+  const C<double> beta = cmk(wk.p[2 * idx], wk.p[2 * idx + 1]);
+  double alpha = sqrt(hh_sum(wk, idx, nb).r);
+  C<double> tau = czero<double>();
+  if (alpha != 0.0) {
+    if (beta.r < 0.0) alpha = -alpha;
+    const C<double> den = cmk(alpha * alpha + beta.r * alpha, beta.i * alpha);
+    const double dd = den.r * den.r + den.i * den.i;
+    tau = cmk(den.r / dd, -den.i / dd);
+  }
+  const C<double> uv = cmk(beta.r + alpha, beta.i);  // unit^H M v
+  C<double>*S = (C<double>*)wk.S, *W = (C<double>*)wk.W;
+  if (j == idx) {
+    for (int l = tid >> 6; l < idx; l += 4) {
+      const C<double> d = hh_sum(wk, l, nb), p = cmk(wk.p[2 * l], -wk.p[2 * l + 1]);
+      if ((tid & 63) == 0) {
+        S[(size_t)l * k + idx] = cconj(d) + alpha * p;
+        W[(size_t)l * k + idx] = p;
+      }
+    }
+    if (tid == 0) {
+      W[(size_t)idx * k + idx] = cconj(uv);
+      wk.hh[4 * idx] = alpha;
+      wk.hh[4 * idx + 1] = tau.r;
+      wk.hh[4 * idx + 2] = tau.i;
+    }
     return;
   }
-  const C<double> beta = unit_mprod(x, i, j, nx, ny, mxc, yf);
-  if (beta.r < 0.0) alpha = -alpha;
-  x[i + (size_t)j * nx] += cmk(alpha * sc, 0.0);
-  // tau = 1 / (alpha^2 + beta alpha)
-  const C<double> den = cmk(alpha * alpha + beta.r * alpha, beta.i * alpha);
-  const double dd = den.r * den.r + den.i * den.i;
-  tau[2 * idx] = den.r / dd;
-  tau[2 * idx + 1] = -den.i / dd;
-  // M (alpha s unit): 4 mx alpha s at (i, j), mx alpha s at (i, j -+ 1) (x-edges of one column)
-  const double u = alpha * sc * mxc;
-  mx_[i + (size_t)j * nx] += cmk(4.0 * u, 0.0);
-  mx_[i + (size_t)(j - 1) * nx] += cmk(u, 0.0);
-  if (j + 1 < ny) mx_[i + (size_t)(j + 1) * nx] += cmk(u, 0.0);
-  else mx_[i] += cconj(yf) * cmk(u, 0.0);
+  const C<double> pj = cmk(wk.p[2 * j], wk.p[2 * j + 1]);
+  const C<double> c = -1.0 * (tau * (hh_sum(wk, j, nb) + alpha * pj));
+  int i0, j0;
+  unit_ij(idx, nx, i0, j0);
+  const size_t at = i0 + (size_t)j0 * nx;
+  const C<double>* x = X.at(idx);
+  C<double>* y = X.at(j);
+  for (size_t e = (size_t)blockIdx.x * blockDim.x + tid; e < E; e += (size_t)gridDim.x * blockDim.x) {
+    C<double> v = x[e], u = y[e];
+    if (e == at) {
+      v.r += alpha * sc;
+      u -= sc * (pj + c * uv);
+    }
+    y[e] = u + c * v;
+  }
 }
 
-// y_v += c_v x for v < nv, c_v = sign * t * d_v with t = tau[2 tidx] (conj
-// when cj), d_v = dots[v] (device complex): the reflections' rank-one updates
-__global__ __launch_bounds__(256) void k_hh_axpy(long long n, int nv, const C<double>* x, C<double>* Y, long long ys,
-                                                 const double* tau, int tidx, int cj, const double* dots)
+// the coefficients c (in W) by back substitution, one workgroup, and what the
+// last k_hh_row would have finished: v_{k - 1}; tau to both outputs
+__global__ __launch_bounds__(1024) void k_hh_coef(mxh_level lv, int k, HhVecs X, HhWork wk, double* tau, double* host)
 {
-  const int v = blockIdx.y;
-  C<double> t = cmk(tau[2 * tidx], cj ? -tau[2 * tidx + 1] : tau[2 * tidx + 1]);
-  const C<double> c = -1.0 * (t * cmk(dots[2 * v], dots[2 * v + 1]));
-  C<double>* y = Y + (size_t)v * ys;
-  for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < (size_t)n; k += (size_t)gridDim.x * blockDim.x)
-    y[k] += c * x[k];
+  extern __shared__ double smem[];
+  const int tid = threadIdx.x, bd = blockDim.x;
+  C<double>*S = (C<double>*)wk.S, *W = (C<double>*)wk.W;
+  C<double>*s = S, *w = W;
+  if (k <= 48) {  // in LDS (73 KB)
+    s = (C<double>*)smem;
+    w = s + k * k;
+    for (int e = tid; e < k * k; e += bd) {
+      s[e] = S[e];
+      w[e] = W[e];
+    }
+  }
+  for (int j = k - 1; j >= 0; j--) {
+    __syncthreads();
+    const C<double> t = cmk(wk.hh[4 * j + 1], -wk.hh[4 * j + 2]);
+    for (int e = tid; e < j * (k - j); e += bd) {
+      const int r = e / (k - j), i = j + e - r * (k - j);
+      w[(size_t)r * k + i] -= s[(size_t)r * k + j] * (t * w[(size_t)j * k + i]);
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < k * k; e += bd) {
+    const int j = e / k, i = e - j * k;
+    if (i >= j) W[e] = cmk(wk.hh[4 * j + 1], -wk.hh[4 * j + 2]) * w[e];
+  }
+  for (int j = tid; j < k; j += bd) {
+    const double r = wk.hh[4 * j + 1], i = wk.hh[4 * j + 2];
+    if (tau) {
+      tau[2 * j] = r;
+      tau[2 * j + 1] = i;
+    }
+    if (host) {
+      host[2 * j] = r;
+      host[2 * j + 1] = i;
+    }
+  }
+  if (tid == 0) {
+    int i0, j0;
+    unit_ij(k - 1, lv.nx, i0, j0);
+    X.at(k - 1)[i0 + (size_t)j0 * lv.nx].r += wk.hh[4 * (k - 1)] * sqrt(0.25 / (lv.hy / lv.hx / 6.0));
+  }
 }
 
-// x_v -= (unit_idx^H M x_v) unit_idx for v < nv (edge2d.c:6281-6283)
-__global__ void k_hh_unitfix(mxh_level lv, C<double> yf, int idx, int nv, C<double>* X, long long xs)
+// V_i = unit_i - sum_{j <= i} v_j c_ji, eight outputs at a time from the last
+// ones down: V may be X
+__global__ __launch_bounds__(64) void k_hh_out(mxh_level lv, int k, HhVecs X, HhVecs V,
+                                               const C<double>* __restrict__ cf)
 {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= nv) return;
-  int i, j;
-  unit_ij(idx, lv.nx, i, j);
-  const double mxc = lv.hy / lv.hx / 6.0, sc = sqrt(0.25 / mxc);
-  C<double>* x = X + (size_t)v * xs;
-  const C<double> p = unit_mprod(x, i, j, lv.nx, lv.ny, mxc, yf);
-  x[i + (size_t)j * lv.nx] -= sc * p;
-}
-
-// V = [unit_0 .. unit_{k-1}]
-__global__ void k_hh_units(mxh_level lv, int k, C<double>* V, long long vs)
-{
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= k) return;
-  int i, j;
-  unit_ij(v, lv.nx, i, j);
-  V[(size_t)v * vs + i + (size_t)j * lv.nx] = cmk(sqrt(0.25 / (lv.hy / lv.hx / 6.0)), 0.0);
+  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x, N = (size_t)lv.nx * lv.ny;
+  if (e >= 2 * N) return;
+  // the unit vector whose entry e is
+  const unsigned row = (unsigned)(e < N ? e : 0) / (unsigned)lv.nx;
+  const long long unit = e < N && (row & 1) ? (long long)(row >> 1) * lv.nx + (long long)(e - (size_t)row * lv.nx) : -1;
+  const double sc = sqrt(0.25 / (lv.hy / lv.hx / 6.0));
+  for (int i0 = (k - 1) & ~7; i0 >= 0; i0 -= 8) {
+    const int m = min(8, k - i0);
+    C<double> acc[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) acc[q] = cmk(unit == i0 + q ? sc : 0.0, 0.0);
+    for (int j0 = 0; j0 <= i0; j0 += 8) {
+      C<double> v[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) v[j] = X.at(min(j0 + j, k - 1))[e];
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const C<double>* c = cf + (size_t)min(j0 + j, k - 1) * k;
+#pragma unroll
+        for (int q = 0; q < 8; q++)  // (outputs past the last one are not written)
+          if (j0 < i0 || q >= j) acc[q] -= c[min(i0 + q, k - 1)] * v[j];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (q < m) V.at(i0 + q)[e] = acc[q];
+  }
 }
 
 template <typename T>
@@ -2538,6 +2699,86 @@ __global__ __launch_bounds__(256) void k_dot(long long n, const C<T>* X, long lo
     size_t w = (size_t)blockIdx.x * (2 * gridDim.y) + 2 * v;
     part[w] = a;
     part[w + 1] = b;
+  }
+}
+
+// conj(y)^T x (EDGE 0) or y^H (alpha K + beta M) x (EDGE 1) in FP64 in one launch:
+// a workgroup's sum, or the last one to finish adds all partial sums in their
+// order, written where the host reads it.  What bounds it is the launch and the
+// wait of the host: a 32^2 grid's product 28 -> 12 us against operator,
+// product, sum and copy.  work: a counter (0 between launches), then the sums.
+#define PRODUCT_TB 1024
+#define PRODUCT_BLOCKS 256
+template <int EDGE>
+__global__ __launch_bounds__(PRODUCT_TB) void k_product(mxh_level lv, mxh_bloch bl, long long n, const C<double>* X,
+                                                       const C<double>* Y, const double* eta, mxh_coef cf,
+                                                       double* work, double* out, double mark)
+{
+  __shared__ double sh[2 * PRODUCT_TB / 64];
+  __shared__ int last;
+  const int tid = threadIdx.x, w = tid >> 6, nw = PRODUCT_TB / 64;
+  double sr = 0.0, si = 0.0;
+  auto add = [&](C<double> a, C<double> b) {
+    sr += a.r * b.r + a.i * b.i;
+    si += a.r * b.i - a.i * b.r;
+  };
+  if (EDGE) {
+    const size_t N = (size_t)lv.nx * lv.ny;
+    const Geo<double> g = make_geo<double>(lv, bl, 0);
+    C<double> axy, mx, my, ox, oy;
+    coefs<double>(lv, cf, 0, axy, mx, my);
+    const EdgeV<double> e = edge_view<double>(X, 0, 0, N);
+    for (size_t k = (size_t)blockIdx.x * PRODUCT_TB + tid; k < N; k += (size_t)gridDim.x * PRODUCT_TB) {
+      const int j = (int)((unsigned)k / (unsigned)lv.nx);
+      apply_at(g, e, eta, (int)k - j * lv.nx, j, axy, mx, my, ox, oy);
+      add(Y[k], ox);
+      add(Y[N + k], oy);
+    }
+  } else {
+    for (size_t k = (size_t)blockIdx.x * PRODUCT_TB + tid; k < (size_t)n; k += (size_t)gridDim.x * PRODUCT_TB)
+      add(Y[k], X[k]);
+  }
+  auto total = [&]() {  // over the workgroup, in thread 0
+    sr = wave_sum(sr);
+    si = wave_sum(si);
+    if ((tid & 63) == 0) {
+      sh[w] = sr;
+      sh[nw + w] = si;
+    }
+    __syncthreads();
+    sr = si = 0.0;
+    if (tid == 0)
+      for (int q = 0; q < nw; q++) {
+        sr += sh[q];
+        si += sh[nw + q];
+      }
+  };
+  total();
+  unsigned* count = (unsigned*)work;
+  double* part = work + 8;
+  if (gridDim.x > 1) {
+    if (tid == 0) {
+      part[2 * blockIdx.x] = sr;
+      part[2 * blockIdx.x + 1] = si;
+      __threadfence();
+      last = atomicAdd(count, 1u) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    sr = si = 0.0;
+    for (int q = tid; q < (int)gridDim.x; q += PRODUCT_TB) {
+      sr += part[2 * q];
+      si += part[2 * q + 1];
+    }
+    total();
+    if (tid == 0) *count = 0;
+  }
+  if (tid == 0) {
+    out[0] = sr;
+    out[1] = si;
+    __threadfence_system();
+    __hip_atomic_store(out + 2, mark, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -4714,7 +4955,7 @@ int mxh_init(void)
                        (const void*)k_fft_rows<float, -1>, (const void*)k_fft_rows<float, 1>,
                        (const void*)k_edge_cycle<double>, (const void*)k_edge_cycle<float>,
                        (const void*)k_node_cycle<double>, (const void*)k_node_cycle<float>,
-                       (const void*)k_coarse_inverse};
+                       (const void*)k_coarse_inverse, (const void*)k_hh_coef};
   for (const void* f : big) {
     e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     if (e != hipSuccess) return (int)e;
@@ -4802,6 +5043,13 @@ int mxh_event_sync(void* ev) { return (int)hipEventSynchronize((hipEvent_t)ev); 
 
 int mxh_d2d(void* dst, const void* src, size_t bytes)
 {
+  // up to a few MB a launch of our own is queued sooner than the runtime's copy
+  if (bytes && bytes <= ((size_t)4 << 20) && !(((size_t)dst | (size_t)src | bytes) & 15)) {
+    hipLaunchKernelGGL(k_copy, dim3(nblocks((long long)(bytes / 16))), dim3(TPB), 0, g_stream, bytes / 16,
+                       (const uint4*)src, (uint4*)dst);
+    LAUNCH_CHECK();
+    return 0;
+  }
   return (int)hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, g_stream);
 }
 
@@ -5518,68 +5766,58 @@ int mxh_lobpcg_combine(long long n, int nprob, const int* pmap, int m, mxh_vecs 
   return 0;
 }
 
-size_t mxh_orthonormalize_work_bytes(int k) { return sizeof(double) * (512 * 4 * (size_t)k + 8 * (size_t)k + 64); }
+size_t mxh_orthonormalize_work_bytes(int k)
+{
+  // HhWork and a table of k vectors
+  return sizeof(double) * ((6 + 2 * HH_NB + 4 * (size_t)k) * (size_t)k) + sizeof(void*) * (size_t)k;
+}
+
+static int hh_run(const mxh_level* lv, double xr, double xi, double yr, double yi, int k, HhVecs X, HhVecs V, double* work,
+                  double* tau, double* host)
+{
+  const long long N = (long long)lv->nx * lv->ny;
+  const HhWork wk = hh_work(work, k);
+  C<double> xf, yf;
+  xf.r = xr;
+  xf.i = xi;
+  yf.r = yr;
+  yf.i = yi;
+  const int nb = N < 256 * HH_NB ? (int)nblocks(N) : HH_NB;
+  for (int i = 0; i < k; i++) {
+    hipLaunchKernelGGL(k_hh_row, dim3(nb, k), dim3(256), 0, g_stream, *lv, xf, yf, i, X, wk);
+    LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_hh_update, dim3(nb, k - i), dim3(256), 0, g_stream, *lv, i, k, nb, X, wk);
+    LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL(k_hh_coef, dim3(1), dim3(1024), k <= 48 ? 2 * sizeof(C<double>) * k * k : 0, g_stream, *lv, k, X,
+                     wk, tau, host);
+  LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_hh_out, dim3(nblocks(2 * N, 64)), dim3(64), 0, g_stream, *lv, k, X, V, (const C<double>*)wk.W);
+  LAUNCH_CHECK();
+  return 0;
+}
 
 int mxh_orthonormalize(const mxh_level* lv, double xr, double xi, double yr, double yi, const double* eta64, int k,
                        double* X, double* V, double* tmp, double* tau, double* work)
 {
-  const int nx = lv->nx, ny = lv->ny;
-  if (k < 1 || ny < 2 || (long long)k > (long long)nx * (ny / 2)) return (int)hipErrorInvalidValue;
-  const long long n = 2LL * nx * ny;
-  mxh_bloch bl;
-  bl.xr = xr;
-  bl.xi = xi;
-  bl.yr = yr;
-  bl.yi = yi;
-  bl.per_problem = nullptr;
-  bl.vpp = 1;
-  bl.vmap = nullptr;
-  C<double> yf;
-  yf.r = yr;
-  yf.i = yi;
-  double* dots = work + 512 * 4 * (size_t)k;
-  double* part = work;
-  C<double>* Xc = (C<double>*)X;
-  C<double>* Vc = (C<double>*)V;
-  C<double>* Tc = (C<double>*)tmp;
-  const mxh_coef mass = {0.0, 0.0, 1.0, 0.0, nullptr};
-  const unsigned nb = nblocks(n) < 1024 ? nblocks(n) : 1024;
-  int e;
-  // forward pass: Householder vectors in X (edge2d.c:6273-6285)
-  for (int i = 0; i < k; i++) {
-    mxh_vecs xi_v = {(void*)(X + 2 * (size_t)i * n), n, nullptr};
-    if ((e = mxh_addeval(MXH_F64, lv, &bl, 1, xi_v, mxh_vecs{tmp, n, nullptr}, eta64, &mass, 0))) return e;
-    if ((e = mxh_dot(MXH_F64, n, 1, mxh_vecs{tmp, 0, nullptr}, xi_v, dots, part))) return e;
-    hipLaunchKernelGGL(k_hh_build, dim3(1), dim3(1), 0, g_stream, *lv, yf, i, Xc + (size_t)i * n, Tc, dots, tau);
-    LAUNCH_CHECK();
-    const int nr = k - i - 1;
-    if (nr < 1) continue;
-    mxh_vecs rest = {(void*)(X + 2 * (size_t)(i + 1) * n), n, nullptr};
-    // d_j = v_i^H M x_j = (M v_i)^H x_j
-    if ((e = mxh_dot(MXH_F64, n, nr, mxh_vecs{tmp, 0, nullptr}, rest, dots + 2, part))) return e;
-    hipLaunchKernelGGL(k_hh_axpy, dim3(nb, nr), dim3(TPB), 0, g_stream, n, nr, (const C<double>*)(Xc + (size_t)i * n),
-                       Xc + (size_t)(i + 1) * n, n, tau, i, 0, dots + 2);
-    LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_hh_unitfix, dim3((nr + 63) / 64), dim3(64), 0, g_stream, *lv, yf, i, nr,
-                       Xc + (size_t)(i + 1) * n, n);
-    LAUNCH_CHECK();
-  }
-  // backward pass: V_i = H_0 ... H_i unit_i (edge2d.c:6287-6296), all i at
-  // once: reflection j applied to V_i for i >= j, j from k - 1 down to 0
-  if ((e = (int)hipMemsetAsync(V, 0, sizeof(double) * 2 * (size_t)n * k, g_stream))) return e;
-  hipLaunchKernelGGL(k_hh_units, dim3((k + 63) / 64), dim3(64), 0, g_stream, *lv, k, Vc, n);
-  LAUNCH_CHECK();
-  for (int j = k - 1; j >= 0; j--) {
-    mxh_vecs xj = {(void*)(X + 2 * (size_t)j * n), n, nullptr};
-    if ((e = mxh_addeval(MXH_F64, lv, &bl, 1, xj, mxh_vecs{tmp, n, nullptr}, eta64, &mass, 0))) return e;
-    const int nr = k - j;
-    mxh_vecs vs = {(void*)(V + 2 * (size_t)j * n), n, nullptr};
-    if ((e = mxh_dot(MXH_F64, n, nr, mxh_vecs{tmp, 0, nullptr}, vs, dots, part))) return e;
-    hipLaunchKernelGGL(k_hh_axpy, dim3(nb, nr), dim3(TPB), 0, g_stream, n, nr, (const C<double>*)(Xc + (size_t)j * n),
-                       Vc + (size_t)j * n, n, tau, j, 1, dots);
-    LAUNCH_CHECK();
-  }
-  return 0;
+  (void)eta64;  // M does not depend on it
+  (void)tmp;
+  if (k < 1 || lv->ny < 2 || (long long)k > (long long)lv->nx * (lv->ny / 2)) return (int)hipErrorInvalidValue;
+  const long long n = 2LL * lv->nx * lv->ny;
+  return hh_run(lv, xr, xi, yr, yi, k, HhVecs{(C<double>*)X, n, nullptr}, HhVecs{(C<double>*)V, n, nullptr},
+                work, tau, nullptr);
+}
+
+int mxh_orthonormalize_vecs(const mxh_level* lv, double xr, double xi, double yr, double yi, int k, void* const* x,
+                            double* tau, double* work)
+{
+  if (k < 1 || lv->ny < 2 || (long long)k > (long long)lv->nx * (lv->ny / 2)) return (int)hipErrorInvalidValue;
+  const HhWork wk = hh_work(work, k);
+  void* table = wk.W + 2 * (size_t)k * k;
+  int e = (int)hipMemcpyAsync(table, x, sizeof(void*) * k, hipMemcpyHostToDevice, g_stream);
+  if (e) return e;
+  const HhVecs X{nullptr, 0, (C<double>* const*)table};
+  return hh_run(lv, xr, xi, yr, yi, k, X, X, work, nullptr, tau);
 }
 
 int mxh_gather(int prec, long long n, int nv, mxh_vecs dst, mxh_vecs src)
@@ -5958,6 +6196,31 @@ int mxh_dot(int prec, long long n, int nv, mxh_vecs x, mxh_vecs y, double* out, 
   LAUNCH_CHECK();
   hipLaunchKernelGGL(k_reduce_partials, dim3(reduce_blocks(2 * nv)), dim3(TPB), 0, g_stream, work, (int)nb, 2 * nv, out,
                      0);
+  LAUNCH_CHECK();
+  return 0;
+}
+
+static unsigned product_blocks(long long n)
+{
+  const long long b = (n + PRODUCT_TB - 1) / PRODUCT_TB;
+  // up to four entries a thread one workgroup needs no second sum
+  return (unsigned)(b <= 4 ? 1 : b < PRODUCT_BLOCKS ? b : PRODUCT_BLOCKS);
+}
+
+int mxh_product_edge(const mxh_level* lv, const mxh_bloch* bl, const void* x, const void* y, const double* eta,
+                     const mxh_coef* cf, double* work, double* out, double mark)
+{
+  const long long N = (long long)lv->nx * lv->ny;
+  hipLaunchKernelGGL(k_product<1>, dim3(product_blocks(N)), dim3(PRODUCT_TB), 0, g_stream, *lv, *bl, 2 * N,
+                     (const C<double>*)x, (const C<double>*)y, eta, *cf, work, out, mark);
+  LAUNCH_CHECK();
+  return 0;
+}
+
+int mxh_product(long long n, const void* x, const void* y, double* work, double* out, double mark)
+{
+  hipLaunchKernelGGL(k_product<0>, dim3(product_blocks(n)), dim3(PRODUCT_TB), 0, g_stream, mxh_level(), mxh_bloch(), n,
+                     (const C<double>*)x, (const C<double>*)y, (const double*)nullptr, mxh_coef(), work, out, mark);
   LAUNCH_CHECK();
   return 0;
 }
