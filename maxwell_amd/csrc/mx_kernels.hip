@@ -2871,22 +2871,24 @@ __global__ __launch_bounds__(256) void k_random(long long n, C<T>* X, long long 
 }
 
 // ----------------------------------------------------------------- adjoint
-__global__ __launch_bounds__(256) void k_curl2(mxh_level lv, mxh_bloch bl, int nv, const C<double>* E,
-                                               long long es, const double* w, double* grad)
+// sum_v |curl e_v|_c^2 / (hx hy) / (e_v^H M e_v) per cell, with the M-norms taken
+// from the Gram sums of the vectors (pair (v, v)).  out may be host memory.
+__global__ __launch_bounds__(256) void k_eta_grad(mxh_level lv, mxh_bloch bl, int nv, const C<double>* E,
+                                                 long long es, const double* gram, double* out)
 {
   const size_t N = (size_t)lv.nx * lv.ny;
   size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= N) return;
-  const int i = (int)(idx % lv.nx), j = (int)(idx / lv.nx);
+  const int j = (int)((unsigned)idx / (unsigned)lv.nx), i = (int)idx - j * lv.nx;
   const double s = 1.0 / (lv.hx * lv.hy);
   double acc = 0.0;
   for (int v = 0; v < nv; v++) {
     Geo<double> g = make_geo<double>(lv, bl, v);
     EdgeV<double> e = edge_view<double>(E, es, v, N);
     C<double> c = cell_curl(g, e, i, j);
-    acc += w[v] * (c.r * c.r + c.i * c.i) * s;
+    acc += (1.0 / gram[4 * (v * (v + 1) / 2 + v) + 2]) * (c.r * c.r + c.i * c.i) * s;
   }
-  grad[idx] += acc;
+  out[idx] = acc;
 }
 
 // ----------------------------------------------------------------- tile-fused AFW sweeps
@@ -6298,11 +6300,11 @@ int mxh_random(int prec, long long n, int nv, mxh_vecs x, unsigned long long see
   return 0;
 }
 
-int mxh_curl2(const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs e, const double* w, double* grad)
+int mxh_eta_grad(const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs e, const double* gram, double* out)
 {
   const long long N = (long long)lv->nx * lv->ny;
-  hipLaunchKernelGGL(k_curl2, dim3(nblocks(N)), dim3(TPB), 0, g_stream, *lv, *bl, nv, (const C<double>*)e.p,
-                     e.stride, w, grad);
+  hipLaunchKernelGGL(k_eta_grad, dim3(nblocks(N)), dim3(TPB), 0, g_stream, *lv, *bl, nv, (const C<double>*)e.p,
+                     e.stride, gram, out);
   LAUNCH_CHECK();
   return 0;
 }
