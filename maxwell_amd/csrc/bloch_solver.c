@@ -53,6 +53,9 @@ struct mx_solver {
   int ne0, nn0;         /* coarse edge / node unknowns */
   /* host scratch */
   double complex *hAe, *hAn;
+  double complex *hC;    /* LOBPCG: 3m x 2m coefficients per problem */
+  double *hgram;         /* LOBPCG: Gram sums (pinned) */
+  void *ev_gram[2];      /* LOBPCG: Gram sums of each half on the host */
   int *hwvalid;         /* LOBPCG: vector's W column written this step */
   int pvalid;           /* LOBPCG: the P columns hold a search direction
                            (from the second Ritz step of the loop on) */
@@ -141,6 +144,10 @@ void mx_solver_destroy(mx_solver *s)
   free(s->hAe);
   free(s->hAn);
   free(s->hwvalid);
+  free(s->hC);
+  mxh_host_free(s->hgram);
+  for (int h = 0; h < 2; h++)
+    if (s->ev_gram[h]) mxh_event_destroy(s->ev_gram[h]);
   mxh_host_free(s->hnorm);
   mxh_host_free(s->hgrad);
   free(s->hbloch);
@@ -294,6 +301,12 @@ int mx_solver_create(const mx_config *cfg, const double *eta, mx_solver **out)
   s->hAe = (double complex *)malloc(sizeof(double complex) * (size_t)s->ne0 * s->ne0 * P);
   s->hAn = (double complex *)malloc(sizeof(double complex) * (size_t)s->nn0 * s->nn0 * P);
   s->hwvalid = (int *)calloc((size_t)nv, sizeof(int));
+  if (s->lobpcg) {
+    s->hC = (double complex *)malloc(sizeof(double complex) * (size_t)vpp * m * 2 * P);
+    s->hgram = (double *)mxh_host_alloc(sizeof(double) * 4 * (size_t)vpp * vpp * P);
+    for (int h = 0; h < 2; h++)
+      if (mxh_event_create(&s->ev_gram[h])) s->ev_gram[h] = NULL;
+  }
   s->hnorm = (double *)mxh_host_alloc(step_bytes(s));
   s->hlam = s->hnorm + 2 * (size_t)nv;
   s->hstat = (int *)(s->hlam + (size_t)vpp * P);
@@ -306,7 +319,8 @@ int mx_solver_create(const mx_config *cfg, const double *eta, mx_solver **out)
   s->dcols = (int *)dalloc(s, sizeof(int) * (size_t)(vpp + 1) * P);
   s->dinfo = (int *)dalloc(s, sizeof(int) * P);
   s->hinfo = (int *)malloc(sizeof(int) * P);
-  if (!s->hAe || !s->hAn || !s->hwvalid || !s->hnorm || !s->hbloch ||
+  if ((s->lobpcg && (!s->hC || !s->hgram || !s->ev_gram[0] || !s->ev_gram[1])) ||
+      !s->hAe || !s->hAn || !s->hwvalid || !s->hnorm || !s->hbloch ||
       !s->gamma || !s->hlist || !s->hslot || !s->dlist || !s->dinfo || !s->hinfo || !s->hcols || !s->dcols)
     goto nomem;
   if (mxh_sync()) goto dev;
@@ -662,6 +676,98 @@ static int lift(mx_solver *s, int nv, const mxh_bloch *bl, double *E, const void
 #define PINVIT_PIVOT 1e-13
 #define LOBPCG_PIVOT 1e-7
 
+/* LOBPCG's small eigenproblems of the list's problems j0 <= j < j1 on the host,
+   from the Gram sums in hgram: the lowest m Ritz pairs give hlam and two
+   coefficient blocks per problem in hC (3m x 2m, column-major): E_new = [E W P]
+   C_E and the next search direction P_new = [W P] C_WP (the W and P rows of
+   C_E).  mxh_ritz solves the same problems, but its parallel Jacobi leaves
+   larger errors in the small components of the lowest vectors when the basis
+   holds directions of rounding noise: next to the Gamma point (|k| = 0.17 on
+   512^2) the first pair then stalled above a tolerance of 1e-8 in 6 of 40 start
+   blocks, in none with the sequential order; and at 3m = 36 the host works
+   beside the device (720 ms a solve against 728). */
+static int lobpcg_problem(mx_solver *s, int j, int p)
+{
+  const int m = s->cfg.block, L = s->L, k = 3 * m, np = k * (k + 1) / 2;
+  const double sk = 1.0 / (s->lv[L].hx * s->lv[L].hy);
+  double w[48], dsc[48];
+  int keep[48];
+  double complex A[48 * 48], B[48 * 48], Lf[48 * 48], As[48 * 48], Bs[48 * 48];
+  const double *g = s->hgram + 4 * (size_t)np * j;
+  /* the Gram holds the problem's listed columns (E, the W of its unlocked
+     vectors, P once it holds a direction) at list positions 0 .. kc - 1 */
+  const int *cl = s->hcols + (size_t)p * (k + 1), kc = cl[0];
+  for (int q = 0; q < 2 * kc * (kc + 1); q++)
+    if (!isfinite(g[q])) return MX_ENOTFINITE;
+  for (int a = 0; a < kc; a++)
+    for (int c = 0; c <= a; c++) {
+      const double *q = g + 4 * (a * (a + 1) / 2 + c);
+      const double complex gk = q[0] + I * q[1], gm = q[2] + I * q[3];
+      A[a + c * k] = sk * gk + gm;
+      B[a + c * k] = gm;
+      A[c + a * k] = conj(A[a + c * k]);
+      B[c + a * k] = conj(gm);
+    }
+  /* greedy column selection by a Cholesky factorisation of the scaled B */
+  int kk = 0;
+  for (int c = 0; c < kc; c++) {
+    const double bcc = creal(B[c + c * k]);
+    if (!(bcc > 0.0) || !isfinite(bcc)) continue;
+    const double d = 1.0 / sqrt(bcc);
+    /* row kk of the factor of the scaled B restricted to the kept columns */
+    double piv = 1.0;
+    for (int t = 0; t < kk; t++) {
+      double complex z = B[c + keep[t] * k] * d * dsc[t];
+      for (int u = 0; u < t; u++) z -= Lf[kk + u * 48] * conj(Lf[t + u * 48]);
+      z /= creal(Lf[t + t * 48]);
+      Lf[kk + t * 48] = z;
+      piv -= creal(z * conj(z));
+    }
+    if (!(piv > LOBPCG_PIVOT)) continue;
+    Lf[kk + kk * 48] = sqrt(piv);
+    keep[kk] = c;
+    dsc[kk] = d;
+    kk++;
+  }
+  if (kk < m) return MX_ELAPACK;
+  for (int t = 0; t < kk; t++)
+    for (int u = 0; u < kk; u++) {
+      As[t + u * kk] = A[keep[t] + keep[u] * k] * dsc[t] * dsc[u];
+      Bs[t + u * kk] = B[keep[t] + keep[u] * k] * dsc[t] * dsc[u];
+    }
+  if (mxd_hegv(kk, As, Bs, w)) return MX_ELAPACK;
+  double complex *Cp = s->hC + (size_t)j * k * 2 * m;
+  for (int q = 0; q < k * 2 * m; q++) Cp[q] = 0.0;
+  for (int i = 0; i < m; i++) {
+    s->hlam[(size_t)p * s->vpp + i] = w[i];
+    for (int t = 0; t < kk; t++) {
+      const int c = cl[1 + keep[t]];
+      const double complex cf = As[t + i * kk] * dsc[t];
+      Cp[c + (size_t)i * k] = cf;
+      if (c >= m) Cp[c + (size_t)(m + i) * k] = cf;
+    }
+  }
+  return MX_OK;
+}
+
+/* The problems are independent (each writes its own hC block and hlam
+   entries), so a team of host threads shares them: at 3m = 36 one
+   eigensolve takes about 2 ms, against a few ms of GPU work per half-batch
+   that it has to hide behind. */
+static int ritz_host_lobpcg(mx_solver *s, int j0, int j1, const int *plist)
+{
+  int status = MX_OK;
+#pragma omp parallel for schedule(dynamic, 1) if (j1 - j0 > 1)
+  for (int j = j0; j < j1; j++) {
+    const int e = lobpcg_problem(s, j, plist ? plist[j] : j);
+    if (e) {
+#pragma omp critical(mx_ritz_status)
+      if (!status) status = e;
+    }
+  }
+  return status;
+}
+
 /* Launches the defects (K + (1 - lam) M) e of nv listed vectors (dvlist:
    device, null = 0..nv-1) into slots slot0 .. slot0 + nv - 1 of r (next
    right-hand sides, MG precision) and their norms to dnorm, without waiting. */
@@ -681,12 +787,12 @@ static int defect_launch(mx_solver *s, int nv, const int *dvlist, double *E, voi
 }
 
 /* Rayleigh-Ritz over the blocks of the listed problems (plist on the host,
-   dplist on the device): Gram sums, the small eigenproblems (mxh_ritz),
+   dplist on the device): Gram sums, the small eigenproblems,
    Eout = Ein C; then the defects of Eout's vectors (the m of each listed
-   problem in list order: dvlist, nvl = na m) to r.  Norms, Ritz values and
-   statuses come back in one copy, the step's only wait.  On the host the
-   eigenproblems (12 x 12: 20-40 us each, 36 x 36: 1 ms) held the GPU up: 64^2 FP64,
-   16 problems, 680 us a step against 450 us of kernels. */
+   problem in list order: dvlist, nvl = na m) to r.  PINVIT: norms, Ritz
+   values and statuses come back in one copy, the step's only wait (on the host
+   the 12 x 12 problems held the GPU up: 64^2 FP64, 16 problems, 680 us a step
+   against 450 us of kernels). */
 static int ritz_defect(mx_solver *s, int na, const int *plist, const int *dplist, int nvl, const int *dvlist,
                        double *Ein, double *Eout, void *r)
 {
@@ -710,17 +816,39 @@ static int ritz_defect(mx_solver *s, int na, const int *plist, const int *dplist
       cl[0] = c;
     }
     CK(mxh_h2d(s->dcols, s->hcols, sizeof(int) * (size_t)(mg + 1) * s->last_nprob));
-    CK(mxh_gram_cols(&s->lv[L], &bl, na, dplist, s->dcols, mg, V(Ein, s->es), s->eta64[L], s->dgram, s->gramwork));
-    CK(mxh_ritz(m, mg, na, dplist, s->dcols, s->dgram, sk, LOBPCG_PIVOT, s->dC, s->dlam, mg, s->dstat));
-  } else {
-    CK(mxh_gram(&s->lv[L], &bl, na, dplist, mg, V(Ein, s->es), s->eta64[L], s->dgram, s->gramwork));
-    CK(mxh_ritz(m, 0, na, dplist, NULL, s->dgram, sk, PINVIT_PIVOT, s->dC, s->dlam, mg, s->dstat));
+    /* in two halves: the host's eigensolves of one run while the GPU sums the
+       other's Gram products or updates and checks it */
+    const int np = mg * (mg + 1) / 2, csz = mg * 2 * m, split = na >= 2;
+    const int nh[2] = {split ? (na + 1) / 2 : na, split ? na / 2 : 0};
+    for (int h = 0, j0 = 0; h < 2 && nh[h]; j0 += nh[h], h++) {
+      double *gout = s->dgram + 4 * (size_t)np * j0;
+      CK(mxh_gram_cols(&s->lv[L], &bl, nh[h], dplist + j0, s->dcols, mg, V(Ein, s->es), s->eta64[L], gout, s->gramwork));
+      CK(mxh_d2h_async(s->hgram + 4 * (size_t)np * j0, gout, sizeof(double) * 4 * (size_t)np * nh[h]));
+      CK(mxh_event_record(s->ev_gram[h]));
+      s->st.launches += 3;
+    }
+    for (int h = 0, j0 = 0; h < 2 && nh[h]; j0 += nh[h], h++) {
+      CK(mxh_event_sync(s->ev_gram[h]));
+      if ((e = ritz_host_lobpcg(s, j0, j0 + nh[h], plist))) {
+        mxh_sync();
+        return e;
+      }
+      double *dC = s->dC + 2 * (size_t)j0 * csz;
+      CK(mxh_h2d(dC, s->hC + (size_t)j0 * csz, sizeof(double complex) * (size_t)csz * nh[h]));
+      CK(mxh_h2d(s->dlam, s->hlam, sizeof(double) * (size_t)mg * s->last_nprob));
+      if (!(m & 1)) /* [E W P] -> E_new (slots 0..m-1), P_new (slots 2m..3m-1) */
+        CK(mxh_lobpcg_combine(n, nh[h], dplist + j0, m, V(Ein, s->es), V(Eout, s->es), dC));
+      else
+        CK(mxh_combine_x(n, nh[h], dplist + j0, mg, 2 * m, m, m, V(Ein, s->es), mg, V(Eout, s->es), mg, dC));
+      s->st.launches++;
+      if ((e = defect_launch(s, nh[h] * m, dvlist + j0 * m, Eout, r, j0 * m))) return e;
+    }
+    CK(mxh_d2h(s->hnorm, s->dnorm, sizeof(double) * 2 * nvl));
+    return MX_OK;
   }
-  if (s->lobpcg && !(m & 1)) /* [E W P] -> E_new (slots 0..m-1), P_new (slots 2m..3m-1) */
-    CK(mxh_lobpcg_combine(n, na, dplist, m, V(Ein, s->es), V(Eout, s->es), s->dC));
-  else if (s->lobpcg)
-    CK(mxh_combine_x(n, na, dplist, mg, 2 * m, m, m, V(Ein, s->es), mg, V(Eout, s->es), mg, s->dC));
-  else if (m > 16)  /* every input read once */
+  CK(mxh_gram(&s->lv[L], &bl, na, dplist, mg, V(Ein, s->es), s->eta64[L], s->dgram, s->gramwork));
+  CK(mxh_ritz(m, 0, na, dplist, NULL, s->dgram, sk, PINVIT_PIVOT, s->dC, s->dlam, mg, s->dstat));
+  if (m > 16)  /* every input read once */
     CK(mxh_combine_x(n, na, dplist, m, m, m, 0, V(Ein, s->es), m, V(Eout, s->es), m, s->dC));
   else
     CK(mxh_block_combine(n, na, dplist, m, V(Ein, s->es), V(Eout, s->es), s->dC));

@@ -1108,9 +1108,8 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gram(mxh_level lv, mxh
 // barrier): 54 us for 16 problems of 9 columns and 638 us for 64 of 36, of
 // which all run at once.  On the host the same problems took 0.5 to 1 ms
 // between device steps that wait for them (64^2 grids in FP64, 16 problems: a
-// solve of 80 ms against 56) and needed two transfers; at 512^2 and 36 columns,
-// where the host could work beside the device, both ways are alike (720 ms
-// against 728).
+// solve of 80 ms against 56) and needed two transfers.  LOBPCG's bases of three
+// blocks stay on the host (bloch_solver.c says why).
 #define RITZ_MAX 48
 
 MXH_DEV double rsqrt64(double a)
