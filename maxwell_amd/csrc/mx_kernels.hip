@@ -173,28 +173,6 @@ MXH_DEV void apply_at(const Geo<T>& g, const EdgeV<T>& e, const T* eta, int i, i
   oy = axy * ky + my * (T(4) * y00 + ym0 + yp0);
 }
 
-// K x (without 1/(hx hy)) and the M stencils at x-edge (i,j) and y-edge (i,j),
-// neighbours read through the Bloch wrap (frame points of the grid).
-template <typename T>
-MXH_DEV void stencil2(const Geo<T>& g, const C<T>* ex, const C<T>* ey, const T* eta, int i, int j, C<T>& kx,
-                      C<T>& ky, C<T>& mxs, C<T>& mys, C<T>& x00, C<T>& y00)
-{
-  x00 = g.at(ex, i, j);
-  y00 = g.at(ey, i, j);
-  const C<T> x0m = g.at(ex, i, j - 1), x0p = g.at(ex, i, j + 1);
-  const C<T> xm0 = g.at(ex, i - 1, j), xmp = g.at(ex, i - 1, j + 1);
-  const C<T> ym0 = g.at(ey, i - 1, j), yp0 = g.at(ey, i + 1, j);
-  const C<T> y0m = g.at(ey, i, j - 1), ypm = g.at(ey, i + 1, j - 1);
-  const T e00 = eta_at(eta, g.nx, g.ny, i, j), e0m = eta_at(eta, g.nx, g.ny, i, j - 1), em0 = eta_at(eta, g.nx, g.ny, i - 1, j);
-  const C<T> c00 = x00 - x0p - y00 + yp0;  // cell (i,j)
-  const C<T> c0m = x0m - x00 - y0m + ypm;  // cell (i,j-1)
-  const C<T> cm0 = xm0 - xmp - ym0 + y00;  // cell (i-1,j)
-  kx = e00 * c00 - e0m * c0m;
-  ky = em0 * cm0 - e00 * c00;
-  mxs = T(4) * x00 + x0m + x0p;
-  mys = T(4) * y00 + ym0 + yp0;
-}
-
 template <typename T>
 MXH_DEV void coefs(const mxh_level& lv, const mxh_coef& cf, int v, C<T>& axy, C<T>& mx, C<T>& my)
 {
@@ -303,6 +281,39 @@ MXH_DEV int row_end(int ny)
   return min(ny, ((int)blockIdx.x + 1) * rpb);
 }
 
+// The defect's map: a workgroup of 256 threads covers bands of rows of one
+// vector, a thread walks its columns (i0, i0 + 256, ...) down rows j0 .. j1 - 1,
+// so the neighbouring rows a stencil reads were read by the same thread or its
+// neighbours just before.  Grids of at most 128 columns put 256 / nx bands side
+// by side into a workgroup (84^2 in FP64, 194 vectors, defect: 41 -> 23 us).
+template <bool NARROW>
+struct Band {
+  int i0, j0, j1;  // no rows: j0 = j1
+  MXH_DEV Band(int nx, int ny)
+  {
+    const int groups = NARROW ? 256 / nx : 1, q = NARROW ? (int)threadIdx.x / nx : 0;
+    const int bands = (int)gridDim.x * groups, rpb = (ny + bands - 1) / bands;
+    i0 = (int)threadIdx.x - q * nx;
+    const int b = q < groups ? (int)blockIdx.x * groups + q : bands;
+    j0 = min(ny, b * rpb);
+    j1 = min(ny, j0 + rpb);
+  }
+};
+static inline bool narrow(const mxh_level* lv) { return lv->nx <= 128; }
+// Its workgroups per vector: four rows a band, fewer where that leaves the chip
+// short of workgroups (four per compute unit), BAND_MAX at most (the partial
+// sums' places).
+#define BAND_MAX 128
+#define BAND_SHORT 4
+static inline unsigned band_blocks(const mxh_level* lv, int nv, int rows)
+{
+  const int groups = narrow(lv) ? 256 / lv->nx : 1;
+  auto blocks = [&](int r) { return (lv->ny + groups * r - 1) / (groups * r); };
+  while (rows > 1 && (long long)nv * blocks(rows) < 1024) rows >>= 1;
+  const int nb = blocks(rows);
+  return (unsigned)(nb < 1 ? 1 : nb < BAND_MAX ? nb : BAND_MAX);
+}
+
 // The frame of an nx x ny grid (rows 0 and ny - 1, columns 0 and nx - 1):
 // the points whose stencils wrap.  The row-mapped kernels run the interior
 // with direct indexing and the frame in a second, small launch with the
@@ -362,26 +373,16 @@ __global__ __launch_bounds__(256) void k_addeval(mxh_level lv, mxh_bloch bl, con
 
 // PINVIT defect r = (K + (1 - lam) M) e in FP64, stored in precision R, plus
 // per-block partial sums of |r|^2 and |M e|^2 over the block's band of rows.
-template <typename R>
-MXH_DEV void defect_point(const Geo<double>& g, const C<double>* ex, const C<double>* ey, const double* eta, int i,
-                          int j, double s, double sx, double sy, double be, C<R>* r, size_t N, double& rr,
-                          double& mm)
-{
-  C<double> kx, ky, mxs, mys, x00, y00;
-  stencil2(g, ex, ey, eta, i, j, kx, ky, mxs, mys, x00, y00);
-  const C<double> mxv = sx * mxs, myv = sy * mys;
-  const C<double> ox = s * kx + be * mxv, oy = s * ky + be * myv;
-  const size_t k = i + (size_t)j * g.nx;
-  r[k] = ccast<R>(ox);
-  r[N + k] = ccast<R>(oy);
-  rr += ox.r * ox.r + ox.i * ox.i + oy.r * oy.r + oy.i * oy.i;
-  mm += mxv.r * mxv.r + mxv.i * mxv.i + myv.r * myv.r + myv.i * myv.i;
-}
-
-template <typename R, bool FRAME>
+//
+// Each thread walks its columns down the band, keeping the values the next
+// row's stencil shares with this one (half the loads per point).  Columns start
+// at 0 (whole cache lines per wave); the Bloch factors are applied in the first
+// and last column and row only.  192 vectors of 512^2 in mixed precision: 548 ->
+// 482 us with its reduction (4.4 -> 5.0 TB/s).
+template <typename R, bool NARROW>
 __global__ __launch_bounds__(256) void k_defect(mxh_level lv, mxh_bloch bl, const C<double>* E, long long es,
                                                 const int* emap, C<R>* Rv, long long rs, const double* eta,
-                                                const double* lam, double* part, int slot0)
+                                                const double* lam, double* part)
 {
   __shared__ double sh[4];
   const int v = blockIdx.y;
@@ -394,52 +395,63 @@ __global__ __launch_bounds__(256) void k_defect(mxh_level lv, mxh_bloch bl, cons
   const EdgeV<double> e = edge_view<double>(E, es, gv, N);
   C<R>* r = Rv + (size_t)v * rs;
   double rr = 0.0, mm = 0.0;
-  if (FRAME) {
-    const int nf = (int)frame_points(nx, ny);
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nf; k += gridDim.x * blockDim.x) {
-      int i, j;
-      frame_point(k, nx, ny, i, j);
-      defect_point<R>(g, e.x, e.y, eta, i, j, s, sx, sy, be, r, N, rr, mm);
-    }
-  } else {
-    // each thread walks its columns down the band, keeping the values the
-    // next row's stencil shares with this one (half the loads per point)
-    const int j0 = max(1, row_first(ny)), j1 = min(ny - 1, row_end(ny));
-    const C<double>* ex = e.x;
-    const C<double>* ey = e.y;
-    if (j0 < j1)
-      for (int i = 1 + (int)threadIdx.x; i < nx - 1; i += blockDim.x) {
-        size_t k = i + (size_t)j0 * nx;
-        C<double> x0m = ex[k - nx], x00 = ex[k], xm0 = ex[k - 1];
-        C<double> y0m = ey[k - nx], ypm = ey[k - nx + 1];
-        double e0m = eta[k - nx];
-        for (int j = j0; j < j1; j++, k += nx) {
-          const C<double> x0p = ex[k + nx], xmp = ex[k + nx - 1];
-          const C<double> y00 = ey[k], ym0 = ey[k - 1], yp0 = ey[k + 1];
-          const double e00 = eta[k], em0 = eta[k - 1];
-          const C<double> c00 = x00 - x0p - y00 + yp0;  // cell (i,j)
-          const C<double> c0m = x0m - x00 - y0m + ypm;  // cell (i,j-1)
-          const C<double> cm0 = xm0 - xmp - ym0 + y00;  // cell (i-1,j)
-          const C<double> kx = e00 * c00 - e0m * c0m, ky = em0 * cm0 - e00 * c00;
-          const C<double> mxv = sx * (4.0 * x00 + x0m + x0p), myv = sy * (4.0 * y00 + ym0 + yp0);
-          const C<double> ox = s * kx + be * mxv, oy = s * ky + be * myv;
-          r[k] = ccast<R>(ox);
-          r[N + k] = ccast<R>(oy);
-          rr += ox.r * ox.r + ox.i * ox.i + oy.r * oy.r + oy.i * oy.i;
-          mm += mxv.r * mxv.r + mxv.i * mxv.i + myv.r * myv.r + myv.i * myv.i;
-          x0m = x00;
-          x00 = x0p;
-          xm0 = xmp;
-          y0m = y00;
-          ypm = yp0;
-          e0m = e00;
-        }
+  const Band<NARROW> band(nx, ny);
+  const int j0 = band.j0, j1 = band.j1;
+  const C<double>* ex = e.x;
+  const C<double>* ey = e.y;
+  if (j0 < j1)
+    for (int i = band.i0; i < nx; i += 256) {
+      const bool wl = i == 0, wr = i == nx - 1;
+      const int im = wl ? nx - 1 : i - 1, ip = wr ? 0 : i + 1;
+      const size_t below = (size_t)(j0 ? j0 - 1 : ny - 1) * nx;
+      size_t k = (size_t)j0 * nx;
+      C<double> x0m = ex[below + i], x00 = ex[k + i], xm0 = ex[k + im];
+      C<double> y0m = ey[below + i], ypm = ey[below + ip];
+      double e0m = eta[below + i];
+      if (wl) xm0 = cconj(g.xf) * xm0;
+      if (wr) ypm = g.xf * ypm;
+      if (j0 == 0) {
+        x0m = cconj(g.yf) * x0m;
+        y0m = cconj(g.yf) * y0m;
+        ypm = cconj(g.yf) * ypm;
       }
-  }
+      for (int j = j0; j < j1; j++, k += nx) {
+        const size_t above = j + 1 < ny ? k + nx : 0;
+        C<double> x0p = ex[above + i], xmp = ex[above + im];
+        C<double> ym0 = ey[k + im], yp0 = ey[k + ip];
+        const C<double> y00 = ey[k + i];
+        const double e00 = eta[k + i], em0 = eta[k + im];
+        if (wl) {
+          xmp = cconj(g.xf) * xmp;
+          ym0 = cconj(g.xf) * ym0;
+        }
+        if (wr) yp0 = g.xf * yp0;
+        if (j + 1 == ny) {
+          x0p = g.yf * x0p;
+          xmp = g.yf * xmp;
+        }
+        const C<double> c00 = x00 - x0p - y00 + yp0;  // cell (i,j)
+        const C<double> c0m = x0m - x00 - y0m + ypm;  // cell (i,j-1)
+        const C<double> cm0 = xm0 - xmp - ym0 + y00;  // cell (i-1,j)
+        const C<double> kx = e00 * c00 - e0m * c0m, ky = em0 * cm0 - e00 * c00;
+        const C<double> mxv = sx * (4.0 * x00 + x0m + x0p), myv = sy * (4.0 * y00 + ym0 + yp0);
+        const C<double> ox = s * kx + be * mxv, oy = s * ky + be * myv;
+        r[k + i] = ccast<R>(ox);
+        r[N + k + i] = ccast<R>(oy);
+        rr += ox.r * ox.r + ox.i * ox.i + oy.r * oy.r + oy.i * oy.i;
+        mm += mxv.r * mxv.r + mxv.i * mxv.i + myv.r * myv.r + myv.i * myv.i;
+        x0m = x00;
+        x00 = x0p;
+        xm0 = xmp;
+        y0m = y00;
+        ypm = yp0;
+        e0m = e00;
+      }
+    }
   double a = block_sum256(rr, sh);
   double b = block_sum256(mm, sh);
   if (threadIdx.x == 0) {
-    size_t w = (size_t)(slot0 + blockIdx.x) * (2 * gridDim.y) + 2 * v;
+    size_t w = (size_t)blockIdx.x * (2 * gridDim.y) + 2 * v;
     part[w] = a;
     part[w + 1] = b;
   }
@@ -5079,22 +5091,27 @@ int mxh_addeval(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_
 int mxh_defect(int rprec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs e, mxh_vecs r,
                const double* eta64, const double* lam, double* out, double* work)
 {
-  const unsigned nb = row_blocks(lv->ny), nf = frame_blocks(lv);
-  const dim3 grid(nb, nv), gridf(nf, nv);
-  if (rprec == MXH_F64) {
-    hipLaunchKernelGGL((k_defect<double, false>), grid, dim3(TPB), 0, g_stream, *lv, *bl, (const C<double>*)e.p,
-                       e.stride, e.map, (C<double>*)r.p, r.stride, eta64, lam, work, 0);
-    hipLaunchKernelGGL((k_defect<double, true>), gridf, dim3(TPB), 0, g_stream, *lv, *bl, (const C<double>*)e.p,
-                       e.stride, e.map, (C<double>*)r.p, r.stride, eta64, lam, work, (int)nb);
-  } else {
-    hipLaunchKernelGGL((k_defect<float, false>), grid, dim3(TPB), 0, g_stream, *lv, *bl, (const C<double>*)e.p,
-                       e.stride, e.map, (C<float>*)r.p, r.stride, eta64, lam, work, 0);
-    hipLaunchKernelGGL((k_defect<float, true>), gridf, dim3(TPB), 0, g_stream, *lv, *bl, (const C<double>*)e.p,
-                       e.stride, e.map, (C<float>*)r.p, r.stride, eta64, lam, work, (int)nb);
-  }
+  const unsigned nb = band_blocks(lv, nv, BAND_SHORT);
+  const dim3 grid(nb, nv);
+  if (rprec == MXH_F64)
+    {
+      auto go = [&](auto k) {
+        hipLaunchKernelGGL(k, grid, dim3(TPB), 0, g_stream, *lv, *bl, (const C<double>*)e.p, e.stride,
+                           e.map, (C<double>*)r.p, r.stride, eta64, lam, work);
+      };
+      narrow(lv) ? go(k_defect<double, true>) : go(k_defect<double, false>);
+    }
+  else
+    {
+      auto go = [&](auto k) {
+        hipLaunchKernelGGL(k, grid, dim3(TPB), 0, g_stream, *lv, *bl, (const C<double>*)e.p, e.stride,
+                           e.map, (C<float>*)r.p, r.stride, eta64, lam, work);
+      };
+      narrow(lv) ? go(k_defect<float, true>) : go(k_defect<float, false>);
+    }
   LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_reduce_partials, dim3(reduce_blocks(2 * nv)), dim3(TPB), 0, g_stream, work, (int)(nb + nf),
-                     2 * nv, out, 0);
+  hipLaunchKernelGGL(k_reduce_partials, dim3(reduce_blocks(2 * nv)), dim3(TPB), 0, g_stream, work, (int)nb, 2 * nv,
+                     out, 0);
   LAUNCH_CHECK();
   return 0;
 }
