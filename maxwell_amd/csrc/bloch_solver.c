@@ -680,12 +680,9 @@ static int lift(mx_solver *s, int nv, const mxh_bloch *bl, double *E, const void
    from the Gram sums in hgram: the lowest m Ritz pairs give hlam and two
    coefficient blocks per problem in hC (3m x 2m, column-major): E_new = [E W P]
    C_E and the next search direction P_new = [W P] C_WP (the W and P rows of
-   C_E).  mxh_ritz solves the same problems, but its parallel Jacobi leaves
-   larger errors in the small components of the lowest vectors when the basis
-   holds directions of rounding noise: next to the Gamma point (|k| = 0.17 on
-   512^2) the first pair then stalled above a tolerance of 1e-8 in 6 of 40 start
-   blocks, in none with the sequential order; and at 3m = 36 the host works
-   beside the device (720 ms a solve against 728). */
+   C_E).  mxh_ritz solves the same problems as accurately; at 3m = 36 the host is
+   no slower, since it works on one half beside the device (512^2, 64 problems:
+   720 ms a solve against 728). */
 static int lobpcg_problem(mx_solver *s, int j, int p)
 {
   const int m = s->cfg.block, L = s->L, k = 3 * m, np = k * (k + 1) / 2;

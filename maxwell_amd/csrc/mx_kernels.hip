@@ -1114,6 +1114,13 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gram(mxh_level lv, mxh
 // without their first m rows.  status: 0, 1 a sum is not finite, 2 fewer than
 // m columns kept; the coefficients are then 0.
 //
+// A rotation is (c, -f; conj(f), c) with c real (and exactly 1 for an angle whose
+// square is lost against 1), not one that turns a column by a phase: a pair that
+// has converged keeps the coefficient 1 and its vector every bit.  Multiplied by
+// a new phase in each step it is rounded anew, and where rounding is all its
+// residual holds (eps |K| / lambda: 1e-8 on 512^2 at |k| = 0.12) the pair leaves
+// the tolerance again: of 64 LOBPCG start blocks 14 stalled that way, 0 do now.
+//
 // Everything stays in LDS in FP64; a step of a factorisation or substitution
 // has one barrier, a Jacobi round two.  What bounds it is that chain (per round
 // a rotation's square roots, a barrier, the LDS reads and writes of A and V, a
@@ -1121,7 +1128,7 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gram(mxh_level lv, mxh
 // which all run at once.  On the host the same problems took 0.5 to 1 ms
 // between device steps that wait for them (64^2 grids in FP64, 16 problems: a
 // solve of 80 ms against 56) and needed two transfers.  LOBPCG's bases of three
-// blocks stay on the host (bloch_solver.c says why).
+// blocks stay on the host, where they run beside the device (bloch_solver.c).
 #define RITZ_MAX 48
 
 MXH_DEV double rsqrt64(double a)
@@ -1141,8 +1148,8 @@ __global__ __launch_bounds__(1024) void k_ritz(int m, int basis, const int* pmap
   const int* cl = cmap ? cmap + (size_t)prob * (k + 1) : nullptr;
   const int n = cl ? min(cl[0], k) : k;
   C<double>*A = (C<double>*)smem, *B = A + n * n, *Vv = B + n * n;
-  __shared__ double dsc[RITZ_MAX], w[RITZ_MAX], rc[RITZ_MAX / 2], rs[RITZ_MAX / 2], red[16];
-  __shared__ C<double> re[RITZ_MAX / 2];
+  __shared__ double dsc[RITZ_MAX], w[RITZ_MAX], rc[RITZ_MAX / 2], red[16];
+  __shared__ C<double> rs[RITZ_MAX / 2];
   __shared__ int keep[RITZ_MAX], ord[RITZ_MAX], bad;
   const double* g = gram + 4 * (size_t)np * jb;
   const int csz = basis ? basis * 2 * m : m * m;
@@ -1287,8 +1294,8 @@ __global__ __launch_bounds__(1024) void k_ritz(int m, int basis, const int* pmap
       };
       if (tid < h) {
         const int p = first(tid), q = second(tid);
-        double cs = 1.0, sn = 0.0;
-        C<double> e = cmk(1.0, 0.0);
+        double cs = 1.0;
+        C<double> f = czero<double>();
         if (p < kk) {
           const C<double> z = A[p + q * kk];
           const double z2 = z.r * z.r + z.i * z.i;
@@ -1296,14 +1303,13 @@ __global__ __launch_bounds__(1024) void k_ritz(int m, int basis, const int* pmap
             const double ri = rsqrt64(z2), r = z2 * ri, d = A[q + q * kk].r - A[p + p * kk].r;
             const double s2 = d * d + 4.0 * z2;
             const double t = copysign(2.0 * r, d) * recip(fabs(d) + s2 * rsqrt64(s2));
-            cs = rsqrt64(1.0 + t * t);
-            sn = t * cs;
-            e = ri * cconj(z);
+            // exactly 1 for the angles that leave a column as it is
+            if (t * t > 0x1p-53) cs = rsqrt64(1.0 + t * t);
+            f = (t * cs * ri) * cconj(z);
           }
         }
         rc[tid] = cs;
-        rs[tid] = sn;
-        re[tid] = e;
+        rs[tid] = f;
       }
       __syncthreads();
       // A <- J^H A J on the 2 x 2 blocks of pairs, V <- V J: an item's slots
@@ -1312,24 +1318,23 @@ __global__ __launch_bounds__(1024) void k_ritz(int m, int basis, const int* pmap
       for (int u = 0; u < 2; u++) {
         if (itK[u] < 0) continue;
         const int K = itK[u], s = first(K), t = second(K);
-        const double cK = rc[K], sK = rs[K];
-        const C<double> eK = re[K], z0 = czero<double>();
+        const double cK = rc[K];
+        const C<double> fK = rs[K], gK = cconj(fK), z0 = czero<double>();
         const bool ok_s = s < kk;
         if (itP[u] >= 0) {
           const int P = itP[u], p = first(P), q = second(P);
           const bool ok_p = p < kk;
           C<double> a = ok_p && ok_s ? A[p + s * kk] : z0, b = ok_p ? A[p + t * kk] : z0;
           C<double> c = ok_s ? A[q + s * kk] : z0, d = A[q + t * kk];
-          // columns: s' = cs s - sn e t, t' = sn s + cs e t
-          const double cP = rc[P], sP = rs[P];
-          const C<double> eP = cconj(re[P]), eb = eK * b, ed = eK * d;
-          const C<double> a1 = cK * a - sK * eb, b1 = sK * a + cK * eb, c1 = cK * c - sK * ed, d1 = sK * c + cK * ed;
-          // rows: p' = cs p - sn conj(e) q, q' = sn p + cs conj(e) q
-          const C<double> ec = eP * c1, ef = eP * d1;
-          a = cP * a1 - sP * ec;
-          c = sP * a1 + cP * ec;
-          b = cP * b1 - sP * ef;
-          d = sP * b1 + cP * ef;
+          // columns: s' = c s - f t, t' = conj(f) s + c t
+          const double cP = rc[P];
+          const C<double> fP = rs[P], gP = cconj(fP);
+          const C<double> a1 = cK * a - fK * b, b1 = gK * a + cK * b, c1 = cK * c - fK * d, d1 = gK * c + cK * d;
+          // rows: p' = c p - conj(f) q, q' = f p + c q
+          a = cP * a1 - gP * c1;
+          c = fP * a1 + cP * c1;
+          b = cP * b1 - gP * d1;
+          d = fP * b1 + cP * d1;
           if (P == K) {
             a.i = d.i = 0.0;
             b = c = z0;
@@ -1340,9 +1345,9 @@ __global__ __launch_bounds__(1024) void k_ritz(int m, int basis, const int* pmap
           A[q + t * kk] = d;
         } else if (ok_s) {
           const int i = -1 - itP[u];
-          const C<double> a = Vv[i + s * kk], b = eK * Vv[i + t * kk];
-          Vv[i + s * kk] = cK * a - sK * b;
-          Vv[i + t * kk] = sK * a + cK * b;
+          const C<double> a = Vv[i + s * kk], b = Vv[i + t * kk];
+          Vv[i + s * kk] = cK * a - fK * b;
+          Vv[i + t * kk] = gK * a + cK * b;
         }
       }
       __syncthreads();
