@@ -382,6 +382,9 @@ int mxh_random(int prec, long long n, int nv, mxh_vecs x, unsigned long long see
                int first_vector);
 
 /* ---- adjoint ---- */
+/* grad[c] += w_v * |curl e_v|_c^2 / (hx hy) summed over the nv vectors. */
+int mxh_curl2(const mxh_level *lv, const mxh_bloch *bl, int nv, mxh_vecs e,
+              const double *w, double *grad);
 /* out[c] = sum_v |curl e_v|_c^2 / (hx hy) / (e_v^H M e_v) (FP64), the M-norms
    from the vectors' Gram sums (mxh_gram); out: device or pinned memory. */
 int mxh_eta_grad(const mxh_level *lv, const mxh_bloch *bl, int nv, mxh_vecs e, const double *gram, double *out);

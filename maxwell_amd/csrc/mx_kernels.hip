@@ -2887,10 +2887,12 @@ __global__ __launch_bounds__(256) void k_random(long long n, C<T>* X, long long 
 }
 
 // ----------------------------------------------------------------- adjoint
-// sum_v |curl e_v|_c^2 / (hx hy) / (e_v^H M e_v) per cell, with the M-norms taken
-// from the Gram sums of the vectors (pair (v, v)).  out may be host memory.
+// sum_v w_v |curl e_v|_c^2 / (hx hy) per cell: ADD, with the weights w, added to
+// out; else with w_v = 1 / (e_v^H M e_v) from the vectors' Gram sums w (pair
+// (v, v)), written to out, which may be host memory.
+template <bool ADD>
 __global__ __launch_bounds__(256) void k_eta_grad(mxh_level lv, mxh_bloch bl, int nv, const C<double>* E,
-                                                 long long es, const double* gram, double* out)
+                                                 long long es, const double* w, double* out)
 {
   const size_t N = (size_t)lv.nx * lv.ny;
   size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2902,9 +2904,9 @@ __global__ __launch_bounds__(256) void k_eta_grad(mxh_level lv, mxh_bloch bl, in
     Geo<double> g = make_geo<double>(lv, bl, v);
     EdgeV<double> e = edge_view<double>(E, es, v, N);
     C<double> c = cell_curl(g, e, i, j);
-    acc += (1.0 / gram[4 * (v * (v + 1) / 2 + v) + 2]) * (c.r * c.r + c.i * c.i) * s;
+    acc += (ADD ? w[v] : 1.0 / w[4 * (v * (v + 1) / 2 + v) + 2]) * (c.r * c.r + c.i * c.i) * s;
   }
-  out[idx] = acc;
+  out[idx] = ADD ? out[idx] + acc : acc;
 }
 
 // ----------------------------------------------------------------- tile-fused AFW sweeps
@@ -6321,11 +6323,18 @@ int mxh_random(int prec, long long n, int nv, mxh_vecs x, unsigned long long see
   return 0;
 }
 
+int mxh_curl2(const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs e, const double* w, double* grad)
+{
+  hipLaunchKernelGGL(k_eta_grad<true>, dim3(nblocks((long long)lv->nx * lv->ny)), dim3(TPB), 0, g_stream, *lv, *bl, nv,
+                     (const C<double>*)e.p, e.stride, w, grad);
+  LAUNCH_CHECK();
+  return 0;
+}
+
 int mxh_eta_grad(const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs e, const double* gram, double* out)
 {
-  const long long N = (long long)lv->nx * lv->ny;
-  hipLaunchKernelGGL(k_eta_grad, dim3(nblocks(N)), dim3(TPB), 0, g_stream, *lv, *bl, nv, (const C<double>*)e.p,
-                     e.stride, gram, out);
+  hipLaunchKernelGGL(k_eta_grad<false>, dim3(nblocks((long long)lv->nx * lv->ny)), dim3(TPB), 0, g_stream, *lv, *bl, nv,
+                     (const C<double>*)e.p, e.stride, gram, out);
   LAUNCH_CHECK();
   return 0;
 }
