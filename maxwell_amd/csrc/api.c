@@ -131,7 +131,7 @@ typedef struct {
   double *out;   /* small device result buffer */
   field *tmp;    /* scratch edge vector */
   size_t ntmp;
-  field *sweep;  /* the smoothers' second buffer (one edge vector), under sweep_lock */
+  field *sweep;  /* the smoothers' second buffer (one edge vector), under cycle_lock */
 } griddev;
 
 static griddev *gdev(const grid2d *gr)
@@ -786,7 +786,15 @@ void restriction_edge2d(field alpha, const edge2d *f, edge2d *c)
   }
 }
 
-/* ---- coarse factor cache: the host factor is uploaded when it changes */
+/* A cycle's device state that vectors share: a grid's second buffer, the coarse
+   factors and their inverses.  Held from where a pointer into it is taken until
+   the last launch that reads it is queued (the library's stream then runs them
+   in order), so that a call from another host thread, with another coarse
+   matrix, changes it before or after. */
+static pthread_mutex_t cycle_lock = PTHREAD_MUTEX_INITIALIZER;
+
+/* ---- coarse factor cache (under cycle_lock): the host factor is uploaded when
+   it changes */
 typedef struct {
   const matrix *key;
   uint64_t sum;
@@ -861,10 +869,6 @@ typedef struct {
   mxh_cycle cy;
   const double *W;
 } cycle_plan;
-
-/* the second buffers are shared by every vector of a grid: held over the
-   launches of a cycle (the library's stream then runs them in order) */
-static pthread_mutex_t sweep_lock = PTHREAD_MUTEX_INITIALIZER;
 
 static field *sweep_buffer(const grid2d *gr)
 {
@@ -957,7 +961,6 @@ static void vcycle_edge_impl(int L, int nu, const matrix *Ac, edge2d **b, edge2d
 {
   if (xzero && !p->fused) HIPCK(mxh_memset(x[L]->x, 0, sizeof(field) * en(x[L])));
   const int lc = p->lc > 0 ? p->lc : 0;
-  if (p->fused) pthread_mutex_lock(&sweep_lock);
   for (int l = L; l > lc; l--) {
     if (p->fused) {
       edge_passes(nu, 0, xzero && l == L, b[l], x[l], b[l - 1], x[l - 1]);
@@ -989,7 +992,6 @@ static void vcycle_edge_impl(int L, int nu, const matrix *Ac, edge2d **b, edge2d
     prolong_edge_impl(1.0, x[l - 1], x[l]);
     for (int i = 0; i < nu; i++) gs_edge(1.0, 1.0, b[l], x[l], 1);
   }
-  if (p->fused) pthread_mutex_unlock(&sweep_lock);
 }
 
 void vcycle_edge2d(int L, int nu, const matrix *Ac, edge2d **b, edge2d **x, edge2d **d)
@@ -998,8 +1000,10 @@ void vcycle_edge2d(int L, int nu, const matrix *Ac, edge2d **b, edge2d **x, edge
 #pragma omp single
   {
     cycle_plan p;
+    pthread_mutex_lock(&cycle_lock);
     plan_edge(&p, L, nu, Ac, b, x);
     vcycle_edge_impl(L, nu, Ac, b, x, &p, 0);
+    pthread_mutex_unlock(&cycle_lock);
   }
 }
 
@@ -1067,7 +1071,11 @@ void hcycle_edge2d(int L, int nu, const matrix *Ac, edge2d **b, edge2d **x, edge
   }
   if (Ac) {
 #pragma omp single
-    edge_coarse_solve(Ac, b[0], x[0]);
+    {
+      pthread_mutex_lock(&cycle_lock);
+      edge_coarse_solve(Ac, b[0], x[0]);
+      pthread_mutex_unlock(&cycle_lock);
+    }
   } else {
     for (int i = 0; i < nu; i++) gssymm_simple_edge2d(1.0, 1.0, b[0], x[0]);
   }
@@ -1468,7 +1476,6 @@ static void node_passes(int nu, int up, const node2d *b, node2d *x, node2d *bc, 
 static void vcycle_node_impl(int L, int nu, const matrix *Ac, node2d **b, node2d **x, const cycle_plan *p)
 {
   const int lc = p->lc > 0 ? p->lc : 0;
-  if (p->fused) pthread_mutex_lock(&sweep_lock);
   for (int l = L; l > lc; l--) {
     if (p->fused) {
       node_passes(nu, 0, b[l], x[l], b[l - 1], x[l - 1]);
@@ -1513,7 +1520,6 @@ static void vcycle_node_impl(int L, int nu, const matrix *Ac, node2d **b, node2d
     HIPCK(mxh_node_prolong(MXH_F64, &lv, &bl, 1, VV(x[l - 1]->v, nn(x[l - 1])), VV(x[l]->v, nn(x[l])), 1.0, 0.0));
     for (int i = 0; i < nu; i++) gs_node(1.0, b[l], x[l], 1);
   }
-  if (p->fused) pthread_mutex_unlock(&sweep_lock);
 }
 
 void vcycle_node2d(int L, int nu, const matrix *Ac, node2d **b, node2d **x, node2d **d)
@@ -1522,8 +1528,10 @@ void vcycle_node2d(int L, int nu, const matrix *Ac, node2d **b, node2d **x, node
 #pragma omp single
   {
     cycle_plan p;
+    pthread_mutex_lock(&cycle_lock);
     plan_node(&p, L, nu, Ac, b, x);
     vcycle_node_impl(L, nu, Ac, b, x, &p);
+    pthread_mutex_unlock(&cycle_lock);
   }
 }
 
@@ -1590,6 +1598,7 @@ void pinvit_edge2d(int l, int smoother_steps, int prec_steps, int gradient_steps
     const long long n = en(e), N = n / 2;
     HIPCK(mxh_addeval(MXH_F64, &lv, &bl, 1, VV(e->x, n), VV(b[l]->x, n), gdev(gr)->eta, &cf, 0));
     cycle_plan pe, pn;
+    pthread_mutex_lock(&cycle_lock);
     plan_edge(&pe, l, smoother_steps, Ae, b, x);
     plan_node(&pn, l, smoother_steps, An, bg, xg);
     if (prec_steps < 1) HIPCK(mxh_memset(x[l]->x, 0, sizeof(field) * n));
@@ -1599,6 +1608,7 @@ void pinvit_edge2d(int l, int smoother_steps, int prec_steps, int gradient_steps
     HIPCK(mxh_lift_rhs(MXH_F64, &lv, &bl, 1, VV(e->x, n), VV(x[l]->x, n), VV(NULL, n), VV(bg[l]->v, N),
                        VV(xg[l]->v, N), NULL, NULL));
     for (int j = 0; j < gradient_steps; j++) vcycle_node_impl(l, smoother_steps, An, bg, xg, &pn);
+    pthread_mutex_unlock(&cycle_lock);
     HIPCK(mxh_lift_apply(MXH_F64, &lv, &bl, 1, VV(xg[l]->v, N), VV(e->x, n), VV(x[l]->x, n), VV(e->x, n), -1.0,
                          NULL, NULL));
   }
