@@ -3880,65 +3880,96 @@ __global__ __launch_bounds__(256, 2) void k_edge_cycle(CycleLevels cl, mxh_bloch
 }
 
 // W[r n + c] = (A^-1)[r, c] from the Cholesky factor L of A (n x n,
-// column-major, per problem): one workgroup per problem, forward and back
-// substitution of the unit vectors.  n <= COARSE_LDS_N: L and W in LDS, a row's
-// multiples leave all other rows at once, one barrier a row (a chain of 2 n
-// barriers).  Larger: one thread per column, W itself holds the running column.
-#define COARSE_LDS_N 64
+// column-major, per problem).  The columns of the inverse are independent: a wave
+// solves for two of them, row lane + 64 q of each in lane `lane`, by forward and
+// back substitution with no barrier.  A step's unknown goes to all lanes by
+// v_readlane and leaves their rows at once; the entries of L it needs depend on
+// nothing, so eight steps' are loaded ahead.  What bounds it is that chain of 2 n
+// steps: 20 us at 32 rows, 34 at 64, 41 at 72, 126 at 200 (64 problems: 530).  One
+// workgroup per problem, with a barrier a row up to 64 rows and a thread per column
+// above, took 31, 106, 644 and 5305 (7340).
+#define INV_COLS 2
+MXH_DEV C<double> lane_value(C<double> v, int lane)
+{
+  union { double d[2]; int i[4]; } u;
+  u.d[0] = v.r;
+  u.d[1] = v.i;
+#pragma unroll
+  for (int q = 0; q < 4; q++) u.i[q] = __builtin_amdgcn_readlane(u.i[q], lane);
+  return cmk(u.d[0], u.d[1]);
+}
+
+template <int R>
 __global__ __launch_bounds__(256) void k_coarse_inverse(int n, const double* L0, double* W0)
 {
-  extern __shared__ double smem[];
+  const int lane = threadIdx.x & 63;
+  const int c0 = __builtin_amdgcn_readfirstlane(((int)blockIdx.y * 4 + (int)(threadIdx.x >> 6)) * INV_COLS);
+  if (c0 >= n) return;
   const C<double>* L = (const C<double>*)L0 + (size_t)blockIdx.x * n * n;
   C<double>* W = (C<double>*)W0 + (size_t)blockIdx.x * n * n;
-  if (n <= COARSE_LDS_N) {
-    C<double>*l = (C<double>*)smem, *w = l + n * n;
-    const int tc = threadIdx.x & 15, tr = threadIdx.x >> 4, nr = blockDim.x >> 4;
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
-      l[e] = L[e];
-      w[e] = cmk(e / n == e % n ? 1.0 : 0.0, 0.0);
-    }
-    for (int k = 0; k < n; k++) {
-      __syncthreads();
-      const double inv = 1.0 / l[k + k * n].r;
-      for (int r = k + 1 + tr; r < n; r += nr) {
-        const C<double> f = inv * l[r + k * n];
-        for (int c = tc; c <= k; c += 16) w[r * n + c] -= f * w[k * n + c];
+  C<double> w[INV_COLS][R];
+  int row[R];  // (lanes past the last row read it and keep zeros)
+#pragma unroll
+  for (int q = 0; q < R; q++) {
+    row[q] = min(lane + 64 * q, n - 1);
+#pragma unroll
+    for (int c = 0; c < INV_COLS; c++) w[c][q] = cmk(lane + 64 * q == c0 + c ? 1.0 : 0.0, 0.0);
+  }
+  // L y = unit vector, from the first unit's row on
+#pragma unroll
+  for (int b = 0; b < R; b++)
+    for (int l0 = max(0, c0 - 64 * b) & ~7; l0 < 64 && 64 * b + l0 < n; l0 += 8) {
+      C<double> a[8][R];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+#pragma unroll
+        for (int q = b; q < R; q++) a[u][q] = L[row[q] + (size_t)min(64 * b + l0 + u, n - 1) * n];
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const int k = 64 * b + l0 + u;
+        if (k >= n) break;  // uniform
+        const double inv = 1.0 / a[u][b].r;
+#pragma unroll
+        for (int c = 0; c < INV_COLS; c++) {
+          const C<double> f = lane_value(inv * w[c][b], l0 + u);
+          if (lane == l0 + u) w[c][b] = f;
+#pragma unroll
+          for (int q = b; q < R; q++)
+            if (lane + 64 * q > k && lane + 64 * q < n) w[c][q] -= a[u][q] * f;
+        }
       }
     }
-    __syncthreads();
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
-      const int r = e / n;
-      w[e] = (1.0 / l[r + r * n].r) * w[e];
-    }
-    for (int k = n - 1; k >= 0; k--) {
-      __syncthreads();
-      const double inv = 1.0 / l[k + k * n].r;
-      for (int r = tr; r < k; r += nr) {
-        const C<double> f = inv * cconj(l[k + r * n]);
-        for (int c = tc; c < n; c += 16) w[r * n + c] -= f * w[k * n + c];
+  // L^H x = y, from the last row up
+#pragma unroll
+  for (int b = R - 1; b >= 0; b--)
+    for (int l0 = min(63, n - 1 - 64 * b) & ~7; l0 >= 0; l0 -= 8) {
+      C<double> a[8][R];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+#pragma unroll
+        for (int q = 0; q <= b; q++) a[u][q] = cconj(L[min(64 * b + l0 + u, n - 1) + (size_t)row[q] * n]);
+#pragma unroll
+      for (int u = 7; u >= 0; u--) {
+        const int k = 64 * b + l0 + u;
+        if (k >= n) continue;  // uniform
+        const double inv = 1.0 / a[u][b].r;
+#pragma unroll
+        for (int c = 0; c < INV_COLS; c++) {
+          const C<double> f = lane_value(inv * w[c][b], l0 + u);
+          if (lane == l0 + u) w[c][b] = f;
+#pragma unroll
+          for (int q = 0; q <= b; q++)
+            if (lane + 64 * q < k) w[c][q] -= a[u][q] * f;
+        }
       }
     }
-    __syncthreads();
-    for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
-      const int r = e / n;
-      W[e] = (1.0 / l[r + r * n].r) * w[e];
-    }
-    return;
-  }
-  const int c = threadIdx.x;
-  if (c >= n) return;
-  for (int r = 0; r < n; r++) {
-    C<double> t = cmk(r == c ? 1.0 : 0.0, 0.0);
-    for (int k = c; k < r; k++) t -= L[r + (size_t)k * n] * W[(size_t)k * n + c];
-    const double d = L[r + (size_t)r * n].r;
-    W[(size_t)r * n + c] = cmk(t.r / d, t.i / d);
-  }
-  for (int r = n - 1; r >= 0; r--) {
-    C<double> t = W[(size_t)r * n + c];
-    for (int k = r + 1; k < n; k++) t -= cconj(L[k + (size_t)r * n]) * W[(size_t)k * n + c];
-    const double d = L[r + (size_t)r * n].r;
-    W[(size_t)r * n + c] = cmk(t.r / d, t.i / d);
-  }
+  // Hermitian: column c as row c
+#pragma unroll
+  for (int c = 0; c < INV_COLS; c++)
+    if (c0 + c < n)
+#pragma unroll
+      for (int q = 0; q < R; q++)
+        if (lane + 64 * q < n) W[(size_t)(c0 + c) * n + lane + 64 * q] = cconj(w[c][q]);
 }
 
 // ---- the nodal counterpart: Gauss-Seidel for the Q1 Laplacian
@@ -4975,7 +5006,7 @@ int mxh_init(void)
                        (const void*)k_fft_rows<float, -1>, (const void*)k_fft_rows<float, 1>,
                        (const void*)k_edge_cycle<double>, (const void*)k_edge_cycle<float>,
                        (const void*)k_node_cycle<double>, (const void*)k_node_cycle<float>,
-                       (const void*)k_coarse_inverse, (const void*)k_hh_coef};
+                       (const void*)k_hh_coef};
   for (const void* f : big) {
     e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     if (e != hipSuccess) return (int)e;
@@ -5318,9 +5349,11 @@ int mxh_cycle_supported(int prec, const mxh_cycle* cy)
 int mxh_coarse_inverse(int n, int nprob, const double* L, double* W)
 {
   if (n < 1 || n > 256 || nprob < 1) return (int)hipErrorInvalidValue;
-  const bool lds = n <= COARSE_LDS_N;
-  hipLaunchKernelGGL(k_coarse_inverse, dim3(nprob), dim3(lds ? 256 : (n + 63) / 64 * 64),
-                     lds ? 2 * sizeof(C<double>) * n * n : 0, g_stream, n, L, W);
+  const dim3 grid(nprob, (n + 4 * INV_COLS - 1) / (4 * INV_COLS));
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, g_stream, n, L, W); };
+  if (n <= 64) go(k_coarse_inverse<1>);
+  else if (n <= 128) go(k_coarse_inverse<2>);
+  else go(k_coarse_inverse<4>);
   LAUNCH_CHECK();
   return 0;
 }
