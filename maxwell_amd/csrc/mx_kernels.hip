@@ -5701,14 +5701,17 @@ static int gram_launch(const mxh_level* lv, const mxh_bloch* bl, int nprob, cons
   // by the registers of the tiles' sums) and a band costs its rows and about
   // one row for its start, so the height minimises rounds x (rows + 1).  36
   // columns, 16 problems of 512^2: 4, 8, 16, 32 rows measured 2.00, 1.79, 1.69,
-  // 1.66 ms, 64 rows (half the units idle) 3.19.
+  // 1.66 ms, 64 rows (half the units idle) 3.19.  Heights from the least that the
+  // buffer takes to twice that, or 64: with 64 as the limit always, tall grids and
+  // many problems had one band a problem (256 x 4096, 33 problems of 12 columns:
+  // 24.3 ms against 3.0).
   const int sets = nprob > sets_cap ? nprob : sets_cap;
   const long long slots = (long long)mxh_cu_count() * (nt == 1 ? 4 : nt == 2 ? 2 : 1);
-  int rpb = lv->ny;
+  const int most = sets / nprob, least = (lv->ny + most - 1) / most;
+  int rpb = least;
   long long cost = -1;
-  for (int r = 1; r <= 64 && r <= lv->ny; r++) {
+  for (int r = least; r <= (least > 32 ? 2 * least : 64) && r <= lv->ny; r++) {
     const long long wgs = (long long)((lv->ny + r - 1) / r) * nprob;
-    if (wgs > sets) continue;
     const long long c = (wgs + slots - 1) / slots * (r + 1);
     if (cost < 0 || c <= cost) {
       cost = c;
