@@ -108,13 +108,17 @@ int mxh_edge_gs_phase(int prec, const mxh_level *lv, const mxh_bloch *bl, int nv
                       int colour);
 
 /* Tile-fused AFW sweeps (grids of at most 64 x 64: the whole grid in LDS)
-   with operator K + M (alpha = beta = 1), reading x and writing the result to xo (a different buffer: workgroups read halo
-   nodes that other workgroups own).  mode bits:
-   1 backward colour order (then nsweep must be 1), 2 x starts at zero,
+   with operator K + M (alpha = beta = 1), reading x and writing the result to
+   xo (a different buffer: workgroups read halo nodes that other workgroups
+   own).  Up to two sweeps per launch.  mode bits:
+   1 backward colour order, 2 x starts at zero,
    4 add P xc_in to x first (coarse correction of the V-cycle),
-   8 after one forward sweep write bc = R (b - (K + M) x) and xc = 0 on the
-   coarse level (vectors of the coarse level, stride bc.stride).
-   Forward sweeps without mode 8 may be fused (nsweep > 1). */
+   8 after the (forward) sweeps write bc = R (b - (K + M) x) and xc = 0 on the
+   coarse level (vectors of the coarse level, stride bc.stride),
+   16 every copy of a node that a workgroup holds has its owner's value to the
+   last bit, also across the periodic boundary (otherwise where that is the
+   faster form): the residual of a vector then holds no gradient fields from
+   copies that were rounded apart. */
 int mxh_afw_tile(int prec, const mxh_level *lv, const mxh_bloch *bl, int nv,
                  mxh_vecs b, mxh_vecs x, mxh_vecs xo, const void *eta, int nsweep,
                  int mode, mxh_vecs xc_in, mxh_vecs bc, mxh_vecs xc);

@@ -951,8 +951,9 @@ static void edge_passes(int nu, int up, int xzero, const edge2d *b, edge2d *x, e
   for (int i = 0; i < passes; i++, cur ^= 1) {
     const int first = i == 0, last = i == passes - 1, sweeps = last ? nu - 2 * i : 2;
     const int mode = up ? 1 + (first ? 4 : 0) : (first && xzero ? 2 : 0) + (last ? 8 : 0);
+    /* 16: a FP64 step is 3e-12 from 64 bits, with copies rounded apart 6e-11 */
     HIPCK(mxh_afw_tile(MXH_F64, &lv, &bl, 1, VV(b->x, n), VV(buf[cur], n), VV(buf[cur ^ 1], n), gdev(x->gr)->eta,
-                       sweeps, mode, mode & 4 ? VV(xc->x, nc) : none, mode & 8 ? VV(bc->x, nc) : none,
+                       sweeps, mode | 16, mode & 4 ? VV(xc->x, nc) : none, mode & 8 ? VV(bc->x, nc) : none,
                        mode & 8 ? VV(xc->x, nc) : none));
   }
 }

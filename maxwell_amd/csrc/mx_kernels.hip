@@ -5230,14 +5230,14 @@ static bool afw_grid_fits(int prec, const mxh_level* lv)
 // residual, FP64 edges / nodes, against the large tiles: 128^2 one vector 10 / 6
 // against 17 / 10, four 16 / 8 against 19 / 11; 256^2 one 15 / 8 against 19 / 10,
 // two 23 / 11 both; FP32 128^2 four 10 against 16), beyond they repeat
-// the halo's work.  One vector takes them at any size for their rounding (512^2
-// 45 us both).  Edge grids of up to 32 x 32 nodes stay whole in LDS (32
-// vectors: 10 us against 14).
+// the halo's work (384^2 one 30 / 13 against 25 / 12); callers that need k_afw_few's
+// rounding ask for it (mode 16).  Edge grids of up to 32 x 32 nodes stay whole in
+// LDS (32 vectors: 10 us against 14).
 #define FEW_MAX 512
 static bool few_fits(const mxh_level* lv, int nv)
 {
   const long long t = (long long)((lv->nx + FEW_T - 1) / FEW_T) * ((lv->ny + FEW_T - 1) / FEW_T);
-  return nv == 1 || t * nv <= FEW_MAX;
+  return t * nv <= FEW_MAX;
 }
 
 template <typename T, int MODE>
@@ -5403,18 +5403,24 @@ int mxh_afw_tile(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh
 {
   if (!xo.p || xo.p == x.p || xo.stride != x.stride) return (int)hipErrorInvalidValue;
   if ((lv->nx & 1) || (lv->ny & 1) || nsweep < 1) return (int)hipErrorInvalidValue;
+  const bool exact = mode & 16;
+  mode &= ~16;
   if ((mode & 8) && (mode & 1)) return (int)hipErrorInvalidValue;
   // the halo must cover the sweeps (and the residual with its restriction)
   if (nsweep * ((mode & 1) ? TILE_SHRINK_BWD : TILE_SHRINK_FWD) + ((mode & 8) ? TILE_SHRINK_RES : 0) > TILE_H)
     return (int)hipErrorInvalidValue;
   if ((mode & 4) && !xc_in.p) return (int)hipErrorInvalidValue;
   if ((mode & 8) && (!bc.p || !xc.p || bc.stride != xc.stride)) return (int)hipErrorInvalidValue;
-  const bool few = few_fits(lv, nv) && (long long)lv->nx * lv->ny > 1024;
-  if (few || afw_grid_fits(prec, lv))
-    return prec == MXH_F64 ? launch_grid_mode<double>(few, mode, lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc)
-                           : launch_grid_mode<float>(few, mode, lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc);
   const int R = prec == MXH_F64 ? TileCfg<double>::R : TileCfg<float>::R, TT = R - 2 * TILE_H;
   const int ntx = (lv->nx + TT - 1) / TT, nty = (lv->ny + TT - 1) / TT;
+  const long long N = (long long)lv->nx * lv->ny;
+  // small tiles, else the whole grid, else square tiles
+  bool few = N > 1024 && few_fits(lv, nv);
+  const bool whole = !few && afw_grid_fits(prec, lv);
+  few |= exact && !whole;
+  if (few || whole)
+    return prec == MXH_F64 ? launch_grid_mode<double>(few, mode, lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc)
+                           : launch_grid_mode<float>(few, mode, lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc);
   dim3 grid(ntx * nty, nv), block((R / 2) * (R / 2));
   long long cs = (mode & 8) ? bc.stride : (mode & 4) ? xc_in.stride : 0;
   int e = prec == MXH_F64
