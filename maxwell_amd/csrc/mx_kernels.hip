@@ -5414,9 +5414,13 @@ int mxh_afw_tile(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh
   const int R = prec == MXH_F64 ? TileCfg<double>::R : TileCfg<float>::R, TT = R - 2 * TILE_H;
   const int ntx = (lv->nx + TT - 1) / TT, nty = (lv->ny + TT - 1) / TT;
   const long long N = (long long)lv->nx * lv->ny;
-  // small tiles, else the whole grid, else square tiles
+  // small tiles, else the whole grid, else square tiles.  A whole FP64 grid near
+  // 64 x 64 takes 28 us (two sweeps and residual) however few its vectors; while
+  // the square tiles fill at most one workgroup per compute unit they are done
+  // before (16 vectors 21 us, 24: 25; 32: 40).  Grids of 48 x 48 take 21 either way.
   bool few = N > 1024 && few_fits(lv, nv);
-  const bool whole = !few && afw_grid_fits(prec, lv);
+  const bool tiles = prec == MXH_F64 && N > 3072 && (long long)ntx * nty * nv <= mxh_cu_count();
+  const bool whole = !few && afw_grid_fits(prec, lv) && (exact || !tiles);
   few |= exact && !whole;
   if (few || whole)
     return prec == MXH_F64 ? launch_grid_mode<double>(few, mode, lv, bl, nv, b, x, xo, eta, nsweep, xc_in, bc, xc)

@@ -16,6 +16,13 @@ from test_gpu_few_vectors import lib  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 
+# 64 x 64 in FP64: 252 and 261 square tiles; 56 x 54 and 56 x 56: 3024 and 3136 nodes
+@pytest.mark.parametrize("nx,ny,nv", [(64, 64, 28), (64, 64, 29), (56, 54, 26), (56, 56, 26)])
+@pytest.mark.parametrize("mode,nsweep", [(1, 2), (5, 2), (8, 2), (10, 1)])
+def test_whole_grids_and_square_tiles(lib, nx, ny, nv, mode, nsweep):  # noqa: F811
+    F.test_small_launches(lib, 0, nx, ny, nv, False, mode, nsweep)
+
+
 @pytest.mark.parametrize("prec", [0, 1])
 @pytest.mark.parametrize("nx,ny,nv", [(12, 40, 3), (64, 64, 20), (62, 68, 20), (150, 162, 4), (290, 288, 1)])
 @pytest.mark.parametrize("mode,nsweep", [(0, 1), (5, 2), (8, 2), (10, 1)])
@@ -50,6 +57,10 @@ def best_time(lib, nx, ny, nv, mode):  # noqa: F811
         best = min(best, (time.perf_counter() - t) / 20)
     print("%d x %d, %d vectors, mode %d: %.1f us" % (nx, ny, nv, mode, 1e6 * best))
     return best
+
+
+def test_time_of_few_vectors_on_the_largest_whole_grid(lib):  # noqa: F811
+    assert best_time(lib, 64, 64, 16, 8) <= 1.15 * best_time(lib, 62, 68, 16, 8)
 
 
 def test_time_of_one_vector_on_a_large_grid(lib):  # noqa: F811
