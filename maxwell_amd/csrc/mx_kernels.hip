@@ -187,6 +187,17 @@ MXH_DEV void coefs(const mxh_level& lv, const mxh_coef& cf, int v, C<T>& axy, C<
   my = cmk(T(br * sy), T(bi * sy));
 }
 
+// the value of one lane (uniform), in all lanes
+MXH_DEV C<double> lane_value(C<double> v, int lane)
+{
+  union { double d[2]; int i[4]; } u;
+  u.d[0] = v.r;
+  u.d[1] = v.i;
+#pragma unroll
+  for (int q = 0; q < 4; q++) u.i[q] = __builtin_amdgcn_readlane(u.i[q], lane);
+  return cmk(u.d[0], u.d[1]);
+}
+
 // ----------------------------------------------------------------- reductions
 MXH_DEV double wave_sum(double v)
 {
@@ -1568,7 +1579,7 @@ MXH_DEV C<double> unit_mprod(const C<double>* y, int i, int j, int nx, int ny, d
 // - sum_j v_j c_j where c_j = conj(tau_j) (w_j - sum_{l > j} S_jl c_l), l <= i.
 //
 // Bound by the chain of 2 k launches on the drivers' grids: 24 vectors of 128^2
-// 1.28 -> 0.45 ms against one launch per product, update and fix of both passes.
+// 1.28 -> 0.42 ms against one launch per product, update and fix of both passes.
 #define HH_NB 64  // partial sums per vector at most (one wave's lanes)
 struct HhVecs {
   C<double>* base;  // vector j at base + j stride, or, with a table, table[j]
@@ -1646,12 +1657,13 @@ MXH_DEV C<double> hh_sum(const HhWork& wk, int j, int nb)
   return cmk(wave_sum(l < nb ? q[0] : 0.0), wave_sum(l < nb ? q[1] : 0.0));
 }
 
-// grid (blocks, k - idx): vector idx + blockIdx.y; nb: blocks of k_hh_row
+// grid (blocks, k - idx): vector idx + blockIdx.y; nb: blocks of k_hh_row.  The
+// workgroups of vector idx share the products with the finished vectors, a wave's
+// sum each (64^2, 300 vectors: 40 us a launch where one workgroup formed them all).
 __global__ __launch_bounds__(256) void k_hh_update(mxh_level lv, int idx, int k, int nb, HhVecs X, HhWork wk)
 {
   const int nx = lv.nx, tid = threadIdx.x, j = idx + blockIdx.y;
   const size_t E = 2 * (size_t)nx * lv.ny;
-  if (j == idx && blockIdx.x) return;
   const double sc = sqrt(0.25 / (lv.hy / lv.hx / 6.0));
   const C<double> beta = cmk(wk.p[2 * idx], wk.p[2 * idx + 1]);
   double alpha = sqrt(hh_sum(wk, idx, nb).r);
@@ -1665,14 +1677,14 @@ __global__ __launch_bounds__(256) void k_hh_update(mxh_level lv, int idx, int k,
   const C<double> uv = cmk(beta.r + alpha, beta.i);  // unit^H M v
   C<double>*S = (C<double>*)wk.S, *W = (C<double>*)wk.W;
   if (j == idx) {
-    for (int l = tid >> 6; l < idx; l += 4) {
+    for (int l = 4 * (int)blockIdx.x + (tid >> 6); l < idx; l += 4 * (int)gridDim.x) {
       const C<double> d = hh_sum(wk, l, nb), p = cmk(wk.p[2 * l], -wk.p[2 * l + 1]);
       if ((tid & 63) == 0) {
         S[(size_t)l * k + idx] = cconj(d) + alpha * p;
         W[(size_t)l * k + idx] = p;
       }
     }
-    if (tid == 0) {
+    if (tid == 0 && blockIdx.x == 0) {
       W[(size_t)idx * k + idx] = cconj(uv);
       wk.hh[4 * idx] = alpha;
       wk.hh[4 * idx + 1] = tau.r;
@@ -1697,15 +1709,20 @@ __global__ __launch_bounds__(256) void k_hh_update(mxh_level lv, int idx, int k,
   }
 }
 
-// the coefficients c (in W) by back substitution, one workgroup, and what the
-// last k_hh_row would have finished: v_{k - 1}; tau to both outputs
+// the coefficients c (in W) by back substitution and what the last k_hh_row would
+// have finished: v_{k - 1}; tau to both outputs.  Up to HH_LDS vectors one workgroup
+// in LDS; more: HH_COLS columns, which do not depend on each other, to a workgroup
+// (300 vectors: 2.2 ms in one workgroup)
+#define HH_LDS 48
+#define HH_COLS 16
 __global__ __launch_bounds__(1024) void k_hh_coef(mxh_level lv, int k, HhVecs X, HhWork wk, double* tau, double* host)
 {
   extern __shared__ double smem[];
   const int tid = threadIdx.x, bd = blockDim.x;
   C<double>*S = (C<double>*)wk.S, *W = (C<double>*)wk.W;
   C<double>*s = S, *w = W;
-  if (k <= 48) {  // in LDS (73 KB)
+  const int ia = k <= HH_LDS ? 0 : (int)blockIdx.x * HH_COLS, ib = k <= HH_LDS ? k : min(k, ia + HH_COLS);
+  if (k <= HH_LDS) {  // 73 KB
     s = (C<double>*)smem;
     w = s + k * k;
     for (int e = tid; e < k * k; e += bd) {
@@ -1713,19 +1730,21 @@ __global__ __launch_bounds__(1024) void k_hh_coef(mxh_level lv, int k, HhVecs X,
       w[e] = W[e];
     }
   }
-  for (int j = k - 1; j >= 0; j--) {
+  for (int j = ib - 1; j >= 0; j--) {
     __syncthreads();
     const C<double> t = cmk(wk.hh[4 * j + 1], -wk.hh[4 * j + 2]);
-    for (int e = tid; e < j * (k - j); e += bd) {
-      const int r = e / (k - j), i = j + e - r * (k - j);
+    const int first = max(ia, j), cols = ib - first;
+    for (int e = tid; e < j * cols; e += bd) {
+      const int r = e / cols, i = first + e - r * cols;
       w[(size_t)r * k + i] -= s[(size_t)r * k + j] * (t * w[(size_t)j * k + i]);
     }
   }
   __syncthreads();
-  for (int e = tid; e < k * k; e += bd) {
-    const int j = e / k, i = e - j * k;
-    if (i >= j) W[e] = cmk(wk.hh[4 * j + 1], -wk.hh[4 * j + 2]) * w[e];
+  for (int e = tid; e < ib * (ib - ia); e += bd) {
+    const int j = e / (ib - ia), i = ia + e - j * (ib - ia);
+    if (i >= j) W[(size_t)j * k + i] = cmk(wk.hh[4 * j + 1], -wk.hh[4 * j + 2]) * w[(size_t)j * k + i];
   }
+  if (blockIdx.x) return;
   for (int j = tid; j < k; j += bd) {
     const double r = wk.hh[4 * j + 1], i = wk.hh[4 * j + 2];
     if (tau) {
@@ -1745,36 +1764,51 @@ __global__ __launch_bounds__(1024) void k_hh_coef(mxh_level lv, int k, HhVecs X,
 }
 
 // V_i = unit_i - sum_{j <= i} v_j c_ji, eight outputs at a time from the last
-// ones down: V may be X
+// ones down: V may be X.  Eight vectors' entries and the 8 x 8 coefficients (one
+// a lane, handed round by v_readlane) are loaded while the eight before are used;
+// with a scalar load per coefficient and no load ahead the step took 5 us (300
+// vectors of 64^2 3.5 ms, 24 of 128^2 33 us).
 __global__ __launch_bounds__(64) void k_hh_out(mxh_level lv, int k, HhVecs X, HhVecs V,
                                                const C<double>* __restrict__ cf)
 {
-  const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x, N = (size_t)lv.nx * lv.ny;
-  if (e >= 2 * N) return;
+  const size_t N = (size_t)lv.nx * lv.ny, at = (size_t)blockIdx.x * 64 + threadIdx.x, e = at < 2 * N ? at : 0;
+  const int lj = threadIdx.x >> 3, lq = threadIdx.x & 7;
   // the unit vector whose entry e is
   const unsigned row = (unsigned)(e < N ? e : 0) / (unsigned)lv.nx;
   const long long unit = e < N && (row & 1) ? (long long)(row >> 1) * lv.nx + (long long)(e - (size_t)row * lv.nx) : -1;
   const double sc = sqrt(0.25 / (lv.hy / lv.hx / 6.0));
   for (int i0 = (k - 1) & ~7; i0 >= 0; i0 -= 8) {
     const int m = min(8, k - i0);
-    C<double> acc[8];
-#pragma unroll
-    for (int q = 0; q < 8; q++) acc[q] = cmk(unit == i0 + q ? sc : 0.0, 0.0);
-    for (int j0 = 0; j0 <= i0; j0 += 8) {
-      C<double> v[8];
+    C<double> acc[8], v[8], c;
+    auto load = [&](int j0) {
 #pragma unroll
       for (int j = 0; j < 8; j++) v[j] = X.at(min(j0 + j, k - 1))[e];
+      c = cf[(size_t)min(j0 + lj, k - 1) * k + min(i0 + lq, k - 1)];
+    };
+    // (vectors past the last one only reach outputs that are not written)
+    auto step = [&](const C<double>* u, C<double> d, bool diag) {
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const C<double>* c = cf + (size_t)min(j0 + j, k - 1) * k;
+      for (int j = 0; j < 8; j++)
 #pragma unroll
-        for (int q = 0; q < 8; q++)  // (outputs past the last one are not written)
-          if (j0 < i0 || q >= j) acc[q] -= c[min(i0 + q, k - 1)] * v[j];
-      }
+        for (int q = 0; q < 8; q++)
+          if (!diag || q >= j) acc[q] -= lane_value(d, 8 * j + q) * u[j];
+    };
+#pragma unroll
+    for (int q = 0; q < 8; q++) acc[q] = cmk(unit == i0 + q ? sc : 0.0, 0.0);
+    load(0);
+    for (int j0 = 0; j0 < i0; j0 += 8) {
+      C<double> u[8], d = c;
+#pragma unroll
+      for (int j = 0; j < 8; j++) u[j] = v[j];
+      load(j0 + 8);
+      step(u, d, false);
     }
+    step(v, c, true);
+    if (at < 2 * N) {
 #pragma unroll
-    for (int q = 0; q < 8; q++)
-      if (q < m) V.at(i0 + q)[e] = acc[q];
+      for (int q = 0; q < 8; q++)
+        if (q < m) V.at(i0 + q)[e] = acc[q];
+    }
   }
 }
 
@@ -3889,15 +3923,6 @@ __global__ __launch_bounds__(256, 2) void k_edge_cycle(CycleLevels cl, mxh_bloch
 // workgroup per problem, with a barrier a row up to 64 rows and a thread per column
 // above, took 31, 106, 644 and 5305 (7340).
 #define INV_COLS 2
-MXH_DEV C<double> lane_value(C<double> v, int lane)
-{
-  union { double d[2]; int i[4]; } u;
-  u.d[0] = v.r;
-  u.d[1] = v.i;
-#pragma unroll
-  for (int q = 0; q < 4; q++) u.i[q] = __builtin_amdgcn_readlane(u.i[q], lane);
-  return cmk(u.d[0], u.d[1]);
-}
 
 template <int R>
 __global__ __launch_bounds__(256) void k_coarse_inverse(int n, const double* L0, double* W0)
@@ -5854,14 +5879,15 @@ static int hh_run(const mxh_level* lv, double xr, double xi, double yr, double y
   yf.r = yr;
   yf.i = yi;
   const int nb = N < 256 * HH_NB ? (int)nblocks(N) : HH_NB;
+  const int ub = max(nb, min(HH_NB, (k + 15) / 16));
   for (int i = 0; i < k; i++) {
     hipLaunchKernelGGL(k_hh_row, dim3(nb, k), dim3(256), 0, g_stream, *lv, xf, yf, i, X, wk);
     LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_hh_update, dim3(nb, k - i), dim3(256), 0, g_stream, *lv, i, k, nb, X, wk);
+    hipLaunchKernelGGL(k_hh_update, dim3(ub, k - i), dim3(256), 0, g_stream, *lv, i, k, nb, X, wk);
     LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(k_hh_coef, dim3(1), dim3(1024), k <= 48 ? 2 * sizeof(C<double>) * k * k : 0, g_stream, *lv, k, X,
-                     wk, tau, host);
+  hipLaunchKernelGGL(k_hh_coef, dim3(k <= HH_LDS ? 1 : (k + HH_COLS - 1) / HH_COLS), dim3(1024),
+                     k <= HH_LDS ? 2 * sizeof(C<double>) * k * k : 0, g_stream, *lv, k, X, wk, tau, host);
   LAUNCH_CHECK();
   hipLaunchKernelGGL(k_hh_out, dim3(nblocks(2 * N, 64)), dim3(64), 0, g_stream, *lv, k, X, V, (const C<double>*)wk.W);
   LAUNCH_CHECK();
