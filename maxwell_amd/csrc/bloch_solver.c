@@ -109,8 +109,10 @@ static long long ndim(const mx_solver *s, int l) { return (long long)s->lv[l].nx
    vectors of a problem at one index; vectors a multiple of 64 KB apart then
    meet on the same memory channels, so such strides get 4 KB more (512^2: the
    LOBPCG update of 16 problems 1.80 -> 1.57 ms, the Gram sums of 24 columns
-   0.97 -> 0.82, the block update of 48 problems 2.05 -> 1.95). */
-static long long block_stride(long long n) { return (16 * n) % 65536 == 0 ? n + 256 : n; }
+   0.97 -> 0.82, the block update of 48 problems 2.05 -> 1.95).  Vectors below
+   1 MB stay dense: solves of 64^2 and 128^2 take the same either way, and a copy
+   to the host in rows costs about 5 us a row (12 vectors of 64^2: 108 -> 175 us). */
+static long long block_stride(long long n) { return (16 * n) % 65536 == 0 && 16 * n >= 1 << 20 ? n + 256 : n; }
 
 void mx_solver_destroy(mx_solver *s)
 {
