@@ -372,6 +372,9 @@ int mxh_dot(int prec, long long n, int nv, mxh_vecs x, mxh_vecs y, double *out,
 int mxh_product(long long n, const void *x, const void *y, double *work, double *out, double mark);
 int mxh_product_edge(const mxh_level *lv, const mxh_bloch *bl, const void *x, const void *y, const double *eta,
                      const mxh_coef *cf, double *work, double *out, double mark);
+/* Waits for the mark of a product at out: 1 once it is there (out[0], out[1] are
+   then valid), 0 if not within limit_us microseconds. */
+int mxh_product_wait(const double *out, double mark, double limit_us);
 /* out[v] = |x_v|_2^2 or max |x_v| (kind 0/1) */
 int mxh_norm(int prec, long long n, int nv, mxh_vecs x, int kind, double *out,
              double *work);

@@ -200,16 +200,13 @@ static field *scratch_edge(const grid2d *gr)
 }
 
 /* the product under way: the mark arrives some microseconds before the stream
-   reports the launch as done (a 32^2 product 12 us against 18); a wait of more than
-   a few dozen is left to the stream, which also reports errors */
+   reports the launch as done (a 32^2 product 12 us against 18); a longer wait is
+   left to the stream, which also reports errors */
+#define MARK_WAIT_US 100.0
 static field product_result(call_slot *s)
 {
   s->mark += 1.0;
-  const volatile double *m = s->host + 2;
-  int spins = 0;
-  while (*m != s->mark && ++spins < 20000) __builtin_ia32_pause();
-  if (*m != s->mark) HIPCK(mxh_sync());
-  __atomic_thread_fence(__ATOMIC_ACQUIRE);
+  if (!mxh_product_wait(s->host, s->mark, MARK_WAIT_US)) HIPCK(mxh_sync());
   const field r = s->host[0] + I * s->host[1];
   give_slot(s);
   return r;

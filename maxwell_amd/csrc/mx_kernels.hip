@@ -21,6 +21,7 @@
 
 #include <stdint.h>
 #include <stdio.h>
+#include <time.h>
 
 #include "mxh.h"
 
@@ -6319,6 +6320,24 @@ int mxh_product(long long n, const void* x, const void* y, double* work, double*
   hipLaunchKernelGGL(k_product<0>, dim3(product_blocks(n)), dim3(PRODUCT_TB), 0, g_stream, mxh_level(), mxh_bloch(), n,
                      (const C<double>*)x, (const C<double>*)y, (const double*)nullptr, mxh_coef(), work, out, mark);
   LAUNCH_CHECK();
+  return 0;
+}
+
+int mxh_product_wait(const double* out, double mark, double limit_us)
+{
+  const volatile double* m = out + 2;
+  timespec t0, t;
+  clock_gettime(CLOCK_MONOTONIC, &t0);
+  do {
+    for (int k = 0; k < 32; k++) {
+      if (*m == mark) {
+        __atomic_thread_fence(__ATOMIC_ACQUIRE);
+        return 1;
+      }
+      __builtin_ia32_pause();
+    }
+    clock_gettime(CLOCK_MONOTONIC, &t);
+  } while (1e6 * (double)(t.tv_sec - t0.tv_sec) + 1e-3 * (double)(t.tv_nsec - t0.tv_nsec) < limit_us);
   return 0;
 }
 
