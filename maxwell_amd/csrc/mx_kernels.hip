@@ -6326,16 +6326,23 @@ int mxh_product(long long n, const void* x, const void* y, double* work, double*
 int mxh_product_wait(const double* out, double mark, double limit_us)
 {
   const volatile double* m = out + 2;
-  timespec t0, t;
-  clock_gettime(CLOCK_MONOTONIC, &t0);
-  do {
-    for (int k = 0; k < 32; k++) {
+  auto look = [&](int times) {
+    for (int k = 0; k < times; k++) {
       if (*m == mark) {
         __atomic_thread_fence(__ATOMIC_ACQUIRE);
-        return 1;
+        return true;
       }
       __builtin_ia32_pause();
     }
+    return false;
+  };
+  // most marks come within the first 1024 looks (about 18 us), which the clock
+  // would make 0.8 us longer
+  if (look(1024)) return 1;
+  timespec t0, t;
+  clock_gettime(CLOCK_MONOTONIC, &t0);
+  do {
+    if (look(64)) return 1;
     clock_gettime(CLOCK_MONOTONIC, &t);
   } while (1e6 * (double)(t.tv_sec - t0.tv_sec) + 1e-3 * (double)(t.tv_nsec - t0.tv_nsec) < limit_us);
   return 0;
