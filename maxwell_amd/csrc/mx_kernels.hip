@@ -316,11 +316,11 @@ static inline bool narrow(const mxh_level* lv) { return lv->nx <= 128; }
 // short of workgroups (four per compute unit), BAND_MAX at most (the partial
 // sums' places).
 #define BAND_MAX 128
-#define BAND_SHORT 4
-static inline unsigned band_blocks(const mxh_level* lv, int nv, int rows)
+static inline unsigned band_blocks(const mxh_level* lv, int nv)
 {
   const int groups = narrow(lv) ? 256 / lv->nx : 1;
   auto blocks = [&](int r) { return (lv->ny + groups * r - 1) / (groups * r); };
+  int rows = 4;
   while (rows > 1 && (long long)nv * blocks(rows) < 1024) rows >>= 1;
   const int nb = blocks(rows);
   return (unsigned)(nb < 1 ? 1 : nb < BAND_MAX ? nb : BAND_MAX);
@@ -3307,6 +3307,12 @@ __global__ __launch_bounds__(R* R / 4) void k_node_tile(mxh_level lv, mxh_bloch 
   }
 }
 
+MXH_DEV int wrap_index(int i, int n)
+{
+  i %= n;
+  return i < 0 ? i + n : i;
+}
+
 // ----------------------------------------------------------------- whole grids in LDS
 // Grids of at most 64 x 64 (one thread per 2 x 2 node block) are smoothed with
 // the whole periodic vector in LDS: no halo is loaded or computed (the square
@@ -3316,12 +3322,6 @@ __global__ __launch_bounds__(R* R / 4) void k_node_tile(mxh_level lv, mxh_bloch 
 // across the boundary.  What bounds it: vector issue of the patch solves at 64^2,
 // the latency of the phases on smaller grids.  192 vectors of 64^2 in FP64, two
 // sweeps and prolongation: 58.6 -> 34.9 us (square tiles before).
-MXH_DEV int wrap_index(int i, int n)
-{
-  i %= n;
-  return i < 0 ? i + n : i;
-}
-
 template <typename T>
 struct GridBlock {
   int hx, hy, I, J;       // blocks per side, this thread's block
@@ -5155,24 +5155,15 @@ int mxh_addeval(int prec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_
 int mxh_defect(int rprec, const mxh_level* lv, const mxh_bloch* bl, int nv, mxh_vecs e, mxh_vecs r,
                const double* eta64, const double* lam, double* out, double* work)
 {
-  const unsigned nb = band_blocks(lv, nv, BAND_SHORT);
-  const dim3 grid(nb, nv);
+  const unsigned nb = band_blocks(lv, nv);
+  auto go = [&](auto kernel, auto* to) {
+    hipLaunchKernelGGL(kernel, dim3(nb, nv), dim3(TPB), 0, g_stream, *lv, *bl, (const C<double>*)e.p, e.stride, e.map, to,
+                       r.stride, eta64, lam, work);
+  };
   if (rprec == MXH_F64)
-    {
-      auto go = [&](auto k) {
-        hipLaunchKernelGGL(k, grid, dim3(TPB), 0, g_stream, *lv, *bl, (const C<double>*)e.p, e.stride,
-                           e.map, (C<double>*)r.p, r.stride, eta64, lam, work);
-      };
-      narrow(lv) ? go(k_defect<double, true>) : go(k_defect<double, false>);
-    }
+    narrow(lv) ? go(k_defect<double, true>, (C<double>*)r.p) : go(k_defect<double, false>, (C<double>*)r.p);
   else
-    {
-      auto go = [&](auto k) {
-        hipLaunchKernelGGL(k, grid, dim3(TPB), 0, g_stream, *lv, *bl, (const C<double>*)e.p, e.stride,
-                           e.map, (C<float>*)r.p, r.stride, eta64, lam, work);
-      };
-      narrow(lv) ? go(k_defect<float, true>) : go(k_defect<float, false>);
-    }
+    narrow(lv) ? go(k_defect<float, true>, (C<float>*)r.p) : go(k_defect<float, false>, (C<float>*)r.p);
   LAUNCH_CHECK();
   hipLaunchKernelGGL(k_reduce_partials, dim3(reduce_blocks(2 * nv)), dim3(TPB), 0, g_stream, work, (int)nb, 2 * nv,
                      out, 0);
