@@ -179,6 +179,19 @@ static void *dalloc(mx_solver *s, size_t bytes)
   return p;
 }
 
+/* The node vectors: right-hand side and solution of the finest level for the
+   direct lifting; with `cycles` all levels' and the second solutions, which only
+   node V-cycles use (768 vectors of 512^2 in FP32: 3.2 GB more). */
+static int node_buffers(mx_solver *s, int cycles)
+{
+  for (int l = cycles ? 0 : s->L; l <= s->L; l++) {
+    void **v[3] = {&s->nb[l], &s->nxv[l], &s->nxv2[l]};
+    for (int i = 0; i < (cycles ? 3 : 2); i++)
+      if (!*v[i] && !(*v[i] = dalloc(s, s->csz * (size_t)ndim(s, l) * s->nvmax))) return MX_ENOMEM;
+  }
+  return MX_OK;
+}
+
 int mx_solver_create(const mx_config *cfg, const double *eta, mx_solver **out)
 {
   *out = NULL;
@@ -252,11 +265,8 @@ int mx_solver_create(const mx_config *cfg, const double *eta, mx_solver **out)
     }
     s->eb[l] = dalloc(s, s->csz * (size_t)edim(s, l) * nv);
     s->ex[l] = dalloc(s, s->csz * (size_t)edim(s, l) * nv);
-    s->nb[l] = dalloc(s, s->csz * (size_t)ndim(s, l) * nv);
-    s->nxv[l] = dalloc(s, s->csz * (size_t)ndim(s, l) * nv);
     s->ex2[l] = dalloc(s, s->csz * (size_t)edim(s, l) * nv);
-    s->nxv2[l] = dalloc(s, s->csz * (size_t)ndim(s, l) * nv);
-    if (!s->eb[l] || !s->ex[l] || !s->nb[l] || !s->nxv[l] || !s->ex2[l] || !s->nxv2[l]) goto nomem;
+    if (!s->eb[l] || !s->ex[l] || !s->ex2[l]) goto nomem;
   }
   /* the coarse levels that fit one workgroup's LDS run as one launch */
   s->lc = -1;
@@ -283,6 +293,7 @@ int mx_solver_create(const mx_config *cfg, const double *eta, mx_solver **out)
     if (!s->lift_table) goto nomem;
     if (mxh_lift_table(s->prec, &s->lv[s->L], s->lift_table)) goto dev;
   }
+  if (node_buffers(s, !s->lift_table)) goto nomem;
   s->es = block_stride(edim(s, s->L));
   s->dE = (double *)dalloc(s, 16 * (size_t)s->es * vpp * P);
   s->dU = (double *)dalloc(s, 16 * (size_t)s->es * vpp * P);
@@ -1325,6 +1336,9 @@ int mx_time_kernel(mx_solver *s, int kind, int reps, double *avg_ms, double *byt
   const int L = s->L, nv = s->last_nprob * s->cfg.block;
   mxh_bloch bl = batch_bloch(s);
   void *e0, *e1;
+  if ((kind == 2 || kind == 3 || kind == 5 || kind == 7 || kind == 11 || (kind >= 15 && kind <= 17)) &&
+      node_buffers(s, 1))
+    return MX_ENOMEM;
   CK(mxh_event_create(&e0));
   if (mxh_event_create(&e1)) {
     mxh_event_destroy(e0);
