@@ -47,7 +47,12 @@ typedef struct {
                          cycles) and runs the cycles only with phase_kernels
                          and on grids mxh_lift_supported refuses */
   int phase_kernels;  /* 0: tile-fused smoother kernels (default); 1: one
-                         launch per colour phase (same arithmetic, for checks) */
+                         launch per colour phase, for checks of the smoothers:
+                         the same sweeps and transfers, but the coarse systems
+                         by substitution instead of their inverses and the
+                         lifting by gradient_steps node V-cycles instead of
+                         directly.  Both converge to the same pairs; iterates
+                         and step counts differ by what the lifting leaves */
   int lock;           /* 1: converged wanted pairs are locked -- kept in the
                          Ritz basis but not preconditioned -- until their
                          residual exceeds tol again; 0: every vector is
@@ -67,11 +72,13 @@ typedef struct {
   int autotune;       /* 1: at the first solve, time the square tiles and
                          row-marching tiles of 32..256 rows on every level
                          for the smoothers in use over the batch, and use the
-                         fastest (overrides march_min / march_rows; the
-                         arithmetic, hence the result, is the same) */
+                         fastest (overrides march_min / march_rows).  Every
+                         choice runs the same sweeps; they round differently
+                         (copies of nodes across the periodic boundary), so
+                         results of two tunings agree to rounding */
   int graphs;         /* 1: capture each block step's preconditioner (the
                          gather of the defects, prec_steps edge V-cycles and
-                         the lifting with its node V-cycles) into a HIP graph
+                         the lifting) into a HIP graph
                          and replay it; it is captured again only when the
                          number of preconditioned vectors changes.  Same
                          kernels and arguments, hence the same result.

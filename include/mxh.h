@@ -280,7 +280,7 @@ int mxh_node_tile(int prec, const mxh_level *lv, const mxh_bloch *bl, int nv,
 /* Row-marching forms of mxh_afw_tile and mxh_node_tile: nsweep (1 or 2)
    sweeps per launch, the same modes (0, 1, 2, 5, 8, 10; zero start,
    prolongation at load, residual + restriction after the last sweep) and the
-   same arithmetic, hence the same result.  A workgroup of 128 * nsweep
+   same sweeps; results agree to rounding.  A workgroup of 128 * nsweep
    threads owns up to 128 - 2H columns (halo H = 6 for one sweep, 10 for two)
    and `rows` rows (0: 128) and streams its region through an LDS ring of
    rows.  Requires nx, ny even and >= 10.  xo must differ from x (halo columns
