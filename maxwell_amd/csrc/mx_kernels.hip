@@ -921,12 +921,12 @@ struct GramArgs {
   int nx, ny, mq, j0, j1;
 };
 
-// The sums of one workgroup's rows over Q tiles (8 vectors each): K (MATS & 1)
-// and M (MATS & 2).
-template <int Q, int MATS = 3>
+// The sums of one workgroup's rows over Q tiles (8 vectors each), or (LAST) of the
+// last tile with itself and those before only: K (MATS & 1) and M (MATS & 2).
+template <int Q, bool LAST = false, int MATS = 3>
 MXH_DEV void gram_rows(const GramArgs& g, double* lds)
 {
-  constexpr int NP = Q * (Q + 1) / 2;
+  constexpr int NP = LAST ? Q : Q * (Q + 1) / 2;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = (lane >> 3) & 1, k2 = 2 * (lane >> 4);
   const int nx = g.nx, ny = g.ny;
@@ -1002,8 +1002,9 @@ MXH_DEV void gram_rows(const GramArgs& g, double* lds)
           F[t][q][0] = lane_xor8<0xc>(f[q].r, f[q].i);
           F[t][q][1] = lane_xor8<0x3>(f[q].i, f[q].r);
         }
+        if (LAST && t + 1 < Q) continue;
         const double a0 = e0 * F[t][0][0], a1 = e1 * F[t][0][1];
-        const int p0 = t * (t + 1) / 2;
+        const int p0 = LAST ? 0 : t * (t + 1) / 2;
         auto mac = [&](v4d* acc, double l, int q, int cell2) {
 #pragma unroll
           for (int c = 0; c <= t; c++)
@@ -1028,31 +1029,28 @@ MXH_DEV void gram_rows(const GramArgs& g, double* lds)
   // im, column j.  With a = row & 7, b = column & 7 the complex sum is
   // rr + ii + i (ri - ir): lanes j < 8 form the real part of rows 4 e + im,
   // e < 2, lanes j >= 8 the imaginary part.  Summed over the waves in order.
-  for (int w = 0; w < 4; w++) {
-    if (wave == w) {
+  constexpr int NM = MATS == 3 ? 2 : 1, PER = NP * NM * 128;  // matrices; sums of a wave
 #pragma unroll
-      for (int p = 0; p < NP; p++)
+  for (int p = 0; p < NP; p++)
 #pragma unroll
-        for (int mat = 0; mat < 2; mat++) {
-          if (!(MATS >> mat & 1)) continue;
-          const v4d d = mat ? M[p] : K[p];
+    for (int mat = 0; mat < NM; mat++) {
+      const v4d d = mat || MATS == 2 ? M[p] : K[p];
 #pragma unroll
-          for (int e = 0; e < 2; e++) {
-            const double o = lane_xor8<0xf>(0.0, d[e + 2]);
-            const double v = h ? d[e] - o : d[e] + o;
-            double* q = lds + ((p * 2 + mat) * 2 + e) * 64 + lane;
-            *q = w ? *q + v : v;
-          }
-        }
+      for (int e = 0; e < 2; e++) {
+        const double o = lane_xor8<0xf>(0.0, d[e + 2]);
+        lds[wave * PER + ((p * NM + mat) * 2 + e) * 64 + lane] = h ? d[e] - o : d[e] + o;
+      }
     }
-    __syncthreads();
-  }
-  for (int w = tid; w < NP * 256; w += 256) {
-    const int l = w & 63, e = (w >> 6) & 1, mat = (w >> 7) & 1;
-    int T, S;
-    pair_ab(w >> 8, T, S);
+  __syncthreads();
+  for (int w = tid; w < PER; w += 256) {
+    const int l = w & 63, e = (w >> 6) & 1, p = w / (NM * 128);
+    const int mat = MATS == 3 ? (w >> 7) & 1 : MATS - 1;
+    int T = Q - 1, S = p;
+    if (!LAST) pair_ab(p, T, S);
     const int a = 8 * T + 4 * e + (l >> 4), b = 8 * S + (l & 7);
-    if ((MATS >> mat & 1) && a < g.mq && b <= a) g.out[4 * (a * (a + 1) / 2 + b) + 2 * mat + ((l >> 3) & 1)] = lds[w];
+    if (a < g.mq && b <= a)
+      g.out[4 * (a * (a + 1) / 2 + b) + 2 * mat + ((l >> 3) & 1)] =
+          ((lds[w] + lds[PER + w]) + lds[2 * PER + w]) + lds[3 * PER + w];
   }
 }
 
@@ -1062,7 +1060,11 @@ MXH_DEV void gram_rows(const GramArgs& g, double* lds)
 // indices in the block, increasing) a problem's sums run over those mq
 // columns only and land at the pair indices of the list (pair a (a+1)/2 + b
 // of list positions a >= b); the rest of its output is left unwritten.
-template <int NT>
+// Workgroups z = 0 take the first FIRST tiles and all their pairs, z > 0 tile
+// FIRST + z - 1 with itself and those before.  All six tiles in one workgroup go over
+// their rows twice, for K and for M: the sums of 21 pairs of both would not fit in
+// registers.
+template <int NT, int FIRST>
 __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gram(mxh_level lv, mxh_bloch bl, int m, const int* pmap,
                                                                const int* cmap, const C<double>* U0, long long us,
                                                                const double* eta, double* part, int rpb)
@@ -1095,21 +1097,28 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gram(mxh_level lv, mxh
   g.j0 = min(lv.ny, (int)blockIdx.x * rpb);
   g.j1 = min(lv.ny, g.j0 + rpb);
   // the tiles this problem's columns fill (uniform)
-  switch (min((mq + 7) / 8, NT)) {
-  case 1: gram_rows<1>(g, smem); break;
-  case 2: if constexpr (NT >= 2) gram_rows<2>(g, smem); break;
-  case 3: if constexpr (NT >= 3) gram_rows<3>(g, smem); break;
-  case 4: if constexpr (NT >= 4) gram_rows<4>(g, smem); break;
-  case 5: if constexpr (NT >= 5) gram_rows<5>(g, smem); break;
-  case 6:
-    // both matrices' sums of 21 tile pairs would not fit in registers: one
-    // after the other (the inputs read twice)
-    if constexpr (NT >= 6) {
-      gram_rows<6, 1>(g, smem);
-      __syncthreads();
-      gram_rows<6, 2>(g, smem);
+  const int nt = min((mq + 7) / 8, NT), z = (int)blockIdx.z;
+  if (z == 0) {
+    switch (min(nt, FIRST)) {
+    case 1: gram_rows<1>(g, smem); break;
+    case 2: if constexpr (FIRST >= 2) gram_rows<2>(g, smem); break;
+    case 3: if constexpr (FIRST >= 3) gram_rows<3>(g, smem); break;
+    case 4: if constexpr (FIRST >= 4) gram_rows<4>(g, smem); break;
+    case 5: if constexpr (FIRST >= 5) gram_rows<5>(g, smem); break;
+    case 6:
+      if constexpr (FIRST >= 6) {
+        gram_rows<6, false, 1>(g, smem);
+        __syncthreads();
+        gram_rows<6, false, 2>(g, smem);
+      }
+      break;
     }
-    break;
+  } else if (FIRST + z <= nt) {
+    switch (FIRST + z) {
+    case 4: if constexpr (NT >= 4 && FIRST < 4) gram_rows<4, true>(g, smem); break;
+    case 5: if constexpr (NT >= 5 && FIRST < 5) gram_rows<5, true>(g, smem); break;
+    case 6: if constexpr (NT >= 6 && FIRST < 6) gram_rows<6, true>(g, smem); break;
+    }
   }
 }
 
@@ -5032,7 +5041,8 @@ int mxh_init(void)
                        (const void*)k_fft_rows<float, -1>, (const void*)k_fft_rows<float, 1>,
                        (const void*)k_edge_cycle<double>, (const void*)k_edge_cycle<float>,
                        (const void*)k_node_cycle<double>, (const void*)k_node_cycle<float>,
-                       (const void*)k_hh_coef};
+                       (const void*)k_gram<4, 4>, (const void*)k_gram<5, 5>, (const void*)k_gram<6, 5>,
+                       (const void*)k_gram<6, 6>, (const void*)k_hh_coef};
   for (const void* f : big) {
     e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_MAX);
     if (e != hipSuccess) return (int)e;
@@ -5717,6 +5727,31 @@ size_t mxh_gram_work_bytes(int m, int nprob)
   return sizeof(double) * 4 * (size_t)(m * (m + 1) / 2) * sets;
 }
 
+// A workgroup's time over r rows and q tiles with p tile pairs, in units of about
+// 0.09 us: a strip's row costs its products and features, a strip its first loads,
+// the workgroup the sums of its waves (fitted to 16^2 to 512^2, within about 15%).
+static double gram_group_cost(const mxh_level* lv, int r, int p, int q)
+{
+  const int ns = (lv->nx + GRAM_STRIP - 1) / GRAM_STRIP;
+  const double strips = ns < 4 ? ns : (ns + 3) / 4, rows = ns < 4 ? 0.25 * (r + 3) : r;
+  if (p > 15) return strips * (rows * (2 * p + 2 * q) + 72.0) + 5.5 * p;  // (two passes)
+  return strips * (rows * (2 * p + q) + 24.0) + 5.5 * p;
+}
+
+// The launch's time with wgs bands of r rows and the first f tiles in one workgroup:
+// rounds of `slots` workgroups (one to four per compute unit, by the registers of the
+// tiles' sums), those of the later tiles in the places that the last round leaves, then
+// in rounds of their own.
+static double gram_cost(const mxh_level* lv, int wgs, int nt, int f, int r, int slots)
+{
+  const int rounds = (wgs + slots - 1) / slots;
+  const double c0 = gram_group_cost(lv, r, f * (f + 1) / 2, f), t = rounds * c0;
+  if (f == nt) return t;
+  const double c1 = gram_group_cost(lv, r, nt, nt), beside = (rounds - 1) * c0 + c1;
+  const int left = wgs * (nt - f) - (rounds * slots - wgs) * (c0 > c1 ? (int)(c0 / c1) : 1);
+  return (t > beside ? t : beside) + (left > 0 ? (left + slots - 1) / slots * c1 : 0.0);
+}
+
 // The Gram launch with at most max(sets_cap, nprob) partial-sum sets in work.
 static int gram_launch(const mxh_level* lv, const mxh_bloch* bl, int nprob, const int* pmap, const int* cmap, int m,
                        mxh_vecs u, const double* eta64, double* out, void* work, int sets_cap)
@@ -5724,44 +5759,56 @@ static int gram_launch(const mxh_level* lv, const mxh_bloch* bl, int nprob, cons
   if (m < 1 || m > GRAM_MMAX || nprob < 1 || sets_cap < 1) return (int)hipErrorInvalidValue;
   const int np = m * (m + 1) / 2, nt = (m + 7) / 8;
   // Row bands: bands * nprob partial sets (sets_cap or nprob) fit the work
-  // buffer.  Workgroups run in rounds of `slots` (one to four per compute unit,
-  // by the registers of the tiles' sums) and a band costs its rows and about
-  // one row for its start, so the height minimises rounds x (rows + 1).  36
-  // columns, 16 problems of 512^2: 4, 8, 16, 32 rows measured 2.00, 1.79, 1.69,
-  // 1.66 ms, 64 rows (half the units idle) 3.19.  Heights from the least that the
-  // buffer takes to twice that, or 64: with 64 as the limit always, tall grids and
-  // many problems had one band a problem (256 x 4096, 33 problems of 12 columns:
-  // 24.3 ms against 3.0).
+  // buffer.  Heights from the least that the buffer takes to twice that, or 64:
+  // with 64 as the limit always, tall grids and many problems had one band a
+  // problem (256 x 4096, 33 problems of 12 columns: 24.3 ms against 3.0).  Blocks of
+  // more than three tiles run whole or with the tiles after the third (of six, after
+  // the fifth) in workgroups of their own, which shortens the longest workgroup
+  // where units would be idle, but loads the first tiles again: for a fifth (a
+  // tenth) less by the model.  36 columns (us, whole and split): one problem of
+  // 16^2 18.8 and 11.4, 72^2 26.0 and 18.1, 500 x 20 78 and 65; 16 problems of 16^2
+  // 27.8 and 20.3, 64 x 256 120 and 170, 128^2 121 and 176.  48 columns (whole, after
+  // the fifth, after the third): one problem of 16^2 37, 19, 12, seven of 72^2 75,
+  // 58, 64, 16 of 512^2 2580, 2800, -.
   const int sets = nprob > sets_cap ? nprob : sets_cap;
-  const long long slots = (long long)mxh_cu_count() * (nt == 1 ? 4 : nt == 2 ? 2 : 1);
+  const int slots = mxh_cu_count() * (nt == 1 ? 4 : nt == 2 ? 2 : 1);
   const int most = sets / nprob, least = (lv->ny + most - 1) / most;
-  int rpb = least;
-  long long cost = -1;
-  for (int r = least; r <= (least > 32 ? 2 * least : 64) && r <= lv->ny; r++) {
-    const long long wgs = (long long)((lv->ny + r - 1) / r) * nprob;
-    const long long c = (wgs + slots - 1) / slots * (r + 1);
-    if (cost < 0 || c <= cost) {
-      cost = c;
-      rpb = r;
+  int rpb = least, first = nt;
+  double cost = -1.0;
+  for (int f = nt; f > 0; f = f == 6 ? 5 : f > 3 ? 3 : 0)
+    for (int r = least; r <= (least > 32 ? 2 * least : 64) && r <= lv->ny; r++) {
+      const int wgs = (lv->ny + r - 1) / r * nprob;
+      const double c = gram_cost(lv, wgs, nt, f, r, slots) * (f == nt ? 1.0 : f == 5 ? 1.1 : 1.25);
+      if (cost < 0.0 || c < cost) {
+        cost = c;
+        first = f;
+        rpb = r;
+      }
+      if (wgs * (nt - f + 1) <= slots) break;  // one round: higher bands only take longer
     }
-  }
   const int bands = (lv->ny + rpb - 1) / rpb;
-  const size_t sh = sizeof(double) * 256 * (size_t)(nt * (nt + 1) / 2);
-  const dim3 grid(bands, nprob);
-#define GRAM_CASE(NT)                                                                                       \
-  case NT:                                                                                                  \
-    hipLaunchKernelGGL(k_gram<NT>, grid, dim3(TPB), sh, g_stream, *lv, *bl, m, pmap, cmap,                  \
-                       (const C<double>*)u.p, u.stride, eta64, (double*)work, rpb);                         \
-    break;
-  switch (nt) {
-    GRAM_CASE(1)
-    GRAM_CASE(2)
-    GRAM_CASE(3)
-    GRAM_CASE(4)
-    GRAM_CASE(5)
-    GRAM_CASE(6)
+  // The waves' sums in LDS, 256 of each tile pair: of the first tiles, at least as many
+  // as a later tile's.  Six tiles whole take 128 of 21 pairs at a time, but a problem's
+  // column list may fill five only.
+  const int most5 = first < 5 ? first : 5;
+  const size_t sh = 4 * sizeof(double) * 128 * (size_t)(most5 * (most5 + 1));
+  const dim3 grid(bands, nprob, nt - first + 1);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(TPB), sh, g_stream, *lv, *bl, m, pmap, cmap, (const C<double>*)u.p, u.stride,
+                       eta64, (double*)work, rpb);
+  };
+  switch (10 * nt + first) {
+  case 11: go(k_gram<1, 1>); break;
+  case 22: go(k_gram<2, 2>); break;
+  case 33: go(k_gram<3, 3>); break;
+  case 43: go(k_gram<4, 3>); break;
+  case 44: go(k_gram<4, 4>); break;
+  case 53: go(k_gram<5, 3>); break;
+  case 55: go(k_gram<5, 5>); break;
+  case 63: go(k_gram<6, 3>); break;
+  case 65: go(k_gram<6, 5>); break;
+  case 66: go(k_gram<6, 6>); break;
   }
-#undef GRAM_CASE
   LAUNCH_CHECK();
   int width = 4 * np * nprob;
   hipLaunchKernelGGL(k_reduce_partials, dim3(reduce_blocks(width)), dim3(TPB), 0, g_stream, (const double*)work,
