@@ -874,10 +874,10 @@ __global__ __launch_bounds__(256) void k_coarse_solve(int n, const double* Lm, c
 // sums of 15 tile pairs take 240 registers) spend 90 MFMAs of 64 cycles per
 // strip row and wave and about a sixth of that on features, which the matrix
 // core does not overlap.  512^2, against a register-blocked vector kernel fed
-// from LDS (bound by its LDS reads and their latency): 36 columns of 16
-// problems 2.66 -> 1.69 ms (37 -> 58 TFLOP/s counting the padded tiles'
-// products once), 32 columns 2.62 -> 1.27, 12 columns of 64 problems 2.2 -> 1.70
-// (3.8 TB/s).  The tile loop's MFMA and vector instructions interleaved by
+// from LDS (bound by its LDS reads and their latency): 36 columns of 64
+// problems 10.8 -> 6.4 ms (60 TFLOP/s with the padded tiles' products, the
+// matrix pipe busy 81% of the cycles), 32 columns of 16 2.62 -> 1.27, 12 columns
+// of 64 2.2 -> 1.64 (3.9 TB/s).  The tile loop's MFMA and vector instructions interleaved by
 // hand, and two waves per SIMD at 3 tiles, measured no better.
 #define GRAM_MMAX 48
 #define GRAM_STRIP 8
@@ -1145,10 +1145,11 @@ __global__ __launch_bounds__(256, NT <= 2 ? 2 : 1) void k_gram(mxh_level lv, mxh
 // Everything stays in LDS in FP64; a step of a factorisation or substitution
 // has one barrier, a Jacobi round two.  What bounds it is that chain (per round
 // a rotation's square roots, a barrier, the LDS reads and writes of A and V, a
-// barrier): 54 us for 16 problems of 9 columns and 638 us for 64 of 36, of
-// which all run at once.  On the host the same problems took 0.5 to 1 ms
-// between device steps that wait for them (64^2 grids in FP64, 16 problems: a
-// solve of 80 ms against 56) and needed two transfers.  LOBPCG's bases of three
+// barrier): 51 us a step of a solve with 64 problems of 12 columns, all of which
+// run at once; random dense pencils, which need more sweeps, 73 us for 16 of 9
+// columns and 945 us for 64 of 36.  On the host the same problems took 0.5 to
+// 1 ms between device steps that wait for them (64^2 grids in FP64, 16 problems:
+// a solve of 80 ms against 56) and needed two transfers.  LOBPCG's bases of three
 // blocks stay on the host, where they run beside the device (bloch_solver.c).
 #define RITZ_MAX 48
 
